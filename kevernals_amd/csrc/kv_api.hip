@@ -167,6 +167,33 @@ std::vector<float> ray_constants(const kv_geometry &q)
     return rc;
 }
 
+// Entries per list of KvGeom::seg_a, or 0 if the lists would take more than
+// KV_SEG_MAX_BYTES.  A ray crosses at most nz + 1 z planes and the y planes
+// between its entry into the volume and its exit, which lie within the z
+// faces' crossings; the margins cover FP32 rounding in the list's builder.
+int seg_stride(const kv_geometry &q)
+{
+    int most = 0;
+    for (int p = 0; p < q.np; ++p) {
+        const double sz = (double)q.src[3 * p + 2] / q.sz, dz = (double)q.det[3 * p + 2] / q.sz - sz;
+        const double sy = (double)q.src[3 * p + 1] / q.sy;
+        double lo = 0.0, hi = 1.0;
+        if (dz != 0.0) {
+            const double a = (-0.5 * q.nz - sz) / dz, b = (0.5 * q.nz - sz) / dz;
+            lo = std::max(lo, std::min(a, b));
+            hi = std::min(hi, std::max(a, b));
+        }
+        for (int v = 0; v < q.nv; ++v) {
+            const double dy = ((double)q.det[3 * p + 1] + (v + 0.5) * q.pv) / q.sy - sy;
+            const double y = std::max(0.0, hi - lo) * std::fabs(dy);
+            most = std::max(most, y < q.ny ? (int)y : q.ny);
+        }
+    }
+    const int64_t n = (int64_t)std::min(most + 8, q.ny + 2) + q.nz + 8 + KV_SEG_PAD;
+    const double bytes = (double)n * q.np * q.nv * sizeof(KvSeg);
+    return bytes <= (double)KV_SEG_MAX_BYTES ? (int)n : 0;
+}
+
 kv_status check_mode(int mode)
 {
     if (mode != KV_MODE_R && mode != KV_MODE_A) {
@@ -232,6 +259,10 @@ void release_geometry(kv_context *ctx)
     free_dev(ctx->d_det);
     free_dev(ctx->d_src);
     free_dev(ctx->d_rc);
+    free_dev(ctx->d_seg_a);
+    free_dev(ctx->d_seg_a_head);
+    ctx->g.seg_a = nullptr;
+    ctx->g.seg_a_head = nullptr;
     free_tables(ctx->tab_r);
     free_tables(ctx->tab_a);
     free_dev(ctx->d_ratio);
@@ -395,6 +426,25 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     g.rc = ctx->d_rc;
     g.walk_fast = walk_fast_ok(q) ? 1 : 0;
     g.bp_posz = bp_posz_ok(q) ? 1 : 0;
+    // Segment lists of the detector rows.  They are an option: without them
+    // (too large, or no memory left) the rays are walked voxel by voxel.
+    g.seg_a = nullptr;
+    g.seg_a_head = nullptr;
+    g.seg_stride = seg_stride(q);
+    if (g.seg_stride > 0) {
+        const size_t rows = (size_t)q.np * q.nv;
+        if (hipMalloc((void **)&ctx->d_seg_a, rows * g.seg_stride * sizeof(KvSeg)) == hipSuccess &&
+            hipMalloc((void **)&ctx->d_seg_a_head, rows * sizeof(KvSegHead)) == hipSuccess) {
+            KV_TRY_HIP(kv_launch_seg_a(g, ctx->d_seg_a, ctx->d_seg_a_head, ctx->stream));
+            KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
+            g.seg_a = ctx->d_seg_a;
+            g.seg_a_head = ctx->d_seg_a_head;
+        } else {
+            (void)hipGetLastError();  // the failed allocation's
+            free_dev(ctx->d_seg_a);
+            free_dev(ctx->d_seg_a_head);
+        }
+    }
     ctx->has_geom = true;
     return KV_OK;
 }
@@ -822,7 +872,7 @@ kv_status kv_log_likelihoods(kv_context *ctx, const float *d_data, const float *
         if (kv_status st = dev_alloc((void **)&ctx->d_ll, (KV_LL_MAX - 1) * nray * sizeof(float)))
             return st;
     }
-    if (n > 1 && !ctx->d_pack) {
+    if (n > 1 && !ctx->g.seg_a && !ctx->d_pack) {
         if (kv_status st = dev_alloc((void **)&ctx->d_pack, 4 * (size_t)kv_nvox(ctx->g) * sizeof(float)))
             return st;
     }

@@ -55,10 +55,18 @@ void layout_items(kv_batch *b)
 {
     long long fp = 0, bp = 0;
     for (auto &P : b->probs) {
-        const int L = P.fp_layout, wu = 64 / L, span = KV_XCDS * std::max(1, KV_FP_STRIPE / wu);
-        P.fp_chunk = span / KV_XCDS;
-        P.fp_tx = ((P.g.nu + wu - 1) / wu + span - 1) / span * span;
-        P.fp_ty = (P.g.nv + 4 * L - 1) / (4 * L);
+        if (P.g.seg_a && b->mode == KV_MODE_A) {
+            P.fp_chunk = KV_ROW_CY;
+            P.fp_tx = kv_row_tiles_x(P.g.nu);
+            P.fp_ty = kv_row_tiles_y(P.g.nv);
+        } else {
+            const int L = P.fp_layout, wu = 64 / L;
+            P.fp_chunk = std::max(1, KV_FP_STRIPE / wu);
+            const int span = KV_XCDS * P.fp_chunk;
+            P.fp_tx = ((P.g.nu + wu - 1) / wu + span - 1) / span * span;
+            P.fp_ty = (P.g.nv + 4 * L - 1) / (4 * L);
+        }
+        const int span = KV_XCDS * P.fp_chunk;
         P.fp_nch = P.fp_tx / span;
         P.fp_dchunk = kv_udiv((unsigned)P.fp_chunk);
         P.fp_dnch = kv_udiv((unsigned)P.fp_nch);

@@ -1,6 +1,8 @@
 // Forward projectors for gfx950.
 //
-// One ray per lane; a 256-thread workgroup is four wavefronts, each covering
+// One ray per lane.  Mode A runs row by row where a geometry's segment lists
+// exist ("mode A, row by row" below).  Otherwise a 256-thread workgroup is
+// four wavefronts, each covering
 // a (64/L) x L tile of detector pixels (8 x 8 for the plain walk; 16 x 4 and
 // 32 x 2 for the walks that gather two and three volumes per step), so the
 // rays of a wavefront stay close in u and v and their voxel gathers at each
@@ -118,12 +120,11 @@ __device__ __forceinline__ unsigned mad_u24(unsigned a, unsigned b, unsigned c)
 }
 
 // a in the lanes whose bit of mask is set, else b: one v_cndmask with a
-// scalar mask (lanes outside the mask's active set are not written).
+// scalar mask.  (Not inline assembly: the compiler does not see the wait
+// states that a mask fresh from a vector compare needs before one.)
 __device__ __forceinline__ float selm(unsigned long long mask, float a, float b)
 {
-    float r;
-    asm("v_cndmask_b32_e64 %0, %1, %2, %3" : "=v"(r) : "v"(b), "v"(a), "s"(mask));
-    return r;
+    return __builtin_amdgcn_inverse_ballot_w64(mask) ? a : b;
 }
 
 // min(1, a) as one instruction (a is never NaN where it is used).
@@ -131,6 +132,15 @@ __device__ __forceinline__ float min1(float a)
 {
     float r;
     asm("v_min_f32 %0, 1.0, %1" : "=v"(r) : "v"(a));
+    return r;
+}
+
+// min(a, b) as one instruction (operands never NaN where it is used); b may
+// be wavefront-uniform.
+__device__ __forceinline__ float minf(float a, float b)
+{
+    float r;
+    asm("v_min_f32 %0, %2, %1" : "=v"(r) : "v"(a), "s"(b));
     return r;
 }
 
@@ -516,9 +526,9 @@ __global__ __launch_bounds__(256) void fp_r_kernel(KvGeom g, const float *__rest
 // the placement, which only decides the caches' locality.  Problems whose
 // iteration count is reached skip their tiles; padding columns (u past the
 // detector) are skipped at the bounds test.
-template <typename Ray>
+template <typename Tile>
 __device__ __forceinline__ void fp_batch_tiles(const KvProblem *__restrict__ probs, int nprob, long long total,
-                                               unsigned long long *counters, int iteration, Ray &&ray)
+                                               unsigned long long *counters, int iteration, Tile &&tile)
 {
     __shared__ long long item_s;
     const int own = (int)(blockIdx.x % (unsigned)KV_XCDS);
@@ -547,10 +557,7 @@ __device__ __forceinline__ void fp_batch_tiles(const KvProblem *__restrict__ pro
             const int tx = (int)(((jc - r * nch) * KV_XCDS + (unsigned)k) * ch + (local - jc * ch));
             const unsigned q = udiv(r, P.fp_dty);
             const int ty = (int)(r - q * (unsigned)P.fp_ty), p = (int)q;
-            int u, v;
-            fp_tile_pixel(P.fp_layout, tx, ty, threadIdx.x, u, v);
-            if (u < P.g.nu && v < P.g.nv)
-                ray(P, p, u, v);
+            tile(P, p, tx, ty);
         }
     }
 }
@@ -560,8 +567,11 @@ __global__ __launch_bounds__(256) void fp_r_batch_kernel(const KvProblem *__rest
                                                          long long total, unsigned long long *counters, int iteration,
                                                          float relax)
 {
-    fp_batch_tiles(probs, nprob, total, counters, iteration, [&](const KvProblem &P, int p, int u, int v) {
-        fp_r_ray<EP>(P.g, P.vol, P.ratio, P.data, relax, p, u, v);
+    fp_batch_tiles(probs, nprob, total, counters, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
+        int u, v;
+        fp_tile_pixel(P.fp_layout, tx, ty, threadIdx.x, u, v);
+        if (u < P.g.nu && v < P.g.nv)
+            fp_r_ray<EP>(P.g, P.vol, P.ratio, P.data, relax, p, u, v);
     });
 }
 
@@ -747,6 +757,427 @@ struct AccA {
     __device__ __forceinline__ float sum() const { return acc + kv_mul_legacy(pw, pv); }
 };
 
+// ------------------------------------------------- mode A, row by row ----
+// The y and z plane crossings of a ray depend only on its view and detector
+// row, so the 64 rays of a wavefront that covers 64 columns of one row share
+// the sequence of (y, z) segments: alpha interval and volume row.  That
+// sequence is a list built once per geometry (seg_a_kernel) and read by
+// scalar loads; each lane only follows its x crossings inside the segments.
+// The crossings, voxel order, lengths and sums are those of walk_a, so the
+// result is bit-identical to it.
+//
+// walk_a was bound by instruction issue and by the L1's tag lookups (29.5
+// vector instructions and one gather of ~34 cache lines per voxel step,
+// because the lanes of an 8x8 tile drift apart in y and z).  A segment holds
+// 1.25 voxel steps on average and costs 13 vector instructions and one load
+// of neighbouring voxels in seg_sums_row, 20 and two loads in seg_sums.
+
+// The x crossings of one lane: the plane its voxel ends at, as f = k - nx/2
+// (an integer or half-integer below 2^24: exact), its step and its crossing
+// hx = (f - s) * inv as plane_a evaluates it, and the voxel's x index j (k - 1
+// going up, k going down).  Voxels off the volume in x (j < 0 or j >= nx)
+// read 0 through the bounds-checked row loads, and all of those ahead of the
+// ray's entry count as one, whose exit is the entry plane.  A lane whose ray
+// never enters the segments' part of the volume rests outside: hx = +INF.
+struct LaneX {
+    float hx, f, st, s, inv, d;
+    int j;
+    bool live;
+};
+
+__device__ __forceinline__ LaneX lane_x(const KvGeom &g, int p, int u, float a, float end)
+{
+    LaneX l;
+    const float4 c = *(const float4 *)(g.rc + (size_t)g.np * KV_RC + ((size_t)p * g.nu + u) * 4);
+    const int n = g.nx;
+    const float h = (float)n / 2.f;
+    l.s = g.rc[KV_RC * p];
+    l.inv = c.w;
+    l.d = c.x - l.s;
+    l.st = l.d > 0.f ? 1.f : -1.f;
+    const float pos = l.s + h;
+    const int up = l.d > 0.f ? 1 : 0;
+    auto exit_of = [&](int i) { return (((float)(i + up) - h) - l.s) * c.w; };
+    if (l.d == 0.f) {
+        l.j = (pos > 0.f && pos < (float)n) ? (int)floorf(pos) : -1;
+        l.live = l.j >= 0;
+    } else {
+        // the voxel with entry <= a < exit, or the outside voxel ahead of
+        // the entry plane; past the far face the ray has left
+        const int st = up ? 1 : -1;
+        int i = (int)fminf(fmaxf(floorf(pos + a * l.d), -1.f), (float)n);
+#pragma clang loop unroll(disable)
+        while ((up ? i >= 0 : i < n) && exit_of(i - st) > a)
+            i -= st;
+#pragma clang loop unroll(disable)
+        while ((up ? i < n : i >= 0) && exit_of(i) <= a)
+            i += st;
+        l.j = i;
+        l.hx = exit_of(i);
+        l.live = (up ? i < n : i >= 0) && ((unsigned)i < (unsigned)n || l.hx < end);
+    }
+    l.f = (float)(l.j + up) - h;
+    if (l.d == 0.f || !l.live) {
+        // nothing is crossed: (f - s) * inv stays +INF
+        l.j = l.live ? l.j : -1;
+        l.f = l.live ? (float)l.j - h : -1.f - h;
+        l.s = -kInf;
+        l.inv = 1.f;
+        l.hx = kInf;
+        l.st = 0.f;
+    }
+    return l;
+}
+
+// Segments per block: a block's loads are in flight while the block before it
+// is walked.  With one segment at a time the loads' latency lay open: 70 % of
+// the wavefronts' time was spent waiting (1024x1024x64 forward pass, 25 views
+// of 2048^2: 5.4 ms against 4.2 ms, both with the gathers of seg_sums).
+constexpr int SEG_DEPTH = 4;
+static_assert(4 * SEG_DEPTH <= KV_SEG_PAD, "seg_sums_row reads at most 4 blocks past its last segment's");
+
+typedef const __attribute__((address_space(4))) KvSegHead KvSegHeadC;
+typedef const __attribute__((address_space(4))) KvSeg KvSegC;
+// A block of segments as one scalar load: b and row of segment k are words
+// 2 k and 2 k + 1.
+typedef unsigned KvSegBlock __attribute__((ext_vector_type(2 * SEG_DEPTH)));
+typedef const __attribute__((address_space(4), aligned(8))) KvSegBlock KvSegBlockC;
+
+// The sums of NV volumes over a row's segments for any rays: two gathers of
+// one volume row per segment and volume, and further turns on a segment with
+// more than one x plane of some lane.
+template <int NV>
+__device__ __forceinline__ void seg_sums(const KvRsrc (&rs)[NV], int nx, KvSegC *sp, int segs, float a, LaneX &l,
+                                         float *sum)
+{
+    // The products of a segment are added SEG_DEPTH segments later.  Weights
+    // start at 0: a legacy product by 0 is +-0 whatever the voxel, and the
+    // sums are never -0.  Likewise a lane that crosses no plane has w2 = 0
+    // and leaves v2 as it was.
+    float w1[SEG_DEPTH], w2[SEG_DEPTH], v1[NV][SEG_DEPTH], v2[NV][SEG_DEPTH];
+#pragma unroll
+    for (int k = 0; k < SEG_DEPTH; ++k) {
+        w1[k] = w2[k] = 0.f;
+#pragma unroll
+        for (int i = 0; i < NV; ++i)
+            v1[i][k] = v2[i][k] = 0.f;
+    }
+    auto add = [&](int k) {
+#pragma unroll
+        for (int i = 0; i < NV; ++i) {
+            sum[i] = sum[i] + kv_mul_legacy(w1[k], v1[i][k]);
+            sum[i] = sum[i] + kv_mul_legacy(w2[k], v2[i][k]);
+        }
+    };
+    float x = a;
+    float b = sp[0].b, nb = sp[1].b;
+    unsigned row = sp[0].row, nrow = sp[1].row;
+    const int dj = (int)l.st;
+    for (int n = 0; n < segs;) {
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k) {
+            add(k);
+#pragma unroll
+            for (int i = 0; i < NV; ++i)
+                v1[i][k] = kv_struct_load_f32(rs[i], l.j, 0, (int)row, 0);
+            const bool cross = l.hx < b;
+            const float x1 = minf(l.hx, b);
+            w1[k] = x1 - x;
+            l.j += cross ? dj : 0;
+            l.f += cross ? l.st : 0.f;
+            l.hx = (l.f - l.s) * l.inv;
+            if (cross)
+#pragma unroll
+                for (int i = 0; i < NV; ++i)
+                    v2[i][k] = kv_struct_load_f32(rs[i], l.j, 0, (int)row, 0);
+            x = minf(l.hx, b);
+            w2[k] = x - x1;
+            // another turn on this segment as long as some lane with a plane
+            // ahead in it is inside the volume (the others read 0 whatever
+            // their weights), so at most nx turns
+            if (__builtin_amdgcn_ballot_w64(l.hx < b && (unsigned)l.j < (unsigned)nx) == 0) {
+                ++n;
+                b = nb;
+                row = nrow;
+                nb = sp[n + 1].b;
+                nrow = sp[n + 1].row;
+            }
+        }
+    }
+#pragma unroll
+    for (int k = 0; k < SEG_DEPTH; ++k)
+        add(k);
+}
+
+// The same for rays that cross at most one x plane per segment and stay
+// within 64 voxels of each other (row_sums decides).  A volume row is then
+// one load of neighbouring voxels, voxel i in lane i % 64, from which each
+// lane takes its two voxels by a lane permute (which selects by index modulo
+// 64 itself).  The gathers were bound by the L1 (10 cycles per load and CU:
+// 4.0 ms at the size above, 8.0 / 11.9 ms for two / three volumes); this form
+// takes 3.0 ms, bound by instruction issue, and 5.9 / 8.6 ms, bound by the
+// L1's row loads.
+//
+// Rows are loaded one block ahead.  A window placed when block n starts holds
+// every voxel of blocks n and n + 1: the lanes' range now, plus `below` /
+// `above` voxels the lanes may move in two blocks and one of slack on each
+// side (lanes are ordered in x up to the rounding of their crossings).
+template <int NV>
+__device__ __forceinline__ void seg_sums_row(const KvRsrc (&rs)[NV], float h, KvSegC *sp, int segs, float a,
+                                             LaneX &l, unsigned long long live, int below, int above, float *sum)
+{
+    // f + MAGIC has an ulp of 1/4: the bits of the sum count quarters of a
+    // voxel, i.e. they are a permute's byte address (64 lanes x 4 bytes) up
+    // to a constant, for |f| < 2^20.
+    constexpr float MAGIC = 3145728.f;  // 1.5 * 2^21
+    const int lane = (int)(threadIdx.x & 63);
+    const int first = __builtin_ctzll(live), last = 63 - __builtin_clzll(live);
+    // bits of (voxel index + fc) + MAGIC: j = k - 1 or k, f = k - h
+    const float up = l.st > 0.f ? 1.f : 0.f;
+    const float ac = MAGIC + (h - up);  // f + ac = j + MAGIC, exact
+    constexpr int MAGIC_BITS = 0x4A400000;
+    int at = __float_as_int(l.f + ac);
+    KvSegBlock q, nq, mq;
+    auto read = [&](KvSegBlock &d) {
+        d = *(KvSegBlockC *)sp;
+        sp += SEG_DEPTH;
+    };
+    // Ends the time a block may be in flight: its words are in scalar
+    // registers from here on (loads of constant memory would otherwise be
+    // moved to, or issued again at, their first use, and waited for there).
+    auto arrived = [](KvSegBlock &d) { asm volatile("" : "+s"(d)); };
+    float ra[NV][SEG_DEPTH], rb[NV][SEG_DEPTH];
+    auto rows = [&](const KvSegBlock &d, float (&r)[NV][SEG_DEPTH]) {
+        const int j0 = (__builtin_amdgcn_readlane(at, first) - MAGIC_BITS) >> 2,
+                  j1 = (__builtin_amdgcn_readlane(at, last) - MAGIC_BITS) >> 2;
+        const int base = min(j0, j1) - 1 - below, width = max(j0, j1) + 2 + above - base;
+        const int o = (lane - base) & 63;
+        const int i = o < width ? base + o : -1;
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k)
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                r[v][k] = kv_struct_load_f32(rs[v], i, 0, (int)d[2 * k + 1], 0);
+    };
+    auto walk = [&](const KvSegBlock &d, const float (&r)[NV][SEG_DEPTH]) {
+        float w1[SEG_DEPTH], w2[SEG_DEPTH], v1[NV][SEG_DEPTH], v2[NV][SEG_DEPTH];
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k) {
+            const float b = __uint_as_float(d[2 * k]);
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                v1[v][k] = __int_as_float(__builtin_amdgcn_ds_bpermute(at, __float_as_int(r[v][k])));
+            const float x1 = minf(l.hx, b);
+            w1[k] = x1 - a;
+            w2[k] = b - x1;
+            l.f += l.hx < b ? l.st : 0.f;
+            l.hx = (l.f - l.s) * l.inv;
+            at = __float_as_int(l.f + ac);
+#pragma unroll
+            for (int v = 0; v < NV; ++v)
+                v2[v][k] = __int_as_float(__builtin_amdgcn_ds_bpermute(at, __float_as_int(r[v][k])));
+            a = b;
+        }
+        __builtin_amdgcn_sched_barrier(0);  // every permute issued before the first is waited for
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k)
+#pragma unroll
+            for (int v = 0; v < NV; ++v) {
+                sum[v] = sum[v] + kv_mul_legacy(w1[k], v1[v][k]);
+                sum[v] = sum[v] + kv_mul_legacy(w2[k], v2[v][k]);
+            }
+    };
+    read(q);
+    read(nq);
+    arrived(q);
+    arrived(nq);
+    rows(q, ra);
+    for (int n = 0; n < segs; n += 2 * SEG_DEPTH) {
+        rows(nq, rb);
+        read(mq);
+        __builtin_amdgcn_sched_barrier(0);
+        walk(q, ra);
+        __builtin_amdgcn_sched_barrier(0);
+        arrived(mq);
+        if (n + SEG_DEPTH >= segs)
+            break;
+        rows(mq, ra);
+        read(q);
+        __builtin_amdgcn_sched_barrier(0);
+        walk(nq, rb);
+        __builtin_amdgcn_sched_barrier(0);
+        arrived(q);
+        nq = q;
+        q = mq;
+    }
+    // the other lanes permuted some lane's voxels with weights of their own
+#pragma unroll
+    for (int v = 0; v < NV; ++v)
+        sum[v] = l.live ? sum[v] : 0.f;
+}
+
+// Line sums (alpha length x voxel, not yet times the ray length) of NV
+// volumes along the ray of view p, column u, row v; v and p are
+// wavefront-uniform.  vol[i] must hold g.nx * g.ny * g.nz floats.
+template <int NV>
+__device__ __forceinline__ void row_sums(const KvGeom &g, const float *const *vol, int p, int u, int v, float *sum)
+{
+    const size_t id = (size_t)p * g.nv + v;
+    KvSegHeadC *hp = (KvSegHeadC *)(size_t)(g.seg_a_head + id);
+    KvSegC *sp = (KvSegC *)(size_t)(g.seg_a + id * (size_t)g.seg_stride);
+    const int segs = hp->segs;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        sum[i] = 0.f;
+    if (segs == 0)
+        return;
+    KvRsrc rs[NV];
+#pragma unroll
+    for (int i = 0; i < NV; ++i) {
+        // records = the voxels of one row: the row itself is the scalar
+        // offset, which the bounds check leaves out
+        const unsigned long long at = (unsigned long long)vol[i];
+        rs[i].x = (int)(unsigned)at;
+        rs[i].y = (int)(((unsigned)(at >> 32) & 0xFFFFu) | (4u << 16));
+        rs[i].z = g.nx;
+        rs[i].w = 0x00020000;
+    }
+    const float a = hp->a, longest = hp->longest, end = hp->end;
+    {
+        // none of the columns' rays between the x faces while in the
+        // segments (by the reference's face alphas, good to a few ulps)
+        const float4 c = *(const float4 *)(g.rc + (size_t)g.np * KV_RC + ((size_t)p * g.nu + u) * 4);
+        if (!__any(c.y == c.z || (fminf(c.y, c.z) < end + 1e-5f && fmaxf(c.y, c.z) > a - 1e-5f)))
+            return;
+    }
+    LaneX l = lane_x(g, p, u, a, end);
+    const unsigned long long live = __builtin_amdgcn_ballot_w64(l.live);
+    if (live == 0)
+        return;
+    // Steepness and distance of the rays in x: |d| planes per unit of alpha,
+    // largest at an end of the wavefront's live columns; the lanes' distance
+    // grows along the rays.  With coordinates below 2^16 voxels FP32
+    // positions are good to a fraction of a voxel.
+    const float df = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.d), __builtin_ctzll(live))),
+                dl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(l.d), 63 - __builtin_clzll(live)));
+    const float steep = fmaxf(fabsf(df), fabsf(dl)) * longest;
+    const int ahead = (int)fminf(steep * (2.f * SEG_DEPTH), 64.f) + 2;
+    const int below = __any(l.live && l.st < 0.f) ? ahead : 0, above = __any(l.live && l.st > 0.f) ? ahead : 0;
+    // One plane per segment at most: crossings lie 1 / |d| apart up to their
+    // FP32 rounding (below 4e-7 in alpha for the two; 1e-6 taken).
+    const bool single = steep + (fabsf(df) + fabsf(dl)) * 1e-6f < 1.f;
+    const float range = end * fabsf(dl - df) + 4.f + (float)(below + above);
+    if (single && range <= 63.f && fmaxf(fabsf(df), fabsf(dl)) < 65536.f && fabsf(g.rc[KV_RC * p]) < 65536.f &&
+        g.nx < 65536)
+        seg_sums_row<NV>(rs, (float)g.nx / 2.f, sp, segs, a, l, live, __builtin_amdgcn_readfirstlane(below),
+                         __builtin_amdgcn_readfirstlane(above), sum);
+    else
+        seg_sums<NV>(rs, g.nx, sp, segs, a, l, sum);
+}
+
+// The mode-A segment list of one (view, detector row) per thread: walk_a
+// restricted to y and z.
+__global__ __launch_bounds__(64) void seg_a_kernel(KvGeom g, KvSeg *__restrict__ seg, KvSegHead *__restrict__ head)
+{
+    const int id = blockIdx.x * 64 + threadIdx.x;
+    if (id >= g.np * g.nv)
+        return;
+    const int p = id / g.nv, v = id - p * g.nv;
+    const float *C = g.rc + KV_RC * p;
+    const float4 cy = *(const float4 *)(g.rc + (size_t)g.np * (KV_RC + 4 * g.nu) + ((size_t)p * g.nv + v) * 4);
+    const float s[2] = {C[1], C[2]}, d[2] = {cy.x - C[1], C[3]}, h[2] = {(float)g.ny / 2.f, (float)g.nz / 2.f};
+    const float inv[2] = {cy.w, C[3] != 0.f ? 1.f / C[3] : 0.f};
+    const int n[2] = {g.ny, g.nz};
+    auto plane = [&](int c, int k) { return (((float)k - h[c]) - s[c]) * inv[c]; };
+    head[id] = KvSegHead{0.f, 0.f, 0.f, 0};
+    float ain = 0.f, aout = 1.f;
+    int ii[2], stp[2];
+    float hi[2];
+    for (int c = 0; c < 2; ++c) {
+        if (d[c] == 0.f) {
+            const float pos = s[c] + h[c];
+            if (!(pos > 0.f && pos < (float)n[c]))
+                return;
+            continue;
+        }
+        const float a0 = plane(c, 0), aN = plane(c, n[c]);
+        ain = fmaxf(ain, fminf(a0, aN));
+        aout = fminf(aout, fmaxf(a0, aN));
+    }
+    if (!(ain < aout))
+        return;
+    for (int c = 0; c < 2; ++c) {
+        if (d[c] == 0.f) {
+            ii[c] = (int)floorf(s[c] + h[c]);
+            hi[c] = kInf;
+            stp[c] = 0;
+            continue;
+        }
+        int i = max(0, min(n[c] - 1, (int)floorf(s[c] + h[c] + ain * d[c])));
+        const int st = d[c] > 0.f ? 1 : -1;
+        // entry and exit crossings of voxel i
+        auto lo_of = [&](int k) { return st > 0 ? plane(c, k) : plane(c, k + 1); };
+        auto hi_of = [&](int k) { return st > 0 ? plane(c, k + 1) : plane(c, k); };
+        while (lo_of(i) > ain && i - st >= 0 && i - st < n[c])
+            i -= st;
+        while (hi_of(i) <= ain && i + st >= 0 && i + st < n[c])
+            i += st;
+        ii[c] = i;
+        hi[c] = hi_of(i);
+        stp[c] = st;
+    }
+    KvSeg *out = seg + (size_t)id * g.seg_stride;
+    const int cap = g.seg_stride - KV_SEG_PAD;
+    float a = ain, longest = 0.f;
+    unsigned row = 0;
+    int m = 0;
+    while (m < cap) {
+        const float best = fminf(hi[0], hi[1]);
+        const float b = fminf(1.f, best);
+        if (b > a) {
+            row = (((unsigned)ii[1] * (unsigned)g.ny + (unsigned)ii[0]) * (unsigned)g.nx) * 4u;
+            out[m++] = KvSeg{b, row};
+            longest = fmaxf(longest, b - a);
+            a = b;
+        }
+        if (best >= aout)
+            break;
+        const int c = hi[0] == best ? 0 : 1;
+        ii[c] += stp[c];
+        hi[c] = stp[c] > 0 ? plane(c, ii[c] + 1) : plane(c, ii[c]);
+    }
+    head[id] = KvSegHead{ain, a, longest, m};
+    for (int k = 0; k < KV_SEG_PAD; ++k)
+        out[m + k] = KvSeg{a, row};
+}
+
+// Length in mm of a ray from the source to its pixel, as ray_setup_a.
+__device__ __forceinline__ float ray_length(const KvGeom &g, int p, int u, int v)
+{
+    RayF f;
+    ray_setup(g, p, u, v, f);
+    const float lx = f.dx * g.sx, ly = f.dy * g.sy, lz = f.dz * g.sz;
+    return sqrtf(lx * lx + ly * ly + lz * lz);
+}
+
+// Epilogue of the mode-A forward pass for the line integral ax of a ray.
+template <int EP>
+__device__ __forceinline__ void fp_a_store(const KvGeom &g, const KvTables &t, float ax, float *__restrict__ out,
+                                           const float *__restrict__ data, int p, int u, int v)
+{
+    const size_t o = ((size_t)p * g.nv + v) * g.nu + u;
+    if (EP == KV_EP_PLAIN) {
+        out[o] = ax;
+    } else {
+        // MLEM ratio on line-integral data, stored premultiplied by the
+        // ray's length factor as the mode-A backprojector weighs it (its
+        // tables' sqrt((lx2 + ly2) + lz2), the same FP32 product it would
+        // form per pixel)
+        const float L = sqrtf((t.lx2[(size_t)p * g.nu + u] + t.ly2[(size_t)p * g.nv + v]) + t.lz2[p]);
+        out[o] = ax > 0.f ? L * (data[o] / ax) : 0.f;
+    }
+}
+
 // One ray of the mode-A forward pass with its epilogue.
 template <int EP>
 __device__ __forceinline__ void fp_a_ray(const KvGeom &g, const KvTables &t, const float *__restrict__ vol,
@@ -764,17 +1195,22 @@ __device__ __forceinline__ void fp_a_ray(const KvGeom &g, const KvTables &t, con
     AccA a;
     a.init(g, vol);
     walk_a(r, [&](bool ok, unsigned k, float len) { a.visit(ok, k, len); });
-    const float ax = r.L * a.sum();
-    if (EP == KV_EP_PLAIN) {
-        out[o] = ax;
-    } else {
-        // MLEM ratio on line-integral data, stored premultiplied by the
-        // ray's length factor as the mode-A backprojector weighs it (its
-        // tables' sqrt((lx2 + ly2) + lz2), the same FP32 product it would
-        // form per pixel)
-        const float L = sqrtf((t.lx2[(size_t)p * g.nu + u] + t.ly2[(size_t)p * g.nv + v]) + t.lz2[p]);
-        out[o] = ax > 0.f ? L * (data[o] / ax) : 0.f;
-    }
+    fp_a_store<EP>(g, t, r.L * a.sum(), out, data, p, u, v);
+}
+
+// The same for column u of a row whose p and v are wavefront-uniform, along
+// the row's segment list.
+template <int EP>
+__device__ __forceinline__ void fp_a_row(const KvGeom &g, const KvTables &t, const float *__restrict__ vol,
+                                         float *__restrict__ out, const float *__restrict__ data, int p, int u, int v)
+{
+    const bool live = u < g.nu;
+    u = live ? u : g.nu - 1;
+    float sum;
+    const float *vols[1] = {vol};
+    row_sums<1>(g, vols, p, u, v, &sum);
+    if (live)
+        fp_a_store<EP>(g, t, ray_length(g, p, u, v) * sum, out, data, p, u, v);
 }
 
 template <int EP>
@@ -787,6 +1223,28 @@ __global__ __launch_bounds__(256) void fp_a_kernel(KvGeom g, KvTables t, const f
     if (u >= g.nu || v >= g.nv)
         return;
     fp_a_ray<EP>(g, t, vol, out, data, p, u, v);
+}
+
+// Pixel of this lane in the row-by-row walks, whose tiles are 64 columns by 4
+// rows, one row per wavefront: the row is wavefront-uniform (a scalar).  The
+// launch order's tx counts KV_ROW_CY tiles of consecutive rows per column, so
+// that a chunk's workgroups follow each other on one XCD.
+__device__ __forceinline__ void fp_row_pixel(int tx, int ty, int &u, int &v)
+{
+    u = tx / KV_ROW_CY * 64 + (int)(threadIdx.x & 63);
+    v = (ty * KV_ROW_CY + tx % KV_ROW_CY) * 4 + __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+}
+
+template <int EP>
+__global__ __launch_bounds__(256) void fp_a_row_kernel(KvGeom g, KvTables t, const float *__restrict__ vol,
+                                                       float *__restrict__ out, const float *__restrict__ data,
+                                                       KvFpMap fm)
+{
+    int tx, ty, p, u, v;
+    fp_xcd_tile(fm, tx, ty, p);
+    fp_row_pixel(tx, ty, u, v);
+    if (v < g.nv && __any(u < g.nu))
+        fp_a_row<EP>(g, t, vol, out, data, p, u, v);
 }
 
 // Mode-A forward projections of NV <= 3 volumes in one walk per ray: one
@@ -878,13 +1336,46 @@ __global__ __launch_bounds__(256) void fp_a_multi_kernel(KvGeom g, const float *
     }
 }
 
+// The same along the rows' segment lists: each volume's rows are read as
+// they lie (neighbouring voxels of one row are neighbouring lanes), so
+// several volumes need no interleaved copy.
+template <int NV>
+__global__ __launch_bounds__(256) void fp_a_row_multi_kernel(KvGeom g, KvMulti m, KvFpMap fm)
+{
+    int tx, ty, p, u, v;
+    fp_xcd_tile(fm, tx, ty, p);
+    fp_row_pixel(tx, ty, u, v);
+    if (v >= g.nv || !__any(u < g.nu))
+        return;
+    const bool live = u < g.nu;
+    u = live ? u : g.nu - 1;
+    float sum[NV];
+    row_sums<NV>(g, m.vol, p, u, v, sum);
+    if (!live)
+        return;
+    const float L = ray_length(g, p, u, v);
+    const size_t o = ((size_t)p * g.nv + v) * g.nu + u;
+#pragma unroll
+    for (int i = 0; i < NV; ++i)
+        m.out[i][o] = L * sum[i];
+}
+
 // Persistent mode-A forward pass (MLEM ratio) over a batch, as
-// fp_r_batch_kernel.
+// fp_r_batch_kernel; reconstructions with segment lists run row by row.
 __global__ __launch_bounds__(256) void fp_a_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
                                                          long long total, unsigned long long *counters, int iteration)
 {
-    fp_batch_tiles(probs, nprob, total, counters, iteration, [&](const KvProblem &P, int p, int u, int v) {
-        fp_a_ray<KV_EP_MLEM>(P.g, P.t, P.vol, P.ratio, P.data, p, u, v);
+    fp_batch_tiles(probs, nprob, total, counters, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
+        int u, v;
+        if (P.g.seg_a) {
+            fp_row_pixel(tx, ty, u, v);
+            if (v < P.g.nv && __any(u < P.g.nu))
+                fp_a_row<KV_EP_MLEM>(P.g, P.t, P.vol, P.ratio, P.data, p, u, v);
+            return;
+        }
+        fp_tile_pixel(P.fp_layout, tx, ty, threadIdx.x, u, v);
+        if (u < P.g.nu && v < P.g.nv)
+            fp_a_ray<KV_EP_MLEM>(P.g, P.t, P.vol, P.ratio, P.data, p, u, v);
     });
 }
 
@@ -928,12 +1419,19 @@ __global__ void trace_kernel(KvGeom g, int mode, int nrays, const int32_t *__res
 struct FpGrid {
     int gxp, gy, chunk, views;
     KvFpMap fm{};
+    // layout 0: the row-by-row walks' chunks (fp_row_pixel)
     FpGrid(const KvGeom &g, int layout)
     {
-        const int wu = 64 / layout, wv = 4 * layout;
-        chunk = std::max(1, KV_FP_STRIPE / wu);
-        gxp = ((g.nu + wu - 1) / wu + KV_XCDS * chunk - 1) / (KV_XCDS * chunk) * (KV_XCDS * chunk);
-        gy = (g.nv + wv - 1) / wv;
+        if (layout == 0) {
+            chunk = KV_ROW_CY;
+            gxp = kv_row_tiles_x(g.nu);
+            gy = kv_row_tiles_y(g.nv);
+        } else {
+            const int wu = 64 / layout, wv = 4 * layout;
+            chunk = std::max(1, KV_FP_STRIPE / wu);
+            gxp = ((g.nu + wu - 1) / wu + KV_XCDS * chunk - 1) / (KV_XCDS * chunk) * (KV_XCDS * chunk);
+            gy = (g.nv + wv - 1) / wv;
+        }
         const unsigned long long per_view = (unsigned long long)gxp * (unsigned long long)gy * 256ull;
         views = (int)std::min<unsigned long long>((unsigned long long)g.np, 0xFFFFFFFFull / per_view);
         fm.layout = layout;
@@ -997,6 +1495,16 @@ hipError_t kv_launch_fp_a_multi(const KvGeom &g, int n, const float *const *vols
     KvMulti m{};
     for (int i = 0; i < n; ++i)
         m.vol[i] = vols[i], m.out[i] = outs[i];
+    if (g.seg_a) {
+        const FpGrid fg(g, 0);
+        return fg.run(g, [&](unsigned nb, int p0) {
+            switch (n) {
+            case 1: fp_a_row_multi_kernel<1><<<nb, 256, 0, s>>>(g, m, fg.map(p0)); break;
+            case 2: fp_a_row_multi_kernel<2><<<nb, 256, 0, s>>>(g, m, fg.map(p0)); break;
+            default: fp_a_row_multi_kernel<3><<<nb, 256, 0, s>>>(g, m, fg.map(p0)); break;
+            }
+        });
+    }
     if (n >= 2) {
         const int64_t nvox = (int64_t)g.nx * g.ny * g.nz;
         const unsigned nb = (unsigned)std::max<int64_t>(1, std::min<int64_t>(8192, (nvox + 255) / 256));
@@ -1021,6 +1529,15 @@ hipError_t kv_launch_fp_a_multi(const KvGeom &g, int n, const float *const *vols
 hipError_t kv_launch_fp_a(const KvGeom &g, const KvTables &t, const float *vol, float *out, int epilogue,
                           const float *data, hipStream_t s)
 {
+    if (g.seg_a && epilogue != KV_EP_COUNT) {
+        const FpGrid fg(g, 0);
+        return fg.run(g, [&](unsigned nb, int p0) {
+            if (epilogue == KV_EP_PLAIN)
+                fp_a_row_kernel<KV_EP_PLAIN><<<nb, 256, 0, s>>>(g, t, vol, out, data, fg.map(p0));
+            else
+                fp_a_row_kernel<KV_EP_MLEM><<<nb, 256, 0, s>>>(g, t, vol, out, data, fg.map(p0));
+        });
+    }
     const int L = KV_FP_LAYOUT;
     const FpGrid fg(g, L);
     return fg.run(g, [&](unsigned nb, int p0) {
@@ -1031,6 +1548,12 @@ hipError_t kv_launch_fp_a(const KvGeom &g, const KvTables &t, const float *vol, 
         else
             fp_a_kernel<KV_EP_MLEM><<<nb, 256, 0, s>>>(g, t, vol, out, data, fg.map(p0));
     });
+}
+
+hipError_t kv_launch_seg_a(const KvGeom &g, KvSeg *seg, KvSegHead *head, hipStream_t s)
+{
+    seg_a_kernel<<<(unsigned)(((int64_t)g.np * g.nv + 63) / 64), 64, 0, s>>>(g, seg, head);
+    return hipGetLastError();
 }
 
 hipError_t kv_launch_trace(const KvGeom &g, int mode, int nrays, const int32_t *rays, int cap, int64_t *idx, float *w,

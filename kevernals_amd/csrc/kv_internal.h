@@ -32,11 +32,34 @@ struct KvGeom {
     // dx = qx - sx_p) and 1 / dx (0 when dx = 0); then the same per view
     // and detector row for y.
     const float *rc;
+    // Mode-A forward walk of a detector row: the (y, z) segments its rays
+    // share (KvSeg lists of seg_stride entries per view and row, built by
+    // kv_set_geometry), and per list its alpha range and count.  Null when the lists would exceed
+    // KV_SEG_MAX_BYTES: the rays are then walked voxel by voxel.
+    const struct KvSeg *seg_a;
+    const struct KvSegHead *seg_a_head;
+    int seg_stride;
     int walk_fast;  // forward walk may use end thresholds and 24-bit indices (see kv_fp.hip)
     int bp_posz;    // every view's z planes at alpha >= 1e-6: clamped backprojection weights (see kv_bp.hip)
 };
 
 constexpr int KV_RC = 16;
+
+// One segment of a detector row's rays between two (y, z) plane crossings:
+// it ends at alpha b and lies in the volume row that starts `row` bytes into
+// the volume.  A list ends in KV_SEG_PAD empty segments, which a walk may
+// read past its last one.
+struct KvSeg {
+    float b;
+    unsigned row;
+};
+struct KvSegHead {
+    float a, end;   // first segment's start and last one's end
+    float longest;  // longest segment
+    int segs;
+};
+constexpr int KV_SEG_PAD = 16;
+constexpr size_t KV_SEG_MAX_BYTES = size_t(1) << 30;
 
 // Unsigned division by a divisor fixed for a launch: n / d =
 // (umulhi(n, m) + n) >> l for every n < 2^31, with l = ceil(log2 d) and
@@ -140,6 +163,8 @@ struct kv_context {
     float *d_det = nullptr;
     float *d_src = nullptr;
     float *d_rc = nullptr;     // KvGeom::rc
+    KvSeg *d_seg_a = nullptr;  // KvGeom::seg_a
+    KvSegHead *d_seg_a_head = nullptr;
     KvTables tab_r{};
     bool tab_r_ok = false;
     KvTables tab_a{};
@@ -219,8 +244,23 @@ constexpr int KV_XCDS = 8;
 constexpr int KV_FP_LAYOUT = 8;
 constexpr int KV_FP_LAYOUT_MULTI[KV_LL_MAX] = {8, 4, 4};
 constexpr int KV_FP_STRIPE = 32;
+// Row-by-row walks: a stripe's chunk is KV_ROW_CY tiles of 64 columns by 4
+// rows on one XCD (fp_row_pixel).  Neighbouring rows read nearly the same
+// volume rows: with one tile per chunk the rotation of stripes over the XCDs
+// sent them to different L2s (1024x1024x64 / 25 views: 3.3 ms; 4, 8 or 16
+// tiles, one or two columns wide, 3.0-3.1 ms).  4 keeps small volumes
+// balanced (256x256x32 / 15 views: 48 us; two columns by 8 tiles 51 us).
+constexpr int KV_ROW_CY = 4;
 constexpr int KV_FP_BATCH_LAYOUT_R = 8;
 constexpr int KV_FP_BATCH_LAYOUT_A = 4;
+
+// Tiles of the row-by-row walks along tx (padded to a chunk per XCD) and ty.
+inline int kv_row_tiles_x(int nu)
+{
+    const int w = 64 * KV_XCDS;
+    return (nu + w - 1) / w * KV_XCDS * KV_ROW_CY;
+}
+inline int kv_row_tiles_y(int nv) { return (nv + 4 * KV_ROW_CY - 1) / (4 * KV_ROW_CY); }
 
 hipError_t kv_launch_fp_r(const KvGeom &g, const float *vol, float *out, int epilogue, const float *data,
                           float relax, hipStream_t s);
@@ -228,12 +268,15 @@ hipError_t kv_launch_fp_r(const KvGeom &g, const float *vol, float *out, int epi
 // premultiplied by the ray's length factor from the mode-A tables t (the
 // input the mode-A backprojector expects); the other epilogues ignore t.
 // Mode-A forward projections of n <= KV_LL_MAX volumes in one walk per ray.
-// For n >= 2 the volumes are first interleaved into pack (4 floats per
-// voxel), so that one gather per step reads every volume.
+// Without segment lists (KvGeom::seg_a null), n >= 2 volumes are first
+// interleaved into pack (4 floats per voxel), so that one gather per step
+// reads every volume; pack is unused (may be null) with them.
 hipError_t kv_launch_fp_a_multi(const KvGeom &g, int n, const float *const *vols, float *pack, float *const *outs,
                                 hipStream_t s);
 hipError_t kv_launch_fp_a(const KvGeom &g, const KvTables &t, const float *vol, float *out, int epilogue,
                           const float *data, hipStream_t s);
+// Fills KvGeom::seg_a and its heads (lists of g.seg_stride entries).
+hipError_t kv_launch_seg_a(const KvGeom &g, KvSeg *seg, KvSegHead *head, hipStream_t s);
 hipError_t kv_launch_trace(const KvGeom &g, int mode, int nrays, const int32_t *rays, int cap, int64_t *idx,
                            float *w, int32_t *counts, hipStream_t s);
 hipError_t kv_launch_tables_r(const KvGeom &g, const KvTables &t, hipStream_t s);
