@@ -126,6 +126,20 @@ bool bp_posz_ok(const kv_geometry &q)
     return true;
 }
 
+// Rounding, in voxels, of an x plane's position relative to the source s in
+// the mode-R walk against exact arithmetic: the run's (-h - s) + k, and h + s
+// of the midpoint (evaluated here, plus half an ulp where the sum with k need
+// not be exact).
+float x_rounding(float h, float s, int n)
+{
+    const float neg = -h - s, pos = h + s;
+    const double e = std::fabs((double)neg + ((double)h + (double)s)) +
+                     std::fabs((double)pos - ((double)h + (double)s));
+    const bool exact = std::floor(2.f * neg) == 2.f * neg && std::fabs(neg) < 4e6f;
+    const float most = std::fabs(neg) + (float)n;
+    return (float)(1.001 * (e + (exact ? 0.0 : 6e-8 * most)));
+}
+
 // KvGeom::rc on the host: the same FP32 operations, in the same order, as
 // the per-ray set-up of the forward kernels (Projector.cu:303-319 and the
 // z terms of :54-61 and :186), so every value is bit-identical.
@@ -159,12 +173,47 @@ std::vector<float> ray_constants(const kv_geometry &q)
         c[6] = okz ? 1.f / dz : 0.f;
         c[8] = D[0] / q.sx;
         c[9] = (D[0] + (float)q.nu * q.pu) / q.sx;
+        c[10] = x_rounding(hx, c[0], q.nx);
         for (int u = 0; u < q.nu; ++u)
             axis(qx + ((size_t)p * q.nu + u) * 4, (D[0] + ((float)u + 0.5f) * q.pu) / q.sx, c[0], hx);
         for (int v = 0; v < q.nv; ++v)
             axis(qy + ((size_t)p * q.nv + v) * 4, (D[1] + ((float)v + 0.5f) * q.pv) / q.sy, c[1], hy);
     }
     return rc;
+}
+
+// Whether the mode-R walk runs row by row (kv_fp.hip): the bound on FP32
+// runs that walk_fast states, and at least the inner half of the columns that
+// meet the volume apart by less than a wavefront's window and crossing at most
+// one x plane per segment (a z slab at most).  Rays that cannot take part are
+// walked one by one in 64x1 tiles, which is slower than the 8x8 tiles of the
+// general launch (10.9 against 8.8 ms at 1024x1024x64, in an earlier form).
+// delta: KvGeom::seg_delta for the columns that meet the volume.
+bool row_r_ok(const kv_geometry &q, float &delta)
+{
+    delta = 0.f;
+    for (int p = 0; p < q.np; ++p) {
+        const double sz = (double)q.src[3 * p + 2] / q.sz, dz = (double)q.det[3 * p + 2] / q.sz - sz;
+        const double sx = (double)q.src[3 * p] / q.sx;
+        if (!(std::fabs(dz) > 1e-3))
+            return false;
+        const double a = (-0.5 * q.nz - sz) / dz, b = (0.5 * q.nz - sz) / dz;
+        const double lo = std::min(a, b), hi = std::max(a, b);
+        if (!(lo > 1e-3) || !(hi < 0.999))
+            return false;
+        double most = 0.0;
+        for (int u : {0, q.nu - 1})
+            most = std::max(most, std::fabs(((double)q.det[3 * p] + (u + 0.5) * q.pu) / q.sx - sx));
+        most = std::min(most, (0.5 * q.nx + std::fabs(sx)) / lo);
+        const double steep = 0.5 * most / std::fabs(dz);
+        const double span = 63.0 * hi * q.pu / q.sx;
+        if (!(steep < 0.9) || !(std::min(span, hi * most * 2.0) + 8.0 + 8.0 * steep <= 63.0))
+            return false;
+        const double planes = std::min(most * (hi - lo), (double)q.nx) + 4.0;
+        delta = std::max(delta, (float)(2.02 * 6e-8 * (3.2 + 0.5 * planes) + 1e-7));
+    }
+    delta = std::max(delta, 1.2e-6f);  // segments that the reference accepts (w > 1e-6)
+    return true;
 }
 
 // Entries per list of KvGeom::seg_a, or 0 if the lists would take more than
@@ -190,8 +239,42 @@ int seg_stride(const kv_geometry &q)
         }
     }
     const int64_t n = (int64_t)std::min(most + 8, q.ny + 2) + q.nz + 8 + KV_SEG_PAD;
-    const double bytes = (double)n * q.np * q.nv * sizeof(KvSeg);
+    const double bytes = (double)n * q.np * q.nv * sizeof(KvSegR);
     return bytes <= (double)KV_SEG_MAX_BYTES ? (int)n : 0;
+}
+
+// KvGeom's rc[KV_RC*p + 11, 12], row_cols and edge_cols: per view the first
+// run of columns whose rays cross no x face inside the z slab (their alpha
+// range is set by the z faces, or y faces inside it, in every row), with the
+// room that the row-by-row walk asks for (x_face_room in kv_fp.hip) and 1e-6
+// more.  Columns whose rays run along the x planes are no hindrance: mode R's
+// result for them is 0.
+void row_columns(const kv_geometry &q, std::vector<float> &rc, int &row_cols, int &edge_cols)
+{
+    row_cols = edge_cols = 0;
+    const double h = 0.5 * q.nx;
+    for (int p = 0; p < q.np; ++p) {
+        float *c = rc.data() + (size_t)KV_RC * p;
+        const float lo = std::max(0.f, std::min(c[4], c[5])), hi = std::min(1.f, std::max(c[4], c[5]));
+        int first = 0, end = 0;
+        for (int u = 0; u < q.nu && lo < hi; ++u) {
+            const float *x = rc.data() + (size_t)q.np * KV_RC + ((size_t)p * q.nu + u) * 4;
+            const double room = (h + std::fabs((double)c[0]) + q.nx) * 2.4e-7 * std::fabs((double)x[3]) + 2e-6;
+            const bool ok = std::fabs(x[0] - c[0]) <= 1e-6f ||
+                            (std::min(x[1], x[2]) + room <= lo && std::max(x[1], x[2]) - room >= hi);
+            if (ok && end == 0)
+                first = u;
+            if (ok)
+                end = u + 1;
+            else if (end != 0)
+                break;
+        }
+        int32_t f = first, e = end;
+        std::memcpy(&c[11], &f, 4);
+        std::memcpy(&c[12], &e, 4);
+        row_cols = std::max(row_cols, end - first);
+        edge_cols = std::max(edge_cols, q.nu - (end - first));
+    }
 }
 
 kv_status check_mode(int mode)
@@ -261,8 +344,12 @@ void release_geometry(kv_context *ctx)
     free_dev(ctx->d_rc);
     free_dev(ctx->d_seg_a);
     free_dev(ctx->d_seg_a_head);
+    free_dev(ctx->d_seg_r);
+    free_dev(ctx->d_seg_r_head);
     ctx->g.seg_a = nullptr;
     ctx->g.seg_a_head = nullptr;
+    ctx->g.seg_r = nullptr;
+    ctx->g.seg_r_head = nullptr;
     free_tables(ctx->tab_r);
     free_tables(ctx->tab_a);
     free_dev(ctx->d_ratio);
@@ -412,8 +499,10 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     }
     KV_TRY_HIP(hipMemcpy(ctx->d_det, q.det, (size_t)q.np * 12, hipMemcpyHostToDevice));
     KV_TRY_HIP(hipMemcpy(ctx->d_src, q.src, (size_t)q.np * 12, hipMemcpyHostToDevice));
+    int row_cols = 0, edge_cols = 0;
     {
-        const std::vector<float> rc = ray_constants(q);
+        std::vector<float> rc = ray_constants(q);
+        row_columns(q, rc, row_cols, edge_cols);
         KV_TRY_HIP(hipMemcpy(ctx->d_rc, rc.data(), rc.size() * 4, hipMemcpyHostToDevice));
     }
     KvGeom &g = ctx->g;
@@ -431,12 +520,15 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     g.seg_a = nullptr;
     g.seg_a_head = nullptr;
     g.seg_stride = seg_stride(q);
+    g.seg_r = nullptr;
+    g.seg_r_head = nullptr;
+    g.row_cols = row_cols;
+    g.edge_cols = edge_cols;
+    const size_t rows = (size_t)q.np * q.nv;
+    auto alloc = [](auto *&p, size_t n) { return hipMalloc((void **)&p, n * sizeof(*p)) == hipSuccess; };
     if (g.seg_stride > 0) {
-        const size_t rows = (size_t)q.np * q.nv;
-        if (hipMalloc((void **)&ctx->d_seg_a, rows * g.seg_stride * sizeof(KvSeg)) == hipSuccess &&
-            hipMalloc((void **)&ctx->d_seg_a_head, rows * sizeof(KvSegHead)) == hipSuccess) {
+        if (alloc(ctx->d_seg_a, rows * g.seg_stride) && alloc(ctx->d_seg_a_head, rows)) {
             KV_TRY_HIP(kv_launch_seg_a(g, ctx->d_seg_a, ctx->d_seg_a_head, ctx->stream));
-            KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
             g.seg_a = ctx->d_seg_a;
             g.seg_a_head = ctx->d_seg_a_head;
         } else {
@@ -445,6 +537,18 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
             free_dev(ctx->d_seg_a_head);
         }
     }
+    if (g.seg_stride > 0 && g.walk_fast && row_cols > 0 && row_r_ok(q, g.seg_delta)) {
+        if (alloc(ctx->d_seg_r, rows * g.seg_stride) && alloc(ctx->d_seg_r_head, rows)) {
+            KV_TRY_HIP(kv_launch_seg_r(g, ctx->d_seg_r, ctx->d_seg_r_head, ctx->stream));
+            g.seg_r = ctx->d_seg_r;
+            g.seg_r_head = ctx->d_seg_r_head;
+        } else {
+            (void)hipGetLastError();
+            free_dev(ctx->d_seg_r);
+            free_dev(ctx->d_seg_r_head);
+        }
+    }
+    KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
     ctx->has_geom = true;
     return KV_OK;
 }

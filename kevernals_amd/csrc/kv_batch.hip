@@ -50,15 +50,33 @@ kv_status fail_hip(hipError_t e, const char *what)
     return KV_ERR_DEVICE;
 }
 
-// Recomputes tile counts and the batch-wide item ranges.
+// Recomputes tile counts and the batch-wide item ranges.  The first n
+// descriptors are the reconstructions; those of mode R that run row by row
+// get a second one for their other columns (KvFpPart).
 void layout_items(kv_batch *b)
 {
+    b->probs.resize((size_t)b->n);
+    for (int i = 0; i < b->n; ++i) {
+        KvProblem &P = b->probs[(size_t)i];
+        P.owner = i;
+        P.fp_part = (b->mode == KV_MODE_A ? P.g.seg_a != nullptr : P.g.seg_r != nullptr) ? KV_FP_ROWS : KV_FP_WHOLE;
+    }
+    for (int i = 0; b->mode == KV_MODE_R && i < b->n; ++i)
+        if (b->probs[(size_t)i].fp_part == KV_FP_ROWS) {
+            KvProblem E = b->probs[(size_t)i];
+            E.fp_part = KV_FP_EDGES;
+            b->probs.push_back(E);
+        }
     long long fp = 0, bp = 0;
     for (auto &P : b->probs) {
-        if (P.g.seg_a && b->mode == KV_MODE_A) {
+        if (P.fp_part == KV_FP_ROWS) {
             P.fp_chunk = KV_ROW_CY;
-            P.fp_tx = kv_row_tiles_x(P.g.nu);
+            P.fp_tx = kv_row_tiles_x(b->mode == KV_MODE_A ? P.g.nu : P.g.row_cols);
             P.fp_ty = kv_row_tiles_y(P.g.nv);
+        } else if (P.fp_part == KV_FP_EDGES) {
+            P.fp_chunk = KV_FP_STRIPE / KV_FP_TILE;
+            P.fp_tx = kv_edge_tiles_x(P.g.edge_cols);
+            P.fp_ty = kv_edge_tiles_y(P.g.nv);
         } else {
             const int L = P.fp_layout, wu = 64 / L;
             P.fp_chunk = std::max(1, KV_FP_STRIPE / wu);
@@ -66,8 +84,7 @@ void layout_items(kv_batch *b)
             P.fp_tx = ((P.g.nu + wu - 1) / wu + span - 1) / span * span;
             P.fp_ty = (P.g.nv + 4 * L - 1) / (4 * L);
         }
-        const int span = KV_XCDS * P.fp_chunk;
-        P.fp_nch = P.fp_tx / span;
+        P.fp_nch = P.fp_tx / (KV_XCDS * P.fp_chunk);
         P.fp_dchunk = kv_udiv((unsigned)P.fp_chunk);
         P.fp_dnch = kv_udiv((unsigned)P.fp_nch);
         P.fp_dty = kv_udiv((unsigned)P.fp_ty);
@@ -75,7 +92,7 @@ void layout_items(kv_batch *b)
         fp += (long long)P.g.np * P.fp_ty * (P.fp_tx / KV_XCDS);
         P.bp_bx = (P.g.nx + 63) / 64;
         P.bp_by = (P.g.ny + 3) / 4;
-        P.bp_bz = (P.g.nz + P.bp_zt - 1) / P.bp_zt;
+        P.bp_bz = P.fp_part == KV_FP_EDGES ? 0 : (P.g.nz + P.bp_zt - 1) / P.bp_zt;
         P.bp_first = bp;
         bp += (long long)P.bp_bx * P.bp_by * P.bp_bz;
     }
@@ -85,6 +102,8 @@ void layout_items(kv_batch *b)
 
 kv_status upload_probs(kv_batch *b)
 {
+    for (size_t i = (size_t)b->n; i < b->probs.size(); ++i)
+        b->probs[i].iters = b->probs[(size_t)b->probs[i].owner].iters;
     const hipError_t e = hipMemcpyAsync(b->d_probs, b->probs.data(), b->probs.size() * sizeof(KvProblem),
                                         hipMemcpyHostToDevice, b->stream);
     return e == hipSuccess ? KV_OK : fail_hip(e, "upload of batch descriptors");
@@ -121,7 +140,7 @@ hipError_t enqueue_iterations(kv_batch *b, int iters, float relax)
     hipError_t e = kv_launch_zero_u64(b->d_counters, kCountersPerIter * iters, b->stream);
     for (int k = 0; k < iters && e == hipSuccess; ++k) {
         unsigned long long *c = b->d_counters + (size_t)kCountersPerIter * k;
-        e = kv_launch_fp_batch(b->mode, b->d_probs, b->n, b->fp_total, c, k, relax, b->fp_grid, b->stream);
+        e = kv_launch_fp_batch(b->mode, b->d_probs, (int)b->probs.size(), b->fp_total, c, k, relax, b->fp_grid, b->stream);
         if (e == hipSuccess)
             e = kv_launch_bp_batch(b->mode, b->d_probs, b->n, b->bp_total, c + KV_XCDS, k, b->bp_grid, b->stream);
     }
@@ -303,7 +322,7 @@ kv_status kv_batch_create(int device, int n, const kv_geometry *geoms, int mode,
     }
     if (st == KV_OK) {
         layout_items(b);
-        e = hipMalloc((void **)&b->d_probs, (size_t)n * sizeof(KvProblem));
+        e = hipMalloc((void **)&b->d_probs, 2 * (size_t)n * sizeof(KvProblem));
         if (e != hipSuccess)
             st = fail_hip(e, "descriptor allocation");
     }

@@ -127,6 +127,20 @@ __device__ __forceinline__ float selm(unsigned long long mask, float a, float b)
     return __builtin_amdgcn_inverse_ballot_w64(mask) ? a : b;
 }
 
+// Distance in alpha from an x face within which the rounding of positions
+// (some ulps of the coordinates, in voxels) may matter.
+__device__ __forceinline__ float x_face_room(float h, float s, int n, float inc)
+{
+    return (h + fabsf(s) + (float)n) * 2.4e-7f * inc + 1e-6f;
+}
+
+// A wavefront-uniform value in a scalar register.
+__device__ __forceinline__ double uniform(double a)
+{
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(a)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(a)));
+}
+
 // min(1, a) as one instruction (a is never NaN where it is used).
 __device__ __forceinline__ float min1(float a)
 {
@@ -403,7 +417,23 @@ __device__ __forceinline__ void walk_r(const KvGeom &g, const RayF &r, Visit &&v
     }
 }
 
-// AlmostEqualRelative(v, 0) of commons/Maths.h:25-34 in FP32.
+// Epilogue of the mode-R forward pass for the value fp of ray o.
+template <int EP>
+__device__ __forceinline__ void fp_r_store(float fp, float *__restrict__ out, const float *__restrict__ data,
+                                           float relax, size_t o)
+{
+    if (EP == KV_EP_PLAIN) {
+        out[o] = fp;
+    } else if (EP == KV_EP_MLEM) {
+        // Reconstructors.h:207-213: the ratio overwrites the projection
+        // unless it is (almost) zero, where the projection value stays.
+        out[o] = almost_equal_zero(fp) ? fp : relax * (data[o] / fp);
+    } else {
+        // Reconstructors.h:90-93
+        out[o] = relax * (data[o] - fp);
+    }
+}
+
 // One ray of the mode-R forward pass with its epilogue.
 template <int EP>
 __device__ __forceinline__ void fp_r_ray(const KvGeom &g, const float *__restrict__ vol, float *__restrict__ out,
@@ -442,17 +472,7 @@ __device__ __forceinline__ void fp_r_ray(const KvGeom &g, const float *__restric
         walk_r<false>(g, r, acc);
     tw = tw + pw;
     tot = tot + kv_mul_legacy(pw, pv);
-    const float fp = tw > 1e-6f ? tot / tw : 0.f;
-    if (EP == KV_EP_PLAIN) {
-        out[o] = fp;
-    } else if (EP == KV_EP_MLEM) {
-        // Reconstructors.h:207-213: the ratio overwrites the projection
-        // unless it is (almost) zero, where the projection value stays.
-        out[o] = almost_equal_zero(fp) ? fp : relax * (data[o] / fp);
-    } else {
-        // Reconstructors.h:90-93
-        out[o] = relax * (data[o] - fp);
-    }
+    fp_r_store<EP>(tw > 1e-6f ? tot / tw : 0.f, out, data, relax, o);
 }
 
 // Pixel of lane `tid` in forward tile (tx, ty) for tile layout L (1, 2, 4 or
@@ -472,7 +492,7 @@ __device__ __forceinline__ void fp_tile_pixel(int layout, int tx, int ty, int ti
 // wavefront-uniform operands it runs on the scalar unit.
 __device__ __forceinline__ unsigned udiv(unsigned n, KvUDiv d) { return (__umulhi(n, d.m) + n) >> d.l; }
 
-// Forward tile of this workgroup in an XCD-aware order.  Workgroups are
+// Forward tile of workgroup w in an XCD-aware order.  Workgroups are
 // handed to the eight XCDs round-robin by linear id.  The launch is
 // one-dimensional over gxp x gy x np tiles; tile columns are grouped in
 // stripes of `chunk` tiles, and each XCD walks its stripes column-fastest,
@@ -492,10 +512,9 @@ __device__ __forceinline__ unsigned udiv(unsigned n, KvUDiv d) { return (__umulh
 // divisions by chunk, the stripe count and gy use precomputed multipliers
 // (they were a tenth of the vector instructions a wavefront issues before
 // its walk).
-__device__ __forceinline__ void fp_xcd_tile(const KvFpMap &fm, int &tx, int &ty, int &p)
+__device__ __forceinline__ void fp_xcd_tile(const KvFpMap &fm, unsigned w, int &tx, int &ty, int &p)
 {
     constexpr unsigned X = KV_XCDS;
-    const unsigned w = blockIdx.x;
     const unsigned j = w / X;
     const unsigned jc = udiv(j, fm.dchunk), t = j - jc * (unsigned)fm.chunk;
     const unsigned r = udiv(jc, fm.dnch), ci = jc - r * (unsigned)fm.nch;
@@ -510,17 +529,24 @@ __global__ __launch_bounds__(256) void fp_r_kernel(KvGeom g, const float *__rest
                                                    const float *__restrict__ data, float relax, KvFpMap fm)
 {
     int tx, ty, p, u, v;
-    fp_xcd_tile(fm, tx, ty, p);
+    fp_xcd_tile(fm, blockIdx.x, tx, ty, p);
     fp_tile_pixel(fm.layout, tx, ty, threadIdx.x, u, v);
     if (u >= g.nu || v >= g.nv)
         return;
     fp_r_ray<EP>(g, vol, out, data, relax, p, u, v);
 }
 
+// Tiles per claim of the batch kernels, at most.  The claims of a list are
+// atomics on one word, some 70 ns each: a mode-R / mode-A iteration of six
+// reconstructions of 384x320x48 and less (18 000 tiles a list) took 1.67 /
+// 1.65 ms with one tile per claim, 0.96 / 0.90 with four, 0.96 / 0.84 with
+// eight.
+constexpr int KV_FP_CLAIM = 8;
+
 // Persistent forward pass over a batch of reconstructions.  The tiles sit in
 // KV_XCDS lists (KvProblem), list k holding the stripes an XCD-ordered
 // launch gives XCD k (fp_xcd_tile); `total` items per list, one counter per
-// list.  A workgroup claims tiles from the list of the XCD a one-dimensional
+// list.  A workgroup claims `per` tiles at a time from the list of the XCD a one-dimensional
 // launch places it on (blockIdx.x % KV_XCDS), then from the other lists in
 // turn, until every list is exhausted: every tile is processed once whatever
 // the placement, which only decides the caches' locality.  Problems whose
@@ -528,20 +554,36 @@ __global__ __launch_bounds__(256) void fp_r_kernel(KvGeom g, const float *__rest
 // detector) are skipped at the bounds test.
 template <typename Tile>
 __device__ __forceinline__ void fp_batch_tiles(const KvProblem *__restrict__ probs, int nprob, long long total,
-                                               unsigned long long *counters, int iteration, Tile &&tile)
+                                               unsigned long long *counters, int per, int iteration, Tile &&tile)
 {
     __shared__ long long item_s;
     const int own = (int)(blockIdx.x % (unsigned)KV_XCDS);
     for (int c = 0; c < KV_XCDS; ++c) {
         const int k = (own + c) % KV_XCDS;
-        for (;;) {
-            if (threadIdx.x == 0)
-                item_s = (long long)atomicAdd(counters + k, 1ull);
-            __syncthreads();
-            const long long item = item_s;
-            __syncthreads();
-            if (item >= total)
-                break;
+        // the next claim is in flight while this one's tiles are walked
+        long long claim = 0;
+        if (threadIdx.x == 0)
+            claim = (long long)atomicAdd(counters + k, (unsigned long long)per);
+        for (long long item = 0, end = 0;; ++item) {
+            if (item >= end) {
+                if (threadIdx.x == 0)
+                    item_s = claim;
+                __syncthreads();
+                // the same for the workgroup: in scalar registers, and with
+                // it the descriptor's fields and the tile's row (left to
+                // itself the compiler takes a value read from LDS to differ
+                // between lanes, and reads them by vector loads)
+                const long long claimed = item_s;
+                item = (long long)(
+                    ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(claimed >> 32)) << 32) |
+                    (unsigned)__builtin_amdgcn_readfirstlane((int)claimed));
+                __syncthreads();
+                if (item >= total)
+                    break;
+                end = min(item + per, total);
+                if (threadIdx.x == 0)
+                    claim = (long long)atomicAdd(counters + k, (unsigned long long)per);
+            }
             int pi = 0;
             while (pi + 1 < nprob && probs[pi + 1].fp_first <= item)
                 ++pi;
@@ -560,19 +602,6 @@ __device__ __forceinline__ void fp_batch_tiles(const KvProblem *__restrict__ pro
             tile(P, p, tx, ty);
         }
     }
-}
-
-template <int EP>
-__global__ __launch_bounds__(256) void fp_r_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
-                                                         long long total, unsigned long long *counters, int iteration,
-                                                         float relax)
-{
-    fp_batch_tiles(probs, nprob, total, counters, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
-        int u, v;
-        fp_tile_pixel(P.fp_layout, tx, ty, threadIdx.x, u, v);
-        if (u < P.g.nu && v < P.g.nv)
-            fp_r_ray<EP>(P.g, P.vol, P.ratio, P.data, relax, p, u, v);
-    });
 }
 
 // ---------------------------------------------------------------- mode A --
@@ -895,7 +924,7 @@ __device__ __forceinline__ void seg_sums(const KvRsrc (&rs)[NV], int nx, KvSegC 
             // another turn on this segment as long as some lane with a plane
             // ahead in it is inside the volume (the others read 0 whatever
             // their weights), so at most nx turns
-            if (__builtin_amdgcn_ballot_w64(l.hx < b && (unsigned)l.j < (unsigned)nx) == 0) {
+            if ((__builtin_amdgcn_ballot_w64(l.hx < b) & __builtin_amdgcn_ballot_w64((unsigned)l.j < (unsigned)nx)) == 0) {
                 ++n;
                 b = nb;
                 row = nrow;
@@ -1151,6 +1180,393 @@ __global__ __launch_bounds__(64) void seg_a_kernel(KvGeom g, KvSeg *__restrict__
         out[m + k] = KvSeg{a, row};
 }
 
+// ------------------------------------------------- mode R, row by row ----
+// As in mode A, the 64 rays of a wavefront on one detector row share the y
+// and z planes.  The reference's runs depend on the ray's alpha range: a run
+// starts at the first plane after alpha_min and sums its increment in FP32.
+// Where the y and z faces set the range, the y run and the z run are the same
+// values for the whole row; their merge is a list built once per geometry
+// (seg_r_kernel), and a lane merges in only its own x run.  The columns whose
+// rays cross no x face inside the z slab are one interval per view (rc[KV_RC p
+// + 11, 12]); the others are walked voxel by voxel in 8x8 tiles by the same
+// launch (a tenth of the rays that meet a 1024x1024x64 volume).
+//
+// A segment [a, b] of the list and at most one x crossing c in it give the
+// reference's segments [a, b], or [a, c] and [c, b].  The reference finds
+// each one's voxel from its midpoint in FP64.  That voxel is the one that
+// stepping from plane to plane gives unless the midpoint lies closer to a
+// plane than the rounding of the run values (about 1e-6 in alpha against a
+// mean segment of 5e-4):
+//  * y and z: the builder finds, in FP64, the sums of two list values
+//    between which the midpoint's row is the segment's own.  It flags
+//    segments whose own midpoint fails, or which the reference rejects, and
+//    turns the bounds into an interval of c (m, r).
+//  * x: a run value differs from the plane's crossing, as the FP64 midpoint
+//    formula has it, by at most E = P/|d| + 2^-24 (3 + n/2) after n
+//    additions of values below 1: P the rounding of the plane's position
+//    (rc[KV_RC p + 10], voxels), 2^-25 per addition, 1/d's rounding in the
+//    first value (2^-24) and in n increments (2^-24 in all), the first
+//    product's and the midpoint sum's (2^-25 each).  A segment longer than
+//    delta = 2 E therefore has its midpoint between the planes that bound
+//    it; delta also covers the acceptance w > 1e-6.
+// Lanes whose c lies within delta of an end of the interval look up the x
+// index in FP64 (one segment in ten of a wavefront), lanes outside it and
+// flagged segments take the reference's whole arithmetic (one in 50).
+// Likewise the x entries before the list's first value and everything after
+// its last one.  Within 4e-5 of the row's alpha range's ends a segment is
+// flagged, so that the ends of the x run (which planes the FP32 positions of
+// Projector.cu:88-120 include) need no thought elsewhere: a run value past
+// the run's end lies beyond alpha_max less that margin.
+//
+// A step of walk_r takes 32.5 vector instructions; a segment, 1.25 steps on
+// average, takes 18 here and one row load instead of gathers.  Forward pass of
+// 1024x1024x64 / 25 views of 2048^2 6.45 -> 4.43 ms, 512x512x48 / 21 views of
+// 1024^2 0.79 -> 0.55, 256x256x32 / 15 views of 512^2 0.087 -> 0.073, 128x128x32
+// / 15 views of 256^2 0.026 -> 0.025 (bound by the latency of a wavefront).
+
+typedef const __attribute__((address_space(4))) KvSegHeadR KvSegHeadRC;
+typedef const __attribute__((address_space(4))) KvSegR KvSegRC;
+typedef unsigned KvSegBlockR __attribute__((ext_vector_type(4 * SEG_DEPTH)));
+typedef const __attribute__((address_space(4), aligned(16))) KvSegBlockR KvSegBlockRC;
+
+// One lane's x run: head, increment, end threshold (walk_r), x index in bytes
+// of a row, and twice the bound E.
+struct LaneR {
+    float hx, inc, tx, delta;
+    int at, dat;
+};
+
+// Ray sums (tot, tw) of the lanes in mask `in` along a row's segment list.
+__device__ __forceinline__ void seg_sums_r(const KvGeom &g, const float *__restrict__ vol, const RayF &r,
+                                           KvSegHeadRC *hp, KvSegRC *sp, unsigned long long in, int below, int above,
+                                           LaneR &l, float &tot, float &tw)
+{
+    // (the y and z terms are uniform: scalar registers)
+    const double bx = uniform((double)(r.hx + r.sx)), by = uniform((double)(r.hy + r.sy)),
+                 bz = uniform((double)(r.hz + r.sz));
+    const double hdx = 0.5 * (double)r.dx, hdy = uniform(0.5 * (double)r.dy), hdz = uniform(0.5 * (double)r.dz);
+    const unsigned nx = (unsigned)g.nx, ny = (unsigned)g.ny, nz = (unsigned)g.nz, nxy = nx * ny;
+    const KvRsrc vrs = voxel_rsrc(g, vol);
+    // the reference's segment (prev, cur): its weight, 0 if rejected, and
+    // its voxel
+    auto exact = [&](float prev, float cur, float &w, float &val) {
+        const double sum = (double)(cur + prev);
+        const int vx = (int)__builtin_fma(sum, hdx, bx);
+        const int vy = (int)__builtin_fma(sum, hdy, by);
+        const int vz = (int)__builtin_fma(sum, hdz, bz);
+        const float d = cur - prev;
+        const bool ok = (unsigned)vx < nx && (unsigned)vy < ny && (unsigned)vz < nz && d > 1e-6f;
+        const unsigned k = mad_u24((unsigned)vz, nxy, mad_u24((unsigned)vy, nx, (unsigned)vx));
+        val = kv_struct_load_f32(vrs, (int)k, 0, 0, 0);
+        w = ok ? d : 0.f;
+    };
+    auto add = [&](float w, float val) {
+        tw = tw + w;
+        tot = tot + kv_mul_legacy(w, val);
+    };
+    auto one = [&](float prev, float cur) {
+        float w, val;
+        exact(prev, cur, w, val);
+        add(w, val);
+    };
+    auto pass = [&](bool c) {
+        const float nv = l.hx + l.inc;
+        l.hx = c ? (nv > l.tx ? kInf : nv) : l.hx;
+        l.at += c ? l.dat : 0;
+    };
+    // entries of the x run below `lim`, from the entry prev on
+    auto entries = [&](float &prev, float lim) {
+        while (__any(l.hx < lim)) {
+            const bool c = l.hx < lim;
+            const float cur = c ? l.hx : prev;
+            one(prev, cur);
+            prev = cur;
+            pass(c);
+        }
+    };
+    const int segs = hp->segs;
+    float a = hp->a;
+    if (__any(l.hx < a)) {
+        // ahead of the list: the x run's head is the first entry
+        float prev = minf(l.hx, a);
+        pass(l.hx < a);
+        entries(prev, a);
+        one(prev, a);
+    }
+    const int lane = (int)(threadIdx.x & 63);
+    const int first = __builtin_ctzll(in), last = 63 - __builtin_clzll(in);
+    KvRsrc rs = vrs;
+    rs.z = g.nx;  // one row's voxels: the row is the scalar offset
+    KvSegBlockR q, nq, mq;
+    auto read = [&](KvSegBlockR &d) {
+        d = *(KvSegBlockRC *)sp;
+        sp += SEG_DEPTH;
+    };
+    auto arrived = [](KvSegBlockR &d) { asm volatile("" : "+s"(d)); };
+    float ra[SEG_DEPTH], rb[SEG_DEPTH];
+    auto rows = [&](const KvSegBlockR &d, float (&row)[SEG_DEPTH]) {
+        const int j0 = __builtin_amdgcn_readlane(l.at, first) >> 2, j1 = __builtin_amdgcn_readlane(l.at, last) >> 2;
+        const int base = min(j0, j1) - 1 - below, width = max(j0, j1) + 2 + above - base;
+        const int of = (lane - base) & 63;
+        const int i = of < width ? base + of : -1;
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k)
+            row[k] = kv_struct_load_f32(rs, i, 0, (int)(d[4 * k + 1] & ~1u), 0);
+    };
+    auto walk = [&](const KvSegBlockR &d, const float (&row)[SEG_DEPTH]) {
+        float w1[SEG_DEPTH], w2[SEG_DEPTH], v1[SEG_DEPTH], v2[SEG_DEPTH];
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k) {
+            const float b = __uint_as_float(d[4 * k]), off = fabsf(l.hx - __uint_as_float(d[4 * k + 2])),
+                        r = __uint_as_float(d[4 * k + 3]);
+            const unsigned long long flag = d[4 * k + 1] & 1u;
+            // (one ballot per compare: the masks combine on the scalar unit)
+            const unsigned long long cross = __builtin_amdgcn_ballot_w64(l.hx < b);
+            const unsigned long long close = cross & __builtin_amdgcn_ballot_w64(off > r - l.delta);
+            const float h0 = l.hx, x1 = minf(h0, b);
+            v1[k] = __int_as_float(__builtin_amdgcn_ds_bpermute(l.at, __float_as_int(row[k])));
+            w1[k] = x1 - a;
+            w2[k] = b - x1;
+            const int at0 = l.at;
+            l.hx = selm(cross, h0 + l.inc, h0);
+            l.at = at0 + __float_as_int(selm(cross, __int_as_float(l.dat), 0.f));
+            v2[k] = __int_as_float(__builtin_amdgcn_ds_bpermute(l.at, __float_as_int(row[k])));
+            if (close | flag) {
+                // a crossing close to a plane, or a flagged segment
+                const float h = h0 > l.tx ? kInf : h0;
+                const unsigned long long c = __builtin_amdgcn_ballot_w64(h < b);
+                const float y1 = minf(h, b);
+                l.hx = selm(c, h + l.inc, h);
+                l.at = at0 + __float_as_int(selm(c, __int_as_float(l.dat), 0.f));
+                float e1, e2, u1, u2;
+                if ((c & __builtin_amdgcn_ballot_w64(off > r)) | flag) {
+                    // flagged, or close to a y or z plane.  The gathers are
+                    // waited for here: left in flight, they would make the
+                    // common path wait too, for the row loads behind them.
+                    exact(a, y1, e1, u1);
+                    exact(y1, b, e2, u2);
+                    asm volatile("" : "+v"(u1), "+v"(u2));
+                } else {
+                    // close to an x plane: the row is the segment's
+                    const int i1 = (int)__builtin_fma((double)(y1 + a), hdx, bx),
+                              i2 = (int)__builtin_fma((double)(b + y1), hdx, bx);
+                    u1 = __int_as_float(__builtin_amdgcn_ds_bpermute(i1 << 2, __float_as_int(row[k])));
+                    u2 = __int_as_float(__builtin_amdgcn_ds_bpermute(i2 << 2, __float_as_int(row[k])));
+                    const float d1 = y1 - a, d2 = b - y1;
+                    e1 = d1 > 1e-6f ? d1 : 0.f;
+                    e2 = d2 > 1e-6f ? d2 : 0.f;
+                }
+                v1[k] = u1;
+                v2[k] = u2;
+                w1[k] = e1;
+                w2[k] = e2;
+            }
+            a = b;
+        }
+#pragma unroll
+        for (int k = 0; k < SEG_DEPTH; ++k) {
+            add(w1[k], v1[k]);
+            add(w2[k], v2[k]);
+        }
+    };
+    read(q);
+    read(nq);
+    arrived(q);
+    arrived(nq);
+    rows(q, ra);
+    for (int i = 0; i < segs; i += 2 * SEG_DEPTH) {
+        rows(nq, rb);
+        read(mq);
+        __builtin_amdgcn_sched_barrier(0);
+        walk(q, ra);
+        __builtin_amdgcn_sched_barrier(0);
+        arrived(mq);
+        if (i + SEG_DEPTH >= segs)
+            break;
+        rows(mq, ra);
+        read(q);
+        __builtin_amdgcn_sched_barrier(0);
+        walk(nq, rb);
+        __builtin_amdgcn_sched_barrier(0);
+        arrived(q);
+        nq = q;
+        q = mq;
+    }
+    // the rest of the x run, with the fillers' 1.0 in its place
+    l.hx = l.hx > l.tx ? kInf : l.hx;
+    float prev = hp->end;
+    if (hp->filler) {
+        entries(prev, 1.f);
+        pass(l.hx == 1.f);
+        one(prev, 1.f);
+        prev = 1.f;
+    }
+    entries(prev, kInf);
+}
+
+// Column u of a row whose p and v are wavefront-uniform, with its epilogue;
+// lanes with u >= end are idle.
+template <int EP>
+__device__ __forceinline__ void fp_r_row(const KvGeom &g, const float *__restrict__ vol, float *__restrict__ out,
+                                         const float *__restrict__ data, float relax, int p, int u, int v, int end)
+{
+    const size_t id = (size_t)p * g.nv + v;
+    KvSegHeadRC *hp = (KvSegHeadRC *)(size_t)(g.seg_r_head + id);
+    KvSegRC *sp = (KvSegRC *)(size_t)(g.seg_r + id * (size_t)g.seg_stride);
+    const bool inside = u < end;
+    const size_t o = id * g.nu + u;
+    u = inside ? u : end - 1;
+    if (hp->empty) {
+        if (inside)
+            fp_r_store<EP>(0.f, out, data, relax, o);
+        return;
+    }
+    RayF r;
+    ray_setup(g, p, u, v, r);
+    const float xlo = fminf(r.a1x, r.aNx), xhi = fmaxf(r.a1x, r.aNx);
+    const float amin = hp->amin, amax = hp->amax;
+    // the reference's early exit: the ray's value is 0
+    const bool live = inside && !fsupeq(fmaxf(amin, xlo), fminf(amax, xhi), 1e-7f);
+    LaneR l;
+    l.inc = fabsf(r.ivx);
+    int lox, hix;
+    axis_range(r.dx, r.sx, r.hx, g.nx, amin, amax, lox, hix);
+    const int cx = hix - lox + 1;
+    l.delta = fmaxf(2.f * (g.rc[KV_RC * p + 10] * l.inc + 6.e-8f * (3.2f + 0.5f * (float)cx)), 1.2e-6f);
+    // the lanes that can follow the list: no x face in the row's alpha range
+    // (x_face_room), x planes farther apart than the segments' ends, and a
+    // rounding bound within the builder's
+    const float room = x_face_room(r.hx, r.sx, g.nx, l.inc);
+    const bool mine = live && xlo + room <= amin && xhi - room >= amax && l.inc > hp->longest + 2.f * l.delta &&
+                      l.delta <= g.seg_delta && hp->segs >= 0;
+    const unsigned long long in = __builtin_amdgcn_ballot_w64(mine);
+    float tot = 0.f, tw = 0.f;
+    bool done = !live;
+    if (in != 0) {
+        // distance of the lanes in voxels, as in row_sums
+        const float df = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.dx), __builtin_ctzll(in))),
+                    dl = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(r.dx), 63 - __builtin_clzll(in)));
+        const float most = fmaxf(fabsf(df), fabsf(dl));
+        const int ahead = (int)fminf(most * hp->longest * (2.f * SEG_DEPTH), 64.f) + 2;
+        const int below = __builtin_amdgcn_readfirstlane(__any(mine && r.dx < 0.f) ? ahead : 0),
+                  above = __builtin_amdgcn_readfirstlane(__any(mine && r.dx > 0.f) ? ahead : 0);
+        if (hp->end * fabsf(dl - df) + 4.f + (float)(below + above) <= 63.f && most + fabsf(r.sx) < 65536.f) {
+            l.hx = mine ? r.ivx * (-r.hx - r.sx + (float)(r.dx > 0 ? lox : hix)) : kInf;
+            l.tx = __builtin_fmaf((float)cx - 0.5f, l.inc, l.hx);
+            l.at = (r.dx > 0 ? lox - 1 : hix) * 4;
+            l.dat = r.dx > 0 ? 4 : -4;
+            seg_sums_r(g, vol, r, hp, sp, in, below, above, l, tot, tw);
+            done = done || mine;
+        }
+    }
+    if (inside && done)
+        fp_r_store<EP>(mine && tw > 1e-6f ? tot / tw : 0.f, out, data, relax, o);
+    if (inside && !done)
+        fp_r_ray<EP>(g, vol, out, data, relax, p, u, v);
+}
+
+// The mode-R segment list of one (view, detector row) per thread: the merge
+// of walk_r's y and z runs for rays whose alpha range the x faces leave
+// alone.
+__global__ __launch_bounds__(64) void seg_r_kernel(KvGeom g, KvSegR *__restrict__ seg, KvSegHeadR *__restrict__ head)
+{
+    const int id = blockIdx.x * 64 + threadIdx.x;
+    if (id >= g.np * g.nv)
+        return;
+    const int p = id / g.nv, v = id - p * g.nv;
+    RayF r;
+    ray_setup(g, p, 0, v, r);
+    KvSegHeadR H{};
+    const float amin = fmaxf(0.f, fmaxf(fminf(r.a1y, r.aNy), fminf(r.a1z, r.aNz)));
+    const float amax = fminf(1.f, fminf(fmaxf(r.a1y, r.aNy), fmaxf(r.a1z, r.aNz)));
+    H.amin = amin;
+    H.amax = amax;
+    // taking the x faces in only raises amin and lowers amax
+    H.empty = fsupeq(amin, amax, 1e-7f) ? 1 : 0;
+    if (H.empty) {
+        head[id] = H;
+        return;
+    }
+    int loy, hiy, loz, hiz;
+    axis_range(r.dy, r.sy, r.hy, g.ny, amin, amax, loy, hiy);
+    axis_range(r.dz, r.sz, r.hz, g.nz, amin, amax, loz, hiz);
+    // |d| > 1e-6 on both axes: else the face alphas are 0 and the row empty
+    float ay = r.ivy * (-r.hy - r.sy + (float)(r.dy > 0 ? loy : hiy));
+    float az = r.stz * (-r.hz - r.sz + (float)(r.dz > 0 ? loz : hiz));
+    const float iy = fabsf(r.ivy), iz = fabsf(r.stz);
+    const int dzr = hiz - loz;
+    int cy = hiy - loy + 1, cz = dzr >= 2 ? dzr - 1 : 1;
+    H.filler = dzr + 1 - cz > 0 ? 1 : 0;
+    const double by = (double)(r.hy + r.sy), bz = (double)(r.hz + r.sz);
+    const double hdy = 0.5 * (double)r.dy, hdz = 0.5 * (double)r.dz;
+    const float delta = g.seg_delta;
+    KvSegR *out = seg + (size_t)id * g.seg_stride;
+    const int cap = g.seg_stride - KV_SEG_PAD;
+    float a = fminf(ay, az), longest = 0.f;
+    H.a = a;
+    unsigned row = 0;
+    int m = 0;
+    bool whole = true;
+    auto next = [&](float cur) {
+        if (cy > 0 && ay == cur) {
+            --cy;
+            ay = cy > 0 ? ay + iy : kInf;
+        }
+        if (cz > 0 && az == cur) {
+            --cz;
+            az = cz > 0 ? az + iz : kInf;
+        }
+    };
+    next(a);
+    while (cy > 0 || cz > 0) {
+        const float b = fminf(ay, az);
+        if (m >= cap) {
+            whole = false;
+            break;
+        }
+        const double sum = (double)(b + a);
+        const double py = __builtin_fma(sum, hdy, by), pz = __builtin_fma(sum, hdz, bz);
+        const int vy = (int)py, vz = (int)pz;
+        const float w = b - a;
+        const double mid = 0.5 * sum, margin = 4e-5;
+        const bool good = (unsigned)vy < (unsigned)g.ny && (unsigned)vz < (unsigned)g.nz && w > 1e-6f && w > delta &&
+                          py >= 0.0 && pz >= 0.0 && mid >= (double)amin + margin && mid <= (double)amax - margin;
+        KvSegR e{b, row | 1u, 0.f, -kInf};
+        if (good) {
+            row = (((unsigned)vz * (unsigned)g.ny + (unsigned)vy) * (unsigned)g.nx) * 4u;
+            // sums between which the midpoint stays in row (vy, vz), in from
+            // the FP32 rounding of a sum below 2
+            const double y0 = ((double)vy - by) / hdy, y1 = ((double)(vy + 1) - by) / hdy;
+            const double z0 = ((double)vz - bz) / hdz, z1 = ((double)(vz + 1) - bz) / hdz;
+            const double lo = fmax(fmin(y0, y1), fmin(z0, z1)) + 2e-7, hi = fmin(fmax(y0, y1), fmax(z0, z1)) - 2e-7;
+            // a crossing within 1e-6 of a or b cuts off a segment that is
+            // rejected wherever it lies
+            double A = fmax(fmax((double)a, (double)amin + margin), lo - (double)a);
+            double B = fmin(fmin((double)b, (double)amax - margin), hi - (double)b);
+            A = A - (double)a <= 9.9e-7 ? (double)a : A;
+            B = (double)b - B <= 9.9e-7 ? (double)b : B;
+            e.row = row;
+            e.m = (float)(0.5 * (A + B));
+            e.r = (float)(0.5 * (B - A) - 2e-7);
+        }
+        out[m++] = e;
+        longest = fmaxf(longest, w);
+        a = b;
+        next(b);
+    }
+    // entries at or above the fillers' 1.0 are left to walk_r
+    if (!(a < 0.999f) || !(H.a > 0.f))
+        whole = false;
+    H.end = a;
+    H.longest = longest;
+    H.segs = whole ? m : -1;
+    // empty segments: a crossing x run entry is impossible (c < a), flagged
+    // or not
+    for (int k = 0; whole && k < KV_SEG_PAD; ++k)
+        out[m + k] = KvSegR{a, row, 0.f, kInf};
+    head[id] = H;
+}
+
 // Length in mm of a ray from the source to its pixel, as ray_setup_a.
 __device__ __forceinline__ float ray_length(const KvGeom &g, int p, int u, int v)
 {
@@ -1218,7 +1634,7 @@ __global__ __launch_bounds__(256) void fp_a_kernel(KvGeom g, KvTables t, const f
                                                    float *__restrict__ out, const float *__restrict__ data, KvFpMap fm)
 {
     int tx, ty, p, u, v;
-    fp_xcd_tile(fm, tx, ty, p);
+    fp_xcd_tile(fm, blockIdx.x, tx, ty, p);
     fp_tile_pixel(fm.layout, tx, ty, threadIdx.x, u, v);
     if (u >= g.nu || v >= g.nv)
         return;
@@ -1241,10 +1657,53 @@ __global__ __launch_bounds__(256) void fp_a_row_kernel(KvGeom g, KvTables t, con
                                                        KvFpMap fm)
 {
     int tx, ty, p, u, v;
-    fp_xcd_tile(fm, tx, ty, p);
+    fp_xcd_tile(fm, blockIdx.x, tx, ty, p);
     fp_row_pixel(tx, ty, u, v);
     if (v < g.nv && __any(u < g.nu))
         fp_a_row<EP>(g, t, vol, out, data, p, u, v);
+}
+
+// Columns of view p whose rays run row by row: [first, end).
+__device__ __forceinline__ void row_columns(const KvGeom &g, int p, int &first, int &end)
+{
+    const float *c = g.rc + KV_RC * p;
+    first = __float_as_int(c[11]);
+    end = __float_as_int(c[12]);
+}
+
+// Pixel of this lane in tile (tx, ty) of the other columns, in 8x8 tiles as
+// fp_tile_pixel's: those left of the interval, then those right of it;
+// u >= g.nu where there is none.
+__device__ __forceinline__ void fp_edge_pixel(const KvGeom &g, int tx, int ty, int p, int &u, int &v)
+{
+    int first, end;
+    row_columns(g, p, first, end);
+    fp_tile_pixel(KV_FP_LAYOUT, tx, ty, threadIdx.x, u, v);
+    u = u < first ? u : end + (u - first);
+}
+
+// The first `row_blocks` workgroups take the row-by-row tiles (map rm), the
+// others the tiles of the remaining columns (map em).
+template <int EP>
+__global__ __launch_bounds__(256, 7) void fp_r_row_kernel(KvGeom g, const float *__restrict__ vol,
+                                                          float *__restrict__ out, const float *__restrict__ data,
+                                                          float relax, KvFpMap rm, KvFpMap em, unsigned row_blocks)
+{
+    int tx, ty, p, u, v;
+    if (blockIdx.x < row_blocks) {
+        int first, end;
+        fp_xcd_tile(rm, blockIdx.x, tx, ty, p);
+        fp_row_pixel(tx, ty, u, v);
+        row_columns(g, p, first, end);
+        u += first;
+        if (v < g.nv && __any(u < end))
+            fp_r_row<EP>(g, vol, out, data, relax, p, u, v, end);
+        return;
+    }
+    fp_xcd_tile(em, blockIdx.x - row_blocks, tx, ty, p);
+    fp_edge_pixel(g, tx, ty, p, u, v);
+    if (u < g.nu && v < g.nv)
+        fp_r_ray<EP>(g, vol, out, data, relax, p, u, v);
 }
 
 // Mode-A forward projections of NV <= 3 volumes in one walk per ray: one
@@ -1314,7 +1773,7 @@ __global__ __launch_bounds__(256) void fp_a_multi_kernel(KvGeom g, const float *
                                                          KvFpMap fm)
 {
     int tx, ty, p, u, v;
-    fp_xcd_tile(fm, tx, ty, p);
+    fp_xcd_tile(fm, blockIdx.x, tx, ty, p);
     fp_tile_pixel(fm.layout, tx, ty, threadIdx.x, u, v);
     if (u >= g.nu || v >= g.nv)
         return;
@@ -1343,7 +1802,7 @@ template <int NV>
 __global__ __launch_bounds__(256) void fp_a_row_multi_kernel(KvGeom g, KvMulti m, KvFpMap fm)
 {
     int tx, ty, p, u, v;
-    fp_xcd_tile(fm, tx, ty, p);
+    fp_xcd_tile(fm, blockIdx.x, tx, ty, p);
     fp_row_pixel(tx, ty, u, v);
     if (v >= g.nv || !__any(u < g.nu))
         return;
@@ -1360,14 +1819,40 @@ __global__ __launch_bounds__(256) void fp_a_row_multi_kernel(KvGeom g, KvMulti m
         m.out[i][o] = L * sum[i];
 }
 
+template <int EP>
+__global__ __launch_bounds__(256) void fp_r_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
+                                                         long long total, unsigned long long *counters, int per,
+                                                         int iteration, float relax)
+{
+    fp_batch_tiles(probs, nprob, total, counters, per, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
+        int u, v;
+        if (P.fp_part == KV_FP_ROWS) {
+            int first, end;
+            fp_row_pixel(tx, ty, u, v);
+            row_columns(P.g, p, first, end);
+            u += first;
+            if (v < P.g.nv && __any(u < end))
+                fp_r_row<EP>(P.g, P.vol, P.ratio, P.data, relax, p, u, v, end);
+            return;
+        }
+        if (P.fp_part == KV_FP_EDGES)
+            fp_edge_pixel(P.g, tx, ty, p, u, v);
+        else
+            fp_tile_pixel(P.fp_layout, tx, ty, threadIdx.x, u, v);
+        if (u < P.g.nu && v < P.g.nv)
+            fp_r_ray<EP>(P.g, P.vol, P.ratio, P.data, relax, p, u, v);
+    });
+}
+
 // Persistent mode-A forward pass (MLEM ratio) over a batch, as
 // fp_r_batch_kernel; reconstructions with segment lists run row by row.
 __global__ __launch_bounds__(256) void fp_a_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
-                                                         long long total, unsigned long long *counters, int iteration)
+                                                         long long total, unsigned long long *counters, int per,
+                                                         int iteration)
 {
-    fp_batch_tiles(probs, nprob, total, counters, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
+    fp_batch_tiles(probs, nprob, total, counters, per, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
         int u, v;
-        if (P.g.seg_a) {
+        if (P.fp_part == KV_FP_ROWS) {
             fp_row_pixel(tx, ty, u, v);
             if (v < P.g.nv && __any(u < P.g.nu))
                 fp_a_row<KV_EP_MLEM>(P.g, P.t, P.vol, P.ratio, P.data, p, u, v);
@@ -1419,28 +1904,34 @@ __global__ void trace_kernel(KvGeom g, int mode, int nrays, const int32_t *__res
 struct FpGrid {
     int gxp, gy, chunk, views;
     KvFpMap fm{};
-    // layout 0: the row-by-row walks' chunks (fp_row_pixel)
-    FpGrid(const KvGeom &g, int layout)
+    // gxp must be a multiple of KV_XCDS * chunk
+    FpGrid(int gxp_, int gy_, int chunk_, int np) : gxp(gxp_), gy(gy_), chunk(chunk_)
     {
-        if (layout == 0) {
-            chunk = KV_ROW_CY;
-            gxp = kv_row_tiles_x(g.nu);
-            gy = kv_row_tiles_y(g.nv);
-        } else {
-            const int wu = 64 / layout, wv = 4 * layout;
-            chunk = std::max(1, KV_FP_STRIPE / wu);
-            gxp = ((g.nu + wu - 1) / wu + KV_XCDS * chunk - 1) / (KV_XCDS * chunk) * (KV_XCDS * chunk);
-            gy = (g.nv + wv - 1) / wv;
-        }
-        const unsigned long long per_view = (unsigned long long)gxp * (unsigned long long)gy * 256ull;
-        views = (int)std::min<unsigned long long>((unsigned long long)g.np, 0xFFFFFFFFull / per_view);
-        fm.layout = layout;
+        const unsigned long long per_view = std::max(1ull, (unsigned long long)gxp * (unsigned long long)gy * 256ull);
+        views = (int)std::min<unsigned long long>((unsigned long long)np, 0xFFFFFFFFull / per_view);
         fm.chunk = chunk;
         fm.nch = gxp / (KV_XCDS * chunk);
         fm.gy = gy;
         fm.dchunk = kv_udiv(chunk);
         fm.dnch = kv_udiv(fm.nch);
         fm.dgy = kv_udiv(gy);
+    }
+    // tiles of a layout over the whole detector
+    FpGrid(const KvGeom &g, int layout)
+        : FpGrid(tiles_x(g.nu, 64 / layout), (g.nv + 4 * layout - 1) / (4 * layout), stripe(64 / layout), g.np)
+    {
+        fm.layout = layout;
+    }
+    // the row-by-row walk over the whole detector
+    static FpGrid rows(const KvGeom &g)
+    {
+        return FpGrid(kv_row_tiles_x(g.nu), kv_row_tiles_y(g.nv), KV_ROW_CY, g.np);
+    }
+    static int stripe(int wu) { return std::max(1, KV_FP_STRIPE / wu); }
+    static int tiles_x(int nu, int wu)
+    {
+        const int span = KV_XCDS * stripe(wu);
+        return ((nu + wu - 1) / wu + span - 1) / span * span;
     }
     KvFpMap map(int p0) const
     {
@@ -1469,6 +1960,35 @@ struct FpGrid {
 hipError_t kv_launch_fp_r(const KvGeom &g, const float *vol, float *out, int epilogue, const float *data, float relax,
                           hipStream_t s)
 {
+    if (g.seg_r && epilogue != KV_EP_COUNT) {
+        const FpGrid rg(kv_row_tiles_x(g.row_cols), kv_row_tiles_y(g.nv), KV_ROW_CY, g.np),
+            eg(kv_edge_tiles_x(g.edge_cols), kv_edge_tiles_y(g.nv), KV_FP_STRIPE / KV_FP_TILE, g.np);
+        // as many views per launch as keep it within 2^32 threads
+        const unsigned long long per_view =
+            256ull * ((unsigned long long)rg.gxp * (unsigned long long)rg.gy +
+                      (unsigned long long)eg.gxp * (unsigned long long)eg.gy);
+        const int views = (int)std::min<unsigned long long>((unsigned long long)g.np, 0xFFFFFFFFull / per_view);
+        if (views < 1)
+            return hipErrorInvalidConfiguration;
+        for (int p0 = 0; p0 < g.np; p0 += views) {
+            const unsigned n = (unsigned)std::min(views, g.np - p0), rb = (unsigned)rg.gxp * (unsigned)rg.gy * n,
+                           nb = rb + (unsigned)eg.gxp * (unsigned)eg.gy * n;
+            switch (epilogue) {
+            case KV_EP_PLAIN:
+                fp_r_row_kernel<KV_EP_PLAIN><<<nb, 256, 0, s>>>(g, vol, out, data, relax, rg.map(p0), eg.map(p0), rb);
+                break;
+            case KV_EP_MLEM:
+                fp_r_row_kernel<KV_EP_MLEM><<<nb, 256, 0, s>>>(g, vol, out, data, relax, rg.map(p0), eg.map(p0), rb);
+                break;
+            default:
+                fp_r_row_kernel<KV_EP_SART><<<nb, 256, 0, s>>>(g, vol, out, data, relax, rg.map(p0), eg.map(p0), rb);
+                break;
+            }
+            if (const hipError_t e = hipGetLastError())
+                return e;
+        }
+        return hipSuccess;
+    }
     const int L = KV_FP_LAYOUT;
     const FpGrid fg(g, L);
     return fg.run(g, [&](unsigned nb, int p0) {
@@ -1496,7 +2016,7 @@ hipError_t kv_launch_fp_a_multi(const KvGeom &g, int n, const float *const *vols
     for (int i = 0; i < n; ++i)
         m.vol[i] = vols[i], m.out[i] = outs[i];
     if (g.seg_a) {
-        const FpGrid fg(g, 0);
+        const FpGrid fg = FpGrid::rows(g);
         return fg.run(g, [&](unsigned nb, int p0) {
             switch (n) {
             case 1: fp_a_row_multi_kernel<1><<<nb, 256, 0, s>>>(g, m, fg.map(p0)); break;
@@ -1530,7 +2050,7 @@ hipError_t kv_launch_fp_a(const KvGeom &g, const KvTables &t, const float *vol, 
                           const float *data, hipStream_t s)
 {
     if (g.seg_a && epilogue != KV_EP_COUNT) {
-        const FpGrid fg(g, 0);
+        const FpGrid fg = FpGrid::rows(g);
         return fg.run(g, [&](unsigned nb, int p0) {
             if (epilogue == KV_EP_PLAIN)
                 fp_a_row_kernel<KV_EP_PLAIN><<<nb, 256, 0, s>>>(g, t, vol, out, data, fg.map(p0));
@@ -1556,6 +2076,12 @@ hipError_t kv_launch_seg_a(const KvGeom &g, KvSeg *seg, KvSegHead *head, hipStre
     return hipGetLastError();
 }
 
+hipError_t kv_launch_seg_r(const KvGeom &g, KvSegR *seg, KvSegHeadR *head, hipStream_t s)
+{
+    seg_r_kernel<<<(unsigned)(((int64_t)g.np * g.nv + 63) / 64), 64, 0, s>>>(g, seg, head);
+    return hipGetLastError();
+}
+
 hipError_t kv_launch_trace(const KvGeom &g, int mode, int nrays, const int32_t *rays, int cap, int64_t *idx, float *w,
                            int32_t *counts, hipStream_t s)
 {
@@ -1566,10 +2092,12 @@ hipError_t kv_launch_trace(const KvGeom &g, int mode, int nrays, const int32_t *
 hipError_t kv_launch_fp_batch(int mode, const KvProblem *probs, int nprob, long long total,
                               unsigned long long *counters, int iteration, float relax, int grid, hipStream_t s)
 {
+    // as many tiles per claim as leave a workgroup some eight claims
+    const int per = (int)std::max<long long>(1, std::min<long long>(KV_FP_CLAIM, total * KV_XCDS / (8ll * grid)));
     if (mode == KV_MODE_A)
-        fp_a_batch_kernel<<<grid, 256, 0, s>>>(probs, nprob, total, counters, iteration);
+        fp_a_batch_kernel<<<grid, 256, 0, s>>>(probs, nprob, total, counters, per, iteration);
     else
-        fp_r_batch_kernel<KV_EP_MLEM><<<grid, 256, 0, s>>>(probs, nprob, total, counters, iteration, relax);
+        fp_r_batch_kernel<KV_EP_MLEM><<<grid, 256, 0, s>>>(probs, nprob, total, counters, per, iteration, relax);
     return hipGetLastError();
 }
 

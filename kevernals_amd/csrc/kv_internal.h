@@ -25,7 +25,11 @@ struct KvGeom {
     // (-nz/2 - sz_p) / dz and (nz/2 - sz_p) / dz and 1 / dz (the last three
     // 0 when |dz| <= 1e-6); for the backprojectors rc[KV_RC*p + 8, 9] =
     // detector corner x over sx and the far detector edge
-    // (det x + nu * pu) / sx (Projector.cu:473-492); then per view and
+    // (det x + nu * pu) / sx (Projector.cu:473-492); rc[KV_RC*p + 10] = the
+    // rounding of x plane positions relative to the source in the mode-R
+    // walk, in voxels (0 when source and half size are exact), [11] and [12] =
+    // the interval of detector columns whose rays cross no x face inside the
+    // z slab (ints); then per view and
     // detector column, at rc + KV_RC*np, four floats: the pixel-centre
     // coordinate qx = (det x + (u + 0.5) pu) / sx, the x-face alphas
     // (-nx/2 - sx_p) / dx and (nx/2 - sx_p) / dx (0 unless |dx| > 1e-6,
@@ -39,6 +43,16 @@ struct KvGeom {
     const struct KvSeg *seg_a;
     const struct KvSegHead *seg_a_head;
     int seg_stride;
+    // The same for the mode-R walk (kv_fp.hip, "mode R, row by row"): null
+    // also where too few rays could take it (row_r_ok).  seg_delta is the
+    // largest alpha distance from a segment's ends within which a lane may
+    // have to look up an x crossing's voxels one by one.
+    const struct KvSegR *seg_r;
+    const struct KvSegHeadR *seg_r_head;
+    float seg_delta;
+    // widest over the views: the interval of columns that run row by row
+    // (rc[KV_RC*p + 11, 12]), and the other columns together
+    int row_cols, edge_cols;
     int walk_fast;  // forward walk may use end thresholds and 24-bit indices (see kv_fp.hip)
     int bp_posz;    // every view's z planes at alpha >= 1e-6: clamped backprojection weights (see kv_bp.hip)
 };
@@ -57,6 +71,22 @@ struct KvSegHead {
     float a, end;   // first segment's start and last one's end
     float longest;  // longest segment
     int segs;
+};
+// Mode R: besides b and row (bit 0: look the segment's voxels up one by one),
+// an x crossing c splits the segment into two that both lie in that volume
+// row if |c - m| <= r.
+struct KvSegR {
+    float b;
+    unsigned row;
+    float m, r;
+};
+struct KvSegHeadR {
+    float a, end;      // first and last (y, z) crossing of the list
+    float amin, amax;  // the row's alpha range, x faces left out
+    float longest;
+    int segs;          // -1: walk the row's rays one by one
+    int filler;        // the list ends in entries of 1.0
+    int empty;         // no ray of the row meets the volume
 };
 constexpr int KV_SEG_PAD = 16;
 constexpr size_t KV_SEG_MAX_BYTES = size_t(1) << 30;
@@ -128,6 +158,12 @@ constexpr int KV_YZ = 8;
 // fused SART residual/update, or the count of accepted (ray, voxel) pairs.
 enum KvEpilogue { KV_EP_PLAIN = 0, KV_EP_MLEM = 1, KV_EP_SART = 2, KV_EP_COUNT = 3 };
 
+// What a batch descriptor's forward tiles are: the whole detector in tiles of
+// fp_layout, the columns (or the whole detector, mode A) that run row by row,
+// or mode R's other columns.  A mode-R reconstruction with segment lists has
+// two descriptors, the second without bricks.
+enum KvFpPart { KV_FP_WHOLE = 0, KV_FP_ROWS = 1, KV_FP_EDGES = 2 };
+
 // One reconstruction of a batch, as the persistent kernels read it (device
 // memory, wave-uniform loads).  Work items are numbered consecutively over
 // the batch.  Forward tiles sit in KV_XCDS lists, one per XCD (stripes of
@@ -144,6 +180,8 @@ struct KvProblem {
     const float *sens;         // mode A: sensitivity A^T 1
     int iters;                 // MLEM iterations for this reconstruction
     int fp_layout;             // forward tile layout: 1, 2, 4 or 8 rows per wavefront
+    int fp_part;               // KvFpPart
+    int owner;                 // index of the reconstruction (its own, or its first descriptor's)
     int fp_tx, fp_ty;          // forward tiles per view (fp_tx padded to a multiple of KV_XCDS * fp_chunk)
     int fp_chunk;              // tile columns per XCD stripe
     int fp_nch;                // stripes per tile row in one list: fp_tx / (KV_XCDS * fp_chunk)
@@ -165,6 +203,8 @@ struct kv_context {
     float *d_rc = nullptr;     // KvGeom::rc
     KvSeg *d_seg_a = nullptr;  // KvGeom::seg_a
     KvSegHead *d_seg_a_head = nullptr;
+    KvSegR *d_seg_r = nullptr;  // KvGeom::seg_r
+    KvSegHeadR *d_seg_r_head = nullptr;
     KvTables tab_r{};
     bool tab_r_ok = false;
     KvTables tab_a{};
@@ -261,6 +301,14 @@ inline int kv_row_tiles_x(int nu)
     return (nu + w - 1) / w * KV_XCDS * KV_ROW_CY;
 }
 inline int kv_row_tiles_y(int nv) { return (nv + 4 * KV_ROW_CY - 1) / (4 * KV_ROW_CY); }
+// Tiles of 8 columns by 32 rows over mode R's other columns.
+constexpr int KV_FP_TILE = 64 / KV_FP_LAYOUT;
+inline int kv_edge_tiles_x(int cols)
+{
+    const int span = KV_XCDS * (KV_FP_STRIPE / KV_FP_TILE);
+    return ((cols + KV_FP_TILE - 1) / KV_FP_TILE + span - 1) / span * span;
+}
+inline int kv_edge_tiles_y(int nv) { return (nv + 4 * KV_FP_LAYOUT - 1) / (4 * KV_FP_LAYOUT); }
 
 hipError_t kv_launch_fp_r(const KvGeom &g, const float *vol, float *out, int epilogue, const float *data,
                           float relax, hipStream_t s);
@@ -277,6 +325,8 @@ hipError_t kv_launch_fp_a(const KvGeom &g, const KvTables &t, const float *vol, 
                           const float *data, hipStream_t s);
 // Fills KvGeom::seg_a and its heads (lists of g.seg_stride entries).
 hipError_t kv_launch_seg_a(const KvGeom &g, KvSeg *seg, KvSegHead *head, hipStream_t s);
+// Fills KvGeom::seg_r and its heads.
+hipError_t kv_launch_seg_r(const KvGeom &g, KvSegR *seg, KvSegHeadR *head, hipStream_t s);
 hipError_t kv_launch_trace(const KvGeom &g, int mode, int nrays, const int32_t *rays, int cap, int64_t *idx,
                            float *w, int32_t *counts, hipStream_t s);
 hipError_t kv_launch_tables_r(const KvGeom &g, const KvTables &t, hipStream_t s);

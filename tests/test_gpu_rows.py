@@ -1,6 +1,7 @@
 """Row-by-row forward walks against the voxel-by-voxel ones.
 
-The row-by-row walks follow a detector row's segment lists; kv_trace_rays
+Mode R is compared with the oracle, the reference's own sequence of operations.
+In mode A the row-by-row walks follow a detector row's segment lists; kv_trace_rays
 records the voxels and weights of the general walk of single rays.  The
 projection is defined by those: FP32 products added in walk order, so a
 row-by-row projection must give the same bits.
@@ -108,6 +109,46 @@ def test_mode_a_rows_touch_only_their_voxels():
             assert not np.isfinite(got[r])
         else:
             assert got[r] == clean[r]
+
+
+CASES_R = {
+    # rays in the middle columns, the volume's x faces, several views
+    "wide": lambda: arc((200, 90, 20), (0.3, 0.3, 1.0), (330, 150), (0.28, 0.3), 5, 20.0),
+    # plane positions that FP32 rounds: odd sizes, sources off the grid
+    "offset": lambda: shifted(arc((167, 71, 13), (0.37, 0.41, 1.3), (215, 117), (0.43, 0.41), 4, 17.0)),
+    # one or two slices: no z entries left in the run, or no filler
+    "slices1": lambda: arc((90, 60, 1), (0.4, 0.4, 2.0), (140, 90), (0.4, 0.5), 3, 10.0),
+    "slices2": lambda: arc((90, 60, 2), (0.4, 0.4, 2.0), (140, 90), (0.4, 0.5), 3, 10.0),
+    "slices3": lambda: arc((90, 60, 3), (0.4, 0.4, 2.0), (140, 90), (0.4, 0.5), 3, 10.0),
+    # longer runs: more rounding in the run values
+    "tall": lambda: arc((140, 400, 64), (0.15, 0.15, 1.0), (260, 300), (0.14, 0.3), 3, 20.0),
+}
+
+
+def shifted(g):
+    src = g.src.copy()
+    src[:, 0] += np.float32(3.137)
+    src[:, 1] -= np.float32(1.77)
+    return g.scaled(src=src)
+
+
+@pytest.mark.parametrize("name", sorted(CASES) + sorted(CASES_R))
+def test_mode_r_rows_equal_the_oracle(name):
+    """Ray sums bit for bit on a volume without equal neighbours, so that one
+    voxel or weight taken differently shows."""
+    import torch
+
+    import kevernals_amd as K
+    from oracle.oracle import Oracle
+
+    print("case", name, flush=True)
+    g = (CASES.get(name) or CASES_R[name])()
+    rng = np.random.Generator(np.random.PCG64(11))
+    vol = rng.random(g.vol_shape, dtype=np.float32) + np.float32(0.1)
+    ctx = K.Context(0, g)
+    out = torch.empty(g.proj_shape, device="cuda")
+    ctx.forward_project(torch.from_numpy(vol).cuda(), out, K.MODE_R)
+    np.testing.assert_array_equal(out.cpu().numpy(), Oracle(g).fp_r(vol))
 
 
 @pytest.mark.parametrize("name", ["faces", "coarse"])
