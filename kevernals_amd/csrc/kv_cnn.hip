@@ -35,7 +35,7 @@ constexpr int HX = BX + 2, HY = BY + 2, HZ = BZ + 2;
 constexpr int HYX = HX * HY, HVOX = HYX * HZ;
 
 constexpr int WX = 32, WY = 4, WZ = 4, WVOX = WX * WY * WZ;
-constexpr int WHX = WX + 2, WHY = WY + 2, WHZ = WZ + 2, WHV = WHX * WHY * WHZ;
+constexpr int WHX = WX + 2, WHY = WY + 2, WHZ = WZ + 2;
 constexpr int WGRID = 512;  // weight-gradient workgroups (fixed: results do not depend on the device)
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -123,14 +123,15 @@ __device__ __forceinline__ void store4(const f32x4 &acc, int g, size_t v, const 
 // pair p: p = 0 holds dx = 0 in k-groups 0-1 and dx = 1 in k-groups 2-3,
 // p = 1 holds dx = 2 in k-groups 0-1 and zeros in 2-3; k-group g covers
 // channels 8 (g & 1) .. +7.  conv1 variants use m = 0 (k-group g holds taps
-// 8g .. 8g+7).
+// 8g .. 8g+7).  One wavefront per operand (one per variant, looping over its
+// operands, took 25 us).
 enum { WV_L2 = 0, WV_L3 = 1, WV_L4 = 2, WV_L3T = 3, WV_L2T = 4, WV_L1 = 5, WV_L4T = 6, WV_COUNT = 7 };
 constexpr int WV_OPS = 18;
 
 __global__ void pack_weights_kernel(const float *__restrict__ p, u32x4 *__restrict__ wpk, int ow1, int ow2, int ow3,
                                     int ow4)
 {
-    const int v = blockIdx.x, lane = threadIdx.x, col = lane & 15, g = lane >> 4;
+    const int v = blockIdx.x, m = blockIdx.y, lane = threadIdx.x, col = lane & 15, g = lane >> 4;
     const float *w;
     int cout, cin, tr;
     switch (v) {
@@ -142,20 +143,18 @@ __global__ void pack_weights_kernel(const float *__restrict__ p, u32x4 *__restri
     case WV_L1: w = p + ow1; cout = 16; cin = 1; tr = 0; break;
     default: w = p + ow4; cout = 1; cin = 16; tr = 1; break;
     }
-    for (int m = 0; m < WV_OPS; ++m) {
-        const int pair = m & 1, dzdy = m >> 1, dx = pair ? 2 : (g >> 1);
-        unsigned int e[8];
+    const int pair = m & 1, dzdy = m >> 1, dx = pair ? 2 : (g >> 1);
+    unsigned int e[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            float val;
-            if (v >= WV_L1)
-                val = m == 0 ? w_elem(w, cout, cin, tr, col, 0, 8 * g + j) : 0.f;
-            else
-                val = pair && g >= 2 ? 0.f : w_elem(w, cout, cin, tr, col, 8 * (g & 1) + j, 3 * dzdy + dx);
-            e[j] = f2bf(val);
-        }
-        wpk[(v * WV_OPS + m) * 64 + lane] = pack8(e);
+    for (int j = 0; j < 8; ++j) {
+        float val;
+        if (v >= WV_L1)
+            val = m == 0 ? w_elem(w, cout, cin, tr, col, 0, 8 * g + j) : 0.f;
+        else
+            val = pair && g >= 2 ? 0.f : w_elem(w, cout, cin, tr, col, 8 * (g & 1) + j, 3 * dzdy + dx);
+        e[j] = f2bf(val);
     }
+    wpk[(v * WV_OPS + m) * 64 + lane] = pack8(e);
 }
 
 // z-chunks of BZ slices per workgroup: weights loaded once per workgroup,
@@ -402,14 +401,39 @@ __global__ __launch_bounds__(256) void conv1_kernel(int nx, int ny, int nz, cons
 // blocks of 16 -- CIN 16: block t = tap t (i = column), block 27 = ones
 // column; CIN 1: column = tap, column 27 = ones.  GSCALAR: gz is FP32
 // [V] (rounded to bf16); ASCALAR: a is FP32 [V] scaled by as (rounded).
+//
+// K is the voxels of a 32x4x4 brick; its 16 x-rows of 32 are one MFMA each per
+// tap.  Operands hold eight x-neighbours of one channel per lane, so the
+// brick and its halo are staged in LDS transposed, one x-row of 34 (padded to
+// 40) bf16 per (channel, z, y): pairs of x-neighbours are loaded 16 bytes
+// (eight channels) each and written as eight dwords.  An x-row read once (16
+// bytes and the next four per lane) holds the operands of all three dx:
+// itself, shifted by one bf16, and by two; wavefront w owns the rows y = w,
+// and a halo row serves the up to three output slices z whose window holds
+// it.  The next brick's loads are in flight while a brick is multiplied.
+// The previous form read each operand as eight bf16 (224 LDS reads for 28
+// MFMAs): at 256x256x32 a 16x16 layer took 253 us against 60 now, the last
+// and the first layer 224 and 49 against 50 and 36 (the two input tensors of a
+// 16x16 layer are 134 MB, 26 us at the rate of a copy).
+constexpr int WROW = 40;                       // bf16 per staged halo row (16-byte aligned)
+constexpr int WROWS = WHY * WHZ;               // halo rows of a brick
+constexpr int WPAIRS = WHX / 2;                // pairs of x-neighbours in a halo row
+constexpr int APLANE = WROWS * WROW + 8;       // bf16 per channel: (APLANE * 2 / 16) odd, so that the
+constexpr int GPLANE = WVOX + 8;               // lanes of a 16-byte read fall in distinct banks
+static_assert((APLANE / 8) % 2 == 1 && (GPLANE / 8) % 2 == 1, "bank spread of the staged planes");
+
 template <int CIN, int COUT, bool GSCALAR, bool ASCALAR>
-__global__ __launch_bounds__(256) void wgrad_kernel(int nx, int ny, int nz, const void *__restrict__ gsrc,
-                                                    const void *__restrict__ asrc, float as,
-                                                    float *__restrict__ partial, int nbx, int nby, int nbricks)
+__global__ __launch_bounds__(256, 2) void wgrad_kernel(int nx, int ny, int nz, const void *__restrict__ gsrc,
+                                                       const void *__restrict__ asrc, float as,
+                                                       float *__restrict__ partial, int nbx, int nby, int nbricks)
 {
     constexpr int NB = CIN == 16 ? 28 : 2;
-    __shared__ __attribute__((aligned(16))) unsigned short gT[COUT][WVOX];
-    __shared__ unsigned short aT[CIN][WHV];
+    constexpr int NCOL = NB * 16;
+    // aT holds the staged input, and at the end the workgroup's sums
+    constexpr int ABYTES = CIN * APLANE * 2 > 16 * NCOL * 4 ? CIN * APLANE * 2 : 16 * NCOL * 4;
+    __shared__ __attribute__((aligned(16))) unsigned char abuf[ABYTES];
+    __shared__ __attribute__((aligned(16))) unsigned short gT[COUT * GPLANE];
+    unsigned short *aT = reinterpret_cast<unsigned short *>(abuf);
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
     const int col = lane & 15, g = lane >> 4;
     f32x4 acc[NB];
@@ -417,136 +441,226 @@ __global__ __launch_bounds__(256) void wgrad_kernel(int nx, int ny, int nz, cons
     for (int nb = 0; nb < NB; ++nb)
         acc[nb] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-    for (int brick = blockIdx.x; brick < nbricks; brick += gridDim.x) {
+    // Staging items: a pair of x-neighbours and, of 16 channels, one half.
+    constexpr int AH = CIN == 16 ? 2 : 1, GH = GSCALAR ? 1 : 2;
+    constexpr int AITEMS = AH * WROWS * WPAIRS, GITEMS = GH * WVOX / 2;
+    constexpr int AR = (AITEMS + 255) / 256, GR = (GITEMS + 255) / 256;
+    constexpr int AW = ASCALAR ? 1 : 4, GW = GSCALAR ? 1 : 4;  // dwords of a voxel's item
+    unsigned av[AR][2][AW], gv[GR][2][GW];
+    auto load = [&](int brick) {
         const int bx = brick % nbx, by = (brick / nbx) % nby, bz = brick / (nbx * nby);
         const int x0 = bx * WX, y0 = by * WY, z0 = bz * WZ;
+        // the halo's z-slabs as one buffer resource (at most six slabs: the
+        // launcher checks they span under 4 GiB); voxels outside the volume
+        // read at its end and give zeros
+        const int zlo = max(z0 - 1, 0), zhi = min(z0 + WZ, nz - 1);
+        auto rsrc = [&](const void *src, unsigned bytes) {
+            const unsigned span = (unsigned)((unsigned long long)(zhi - zlo + 1) * nx * ny * bytes);
+            return __builtin_amdgcn_make_buffer_rsrc(
+                (void *)((const char *)src + (size_t)zlo * nx * ny * bytes), (short)0, (int)span, 0x00020000);
+        };
+        auto offset = [&](int gx, int gy, int gz, unsigned bytes, unsigned h) {
+            const bool ok = gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz;
+            const unsigned v = ((unsigned)(gz - zlo) * (unsigned)ny + (unsigned)gy) * (unsigned)nx + (unsigned)gx;
+            return ok ? v * bytes + h * 16u : 0xFFFFFFF0u;
+        };
+        const __amdgpu_buffer_rsrc_t ar = rsrc(asrc, ASCALAR ? 4u : 32u), gr = rsrc(gsrc, GSCALAR ? 4u : 32u);
+#pragma unroll
+        for (int k = 0; k < AR; ++k) {
+            const int q = tid + 256 * k, h = q / (WROWS * WPAIRS), r = q % (WROWS * WPAIRS);
+            const int row = r / WPAIRS, lx = r % WPAIRS * 2;
+            const int gx = x0 + lx - 1, gy = y0 + row % WHY - 1, gz = q < AITEMS ? z0 + row / WHY - 1 : -1;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int off = (int)offset(gx + e, gy, gz, ASCALAR ? 4u : 32u, (unsigned)h);
+                if constexpr (ASCALAR) {
+                    av[k][e][0] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(ar, off, 0, 0);
+                } else {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(ar, off, 0, 0);
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        av[k][e][w] = (unsigned)v[w];
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < GR; ++k) {
+            const int q = tid + 256 * k, h = q / (WVOX / 2), v0 = q % (WVOX / 2) * 2;
+            const int gx = x0 + (v0 & 31), gy = y0 + ((v0 >> 5) & 3), gz = q < GITEMS ? z0 + (v0 >> 7) : -1;
+#pragma unroll
+            for (int e = 0; e < 2; ++e) {
+                const int off = (int)offset(gx + e, gy, gz, GSCALAR ? 4u : 32u, (unsigned)h);
+                if constexpr (GSCALAR) {
+                    gv[k][e][0] = (unsigned)__builtin_amdgcn_raw_buffer_load_b32(gr, off, 0, 0);
+                } else {
+                    const auto v = __builtin_amdgcn_raw_buffer_load_b128(gr, off, 0, 0);
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        gv[k][e][w] = (unsigned)v[w];
+                }
+            }
+        }
+    };
+    // dwords (x, x + 1) of the eight channels of two voxels' halves
+    auto pair_lo = [](unsigned a, unsigned b) { return (a & 0xFFFFu) | (b << 16); };
+    auto pair_hi = [](unsigned a, unsigned b) { return (a >> 16) | (b & 0xFFFF0000u); };
+    auto store = [&]() {
+#pragma unroll
+        for (int k = 0; k < AR; ++k) {
+            const int q = tid + 256 * k, h = q / (WROWS * WPAIRS), r = q % (WROWS * WPAIRS);
+            const int row = r / WPAIRS, lx = r % WPAIRS * 2;
+            if (q < AITEMS) {
+                unsigned *d = reinterpret_cast<unsigned *>(aT + 8 * h * APLANE + row * WROW + lx);
+                if constexpr (ASCALAR) {
+                    *d = f2bf2(as * __uint_as_float(av[k][0][0]), as * __uint_as_float(av[k][1][0]));
+                } else {
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        d[(2 * w) * (APLANE / 2)] = pair_lo(av[k][0][w], av[k][1][w]);
+                        d[(2 * w + 1) * (APLANE / 2)] = pair_hi(av[k][0][w], av[k][1][w]);
+                    }
+                }
+            }
+        }
+#pragma unroll
+        for (int k = 0; k < GR; ++k) {
+            const int q = tid + 256 * k, h = q / (WVOX / 2), v0 = q % (WVOX / 2) * 2;
+            if (q < GITEMS) {
+                unsigned *d = reinterpret_cast<unsigned *>(gT + 8 * h * GPLANE + v0);
+                if constexpr (GSCALAR) {
+                    *d = f2bf2(__uint_as_float(gv[k][0][0]), __uint_as_float(gv[k][1][0]));
+                } else {
+#pragma unroll
+                    for (int w = 0; w < 4; ++w) {
+                        d[(2 * w) * (GPLANE / 2)] = pair_lo(gv[k][0][w], gv[k][1][w]);
+                        d[(2 * w + 1) * (GPLANE / 2)] = pair_hi(gv[k][0][w], gv[k][1][w]);
+                    }
+                }
+            }
+        }
+    };
+    // the ten bf16 of a staged row from this lane's x on
+    struct Row {
+        unsigned w[5];
+    };
+    auto read_row = [&](int ci, int row) {
+        const unsigned short *p = aT + ci * APLANE + row * WROW + 8 * g;
+        const u32x4 v = *reinterpret_cast<const u32x4 *>(p);
+        return Row{{v[0], v[1], v[2], v[3], *reinterpret_cast<const unsigned *>(p + 8)}};
+    };
+
+    const unsigned one = 0x3F803F80u;  // two bf16 1.0
+    int brick = blockIdx.x;
+    if (brick < nbricks)
+        load(brick);
+    for (; brick < nbricks; brick += gridDim.x) {
         __syncthreads();  // the previous brick's operands are consumed
-        if (GSCALAR) {
-            const float *gf = static_cast<const float *>(gsrc);
-            for (int q = tid; q < WVOX; q += 256) {
-                const int gx = x0 + (q & 31), gy = y0 + ((q >> 5) & 3), gz = z0 + (q >> 7);
-                unsigned int v = 0u;
-                if (gx < nx && gy < ny && gz < nz)
-                    v = f2bf(gf[vidx(gx, gy, gz, nx, ny)]);
-                gT[0][q] = (unsigned short)v;
-            }
-        } else {
-            const u32x4 *g16 = static_cast<const u32x4 *>(gsrc);
-            for (int c = tid; c < 2 * WVOX; c += 256) {
-                const int q = c >> 1, h = c & 1;
-                const int gx = x0 + (q & 31), gy = y0 + ((q >> 5) & 3), gz = z0 + (q >> 7);
-                u32x4 v = {0u, 0u, 0u, 0u};
-                if (gx < nx && gy < ny && gz < nz)
-                    v = g16[vidx(gx, gy, gz, nx, ny) * 2 + h];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    gT[8 * h + 2 * j][q] = (unsigned short)(v[j] & 0xFFFFu);
-                    gT[8 * h + 2 * j + 1][q] = (unsigned short)(v[j] >> 16);
-                }
-            }
-        }
-        if (ASCALAR) {
-            const float *af = static_cast<const float *>(asrc);
-            for (int q = tid; q < WHV; q += 256) {
-                const int lx = q % WHX, ly = (q / WHX) % WHY, lz = q / (WHX * WHY);
-                const int gx = x0 + lx - 1, gy = y0 + ly - 1, gz = z0 + lz - 1;
-                unsigned int v = 0u;
-                if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz)
-                    v = f2bf(as * af[vidx(gx, gy, gz, nx, ny)]);
-                aT[0][q] = (unsigned short)v;
-            }
-        } else {
-            const u32x4 *a16 = static_cast<const u32x4 *>(asrc);
-            for (int c = tid; c < 2 * WHV; c += 256) {
-                const int q = c >> 1, h = c & 1;
-                const int lx = q % WHX, ly = (q / WHX) % WHY, lz = q / (WHX * WHY);
-                const int gx = x0 + lx - 1, gy = y0 + ly - 1, gz = z0 + lz - 1;
-                u32x4 v = {0u, 0u, 0u, 0u};
-                if (gx >= 0 && gx < nx && gy >= 0 && gy < ny && gz >= 0 && gz < nz)
-                    v = a16[vidx(gx, gy, gz, nx, ny) * 2 + h];
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-                    aT[8 * h + 2 * j][q] = (unsigned short)(v[j] & 0xFFFFu);
-                    aT[8 * h + 2 * j + 1][q] = (unsigned short)(v[j] >> 16);
-                }
-            }
-        }
+        store();
         __syncthreads();
-        // each wave takes 4 of the 16 k-chunks (rows of 32 voxels)
-        for (int kc = wv; kc < 16; kc += 4) {
-            const int ky = kc & 3, kz = kc >> 2;
-            u32x4 Aop = {0u, 0u, 0u, 0u};
+        if (brick + (int)gridDim.x < nbricks)
+            load(brick + (int)gridDim.x);
+        // this wavefront's four x-rows of the gradient: y = wv, z = 0..3
+        u32x4 A[WZ];
+#pragma unroll
+        for (int z = 0; z < WZ; ++z) {
+            A[z] = u32x4{0u, 0u, 0u, 0u};
             if (col < COUT)
-                Aop = *reinterpret_cast<const u32x4 *>(&gT[col][kc * 32 + 8 * g]);
+                A[z] = *reinterpret_cast<const u32x4 *>(&gT[col * GPLANE + (z * WY + wv) * 32 + 8 * g]);
+        }
+        if constexpr (CIN == 16) {
+#pragma unroll
+            for (int zr = 0; zr < WHZ; ++zr)
+#pragma unroll
+                for (int dy = 0; dy < 3; ++dy) {
+                    const Row r = read_row(col, zr * WHY + wv + dy);
+                    const u32x4 b0 = {r.w[0], r.w[1], r.w[2], r.w[3]}, b2 = {r.w[1], r.w[2], r.w[3], r.w[4]};
+                    u32x4 b1;
+#pragma unroll
+                    for (int w = 0; w < 4; ++w)
+                        b1[w] = __builtin_amdgcn_alignbit(r.w[w + 1], r.w[w], 16);
+#pragma unroll
+                    for (int z = 0; z < WZ; ++z) {
+                        const int dz = zr - z;
+                        if (dz >= 0 && dz <= 2) {
+                            f32x4 *a = acc + 9 * dz + 3 * dy;
+                            a[0] = mfma(A[z], b0, a[0]);
+                            a[1] = mfma(A[z], b1, a[1]);
+                            a[2] = mfma(A[z], b2, a[2]);
+                        }
+                    }
+                }
+            const unsigned o = col == 0 ? one : 0u;
+#pragma unroll
+            for (int z = 0; z < WZ; ++z)
+                acc[27] = mfma(A[z], u32x4{o, o, o, o}, acc[27]);
+        } else {
+            // column t: its own row and shift
 #pragma unroll
             for (int nb = 0; nb < NB; ++nb) {
-                const int t = CIN == 16 ? nb : 16 * nb + col;
-                const int ci = CIN == 16 ? col : 0;
-                unsigned int e[8];
-                if (t < 27) {
-                    const int base = ((kz + tap_dz(t) + 1) * WHY + (ky + tap_dy(t) + 1)) * WHX + 8 * g + tap_dx(t) + 1;
+                const int t = 16 * nb + col, tt = t < 27 ? t : 0, s = tt % 3;
+                const int row0 = tt / 9 * WHY + tt / 3 % 3 + wv;
+                const unsigned fill = t == 27 ? one : 0u;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        e[j] = aT[ci][base + j];
-                } else {
-                    const unsigned int one = (t == 27 && (CIN == 1 || col == 0)) ? 0x3F80u : 0u;
+                for (int z = 0; z < WZ; ++z) {
+                    const Row r = read_row(0, row0 + z * WHY);
+                    u32x4 b;
 #pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        e[j] = one;
+                    for (int w = 0; w < 4; ++w) {
+                        const unsigned e = s == 0 ? r.w[w]
+                                                  : (s == 1 ? __builtin_amdgcn_alignbit(r.w[w + 1], r.w[w], 16)
+                                                            : r.w[w + 1]);
+                        b[w] = t < 27 ? e : fill;
+                    }
+                    acc[nb] = mfma(A[z], b, acc[nb]);
                 }
-                acc[nb] = mfma(Aop, pack8(e), acc[nb]);
             }
         }
     }
-    // the four waves hold partial sums over different k-chunks: add them in
+    // the four waves hold partial sums over different x-rows: add them in
     // wave order through LDS, then write this workgroup's partial
     __syncthreads();
-    float *stage = reinterpret_cast<float *>(&aT[0][0]);  // reused: needs 16*NB*16 floats
-    constexpr int NCOL = NB * 16;
-    static_assert(sizeof(aT) >= 16 * NCOL * 4 || CIN == 1, "staging space");
+    float *stage = reinterpret_cast<float *>(abuf);
     float *out = partial + (size_t)blockIdx.x * 16 * NCOL;
-    if (CIN == 16) {
-        for (int w = 0; w < 4; ++w) {
-            if (wv == w) {
+    for (int w = 0; w < 4; ++w) {
+        if (wv == w) {
 #pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
+            for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float &dst = stage[(4 * g + i) * NCOL + nb * 16 + col];
-                        dst = (w == 0 ? 0.f : dst) + acc[nb][i];
-                    }
-            }
-            __syncthreads();
+                for (int i = 0; i < 4; ++i) {
+                    float &dst = stage[(4 * g + i) * NCOL + nb * 16 + col];
+                    dst = (w == 0 ? 0.f : dst) + acc[nb][i];
+                }
         }
-        for (int k = tid; k < 16 * NCOL; k += 256)
-            out[k] = stage[k];
-    } else {
-        __shared__ float st1[16 * 32];
-        for (int w = 0; w < 4; ++w) {
-            if (wv == w) {
-#pragma unroll
-                for (int nb = 0; nb < NB; ++nb)
-#pragma unroll
-                    for (int i = 0; i < 4; ++i) {
-                        float &dst = st1[(4 * g + i) * NCOL + nb * 16 + col];
-                        dst = (w == 0 ? 0.f : dst) + acc[nb][i];
-                    }
-            }
-            __syncthreads();
-        }
-        for (int k = tid; k < 16 * NCOL; k += 256)
-            out[k] = st1[k];
+        __syncthreads();
     }
+    for (int k = tid; k < 16 * NCOL; k += 256)
+        out[k] = stage[k];
 }
 
 // Sums the workgroup partials (fixed order, FP64) and scatters them into the
-// gradient blob: W[o][i][t] at wofs, b[o] at wofs + cout*cin*27.
-__global__ void wgrad_reduce_kernel(const float *__restrict__ partial, int nblk, int cin, int cout, int ncol,
-                                    float *__restrict__ grad)
+// gradient blob: W[o][i][t] at wofs, b[o] at wofs + cout*cin*27.  A workgroup
+// of 16 wavefronts takes 64 entries; wavefront w sums the w-th sixteenth of
+// the partials, then wavefront 0 the sixteen sums.  (One thread per entry
+// summing all 512 took 127 us a layer, its loads in series on 28 workgroups.)
+__global__ __launch_bounds__(1024) void wgrad_reduce_kernel(const float *__restrict__ partial, int nblk, int cin,
+                                                            int cout, int ncol, float *__restrict__ grad)
 {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= 16 * ncol)
+    __shared__ double sums[16][64];
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int k = blockIdx.x * 64 + lane;  // 16 * ncol is a multiple of 64
+    const int per = (nblk + 15) / 16, b0 = wv * per, b1 = min(b0 + per, nblk);
+    double s = 0.0;
+#pragma unroll 8
+    for (int b = b0; b < b1; ++b)
+        s += (double)partial[(size_t)b * 16 * ncol + k];
+    sums[wv][lane] = s;
+    __syncthreads();
+    if (wv != 0)
         return;
+    s = 0.0;
+#pragma unroll
+    for (int w = 0; w < 16; ++w)
+        s += sums[w][lane];
     const int o = k / ncol, c = k % ncol;
     if (o >= cout)
         return;
@@ -567,9 +681,6 @@ __global__ void wgrad_reduce_kernel(const float *__restrict__ partial, int nblk,
         else
             return;
     }
-    double s = 0.0;
-    for (int b = 0; b < nblk; ++b)
-        s += (double)partial[(size_t)b * 16 * ncol + k];
     grad[dst] = (float)s;
 }
 
@@ -706,7 +817,7 @@ hipError_t launch_wgrad(const Layout &L, int nx, int ny, int nz, const void *gsr
     wgrad_kernel<CIN, COUT, GS, AS><<<L.wgrid, 256, 0, s>>>(nx, ny, nz, gsrc, asrc, as, partial, L.nbx, L.nby,
                                                            L.nbricks);
     const int ncol = (CIN == 16 ? 28 : 2) * 16;
-    wgrad_reduce_kernel<<<(16 * ncol + 255) / 256, 256, 0, s>>>(partial, L.wgrid, CIN, COUT, ncol, grad);
+    wgrad_reduce_kernel<<<16 * ncol / 64, 1024, 0, s>>>(partial, L.wgrid, CIN, COUT, ncol, grad);
     return hipGetLastError();
 }
 
@@ -761,7 +872,7 @@ kv_status kv_cnn_forward(kv_context *ctx, const float *d_params, float scale, co
     auto W = [&](int v) { return wpk + v * WV_OPS * 64; };
     auto c16 = [](const unsigned short *q) { return reinterpret_cast<const u32x4 *>(q); };
     const float *p = d_params;
-    pack_weights_kernel<<<WV_COUNT, 64, 0, s>>>(p, wpk, P_W1, P_W2, P_W3, P_W4);
+    pack_weights_kernel<<<dim3(WV_COUNT, WV_OPS), 64, 0, s>>>(p, wpk, P_W1, P_W2, P_W3, P_W4);
     conv1_kernel<EP_RELU><<<grid, 256, 0, s>>>(nx, ny, nz, d_x, scale, W(WV_L1), p + P_B1, a1, nullptr);
     conv16_kernel<EP_RELU><<<grid, 256, 0, s>>>(nx, ny, nz, c16(a1), W(WV_L2), p + P_B2, a2, nullptr, nullptr,
                                                 nullptr, nullptr, 0.f, 0.f, nullptr);
@@ -799,7 +910,7 @@ kv_status kv_cnn_gradient(kv_context *ctx, const float *d_params, float scale, c
     u32x4 *wpk = at<u32x4>(d_work, L.wpk);
     auto W = [&](int v) { return wpk + v * WV_OPS * 64; };
 
-    pack_weights_kernel<<<WV_COUNT, 64, 0, s>>>(p, wpk, P_W1, P_W2, P_W3, P_W4);
+    pack_weights_kernel<<<dim3(WV_COUNT, WV_OPS), 64, 0, s>>>(p, wpk, P_W1, P_W2, P_W3, P_W4);
     conv1_kernel<EP_RELU><<<grid, 256, 0, s>>>(nx, ny, nz, d_x, scale, W(WV_L1), p + P_B1, a1, nullptr);
     conv16_kernel<EP_RELU><<<grid, 256, 0, s>>>(nx, ny, nz, c16(a1), W(WV_L2), p + P_B2, a2, nullptr, nullptr,
                                                 nullptr, nullptr, 0.f, 0.f, nullptr);
