@@ -149,7 +149,7 @@ kv_status kv_shift_and_add(kv_context *ctx, const float *d_proj, const float *sr
  * The source y positions, plane heights and the row-shift table are staged in
  * a fixed array that the library holds on each GPU until the process ends
  * ((KV_SAA_NOALLOC_MAX_VIEWS + KV_SAA_NOALLOC_MAX_PLANES +
- * KV_SAA_NOALLOC_MAX_SHIFTS) * 4 bytes = 276 KiB); a call with more than
+ * KV_SAA_NOALLOC_MAX_SHIFTS + 8) * 4 bytes: 276 KiB); a call with more than
  * KV_SAA_NOALLOC_MAX_VIEWS views, KV_SAA_NOALLOC_MAX_PLANES planes or
  * KV_SAA_NOALLOC_MAX_SHIFTS plane-view pairs returns KV_ERR_INVALID.  The
  * array is shared by every call on a GPU and keeps the last call's contents:

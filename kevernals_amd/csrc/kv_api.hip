@@ -850,7 +850,7 @@ kv_status saa_check(kv_context *ctx, const float *d_proj, const float *src_y, in
                 return KV_ERR_INVALID;
             }
             if (shifts)
-                shifts[(size_t)k * g.np + p] = (int32_t)t;
+                shifts[(size_t)p * nplanes + k] = (int32_t)t;
         }
     }
     return KV_OK;
@@ -863,17 +863,17 @@ kv_status kv_shift_and_add(kv_context *ctx, const float *d_proj, const float *sr
     if (kv_status st = check_ctx(ctx, true))
         return st;
     const KvGeom &g = ctx->g;
-    std::vector<int32_t> shifts((size_t)std::max(nplanes, 0) * g.np);
+    std::vector<int32_t> shifts((size_t)std::max(nplanes, 0) * g.np + KV_SAA_PAD, 0);
     if (kv_status st = saa_check(ctx, d_proj, src_y, nplanes, plane_z, sid, fulcrum_z, voxel_dy, d_out,
                                  shifts.data()))
         return st;
-    const int kc = kv_saa_chunk(nplanes, g.np, [&](int k, int p) { return shifts[(size_t)k * g.np + p]; });
+    const KvSaaPlan plan = kv_saa_plan(nplanes, g.np, [&](int k, int p) { return shifts[(size_t)p * nplanes + k]; });
     int32_t *d_shifts = nullptr;
     if (kv_status st = dev_alloc((void **)&d_shifts, shifts.size() * 4))
         return st;
     hipError_t e = hipMemcpyAsync(d_shifts, shifts.data(), shifts.size() * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess)
-        e = kv_launch_saa(g.nu, g.nv, g.np, d_proj, d_shifts, nplanes, kc, d_out, ctx->stream);
+        e = kv_launch_saa(g.nu, g.nv, g.np, d_proj, d_shifts, nplanes, plan, d_out, ctx->stream);
     if (e == hipSuccess)
         e = hipStreamSynchronize(ctx->stream);
     (void)hipFree(d_shifts);
@@ -908,7 +908,7 @@ kv_status kv_shift_and_add_noalloc(kv_context *ctx, const float *d_proj, const f
     const float mF = sid / (sid - fulcrum_z);
     // the shifts the device evaluates, recomputed here (same expressions) to
     // pick the kernel's plane chunk
-    const int kc = kv_saa_chunk(nplanes, g.np, [&](int k, int p) {
+    const KvSaaPlan plan = kv_saa_plan(nplanes, g.np, [&](int k, int p) {
         const float mZ = sid / (sid - plane_z[k]);
         const float coeff = mZ - mF;
         const float world = src_y[p] * coeff;
@@ -920,7 +920,7 @@ kv_status kv_shift_and_add_noalloc(kv_context *ctx, const float *d_proj, const f
     if (e == hipSuccess)
         e = kv_launch_saa_shifts(g.np, nplanes, sid, mF, voxel_dy, d_sy, d_pz, d_shifts, ctx->stream);
     if (e == hipSuccess)
-        e = kv_launch_saa(g.nu, g.nv, g.np, d_proj, d_shifts, nplanes, kc, d_out, ctx->stream);
+        e = kv_launch_saa(g.nu, g.nv, g.np, d_proj, d_shifts, nplanes, plan, d_out, ctx->stream);
     // the caller's host arrays are read by the copies: return when they are done
     if (e == hipSuccess)
         e = hipStreamSynchronize(ctx->stream);

@@ -355,17 +355,24 @@ int kv_bp_batch_blocks_per_cu(int mode);
 // (kv_misc.hip): _init resolves it once per device, with that device current;
 // kv_internal_scratch returns it (nullptr before _init).  Word layout:
 // [src_y: KV_SAA_NOALLOC_MAX_VIEWS][plane_z: KV_SAA_NOALLOC_MAX_PLANES]
-// [shifts: KV_SAA_NOALLOC_MAX_SHIFTS].
+// [shifts: KV_SAA_NOALLOC_MAX_SHIFTS + KV_SAA_PAD].
 hipError_t kv_internal_scratch_init(int device);
 int32_t *kv_internal_scratch(int device);
 hipError_t kv_launch_saa_shifts(int np, int nplanes, float sid, float mF, float voxel_dy, const float *src_y,
                                 const float *plane_z, int32_t *shifts, hipStream_t s);
+// The shift table of a shift-and-add: the planes' row shifts view by view
+// (shift of plane k, view p at [p * nplanes + k]), and KV_SAA_PAD more words
+// that may be read.
+constexpr int KV_SAA_PAD = 8;
 // Planes per chunk of the shift-and-add kernel for these shifts (shift(k, p)
-// = row shift of plane k, view p): the largest of 8, 4, 2 whose staged rows
-// fit the kernel's LDS, else 1.
-int kv_saa_chunk(int nplanes, int np, const std::function<int(int, int)> &shift);
-hipError_t kv_launch_saa(int nu, int nv, int np, const float *proj, const int32_t *shifts, int nplanes, int kc,
-                         float *out, hipStream_t s);
+// = row shift of plane k, view p), the largest of 8, 4, 2 whose staged rows
+// fit the kernel's LDS, else 1; and the staged rows, 32 or 64.
+struct KvSaaPlan {
+    int kc, rows;
+};
+KvSaaPlan kv_saa_plan(int nplanes, int np, const std::function<int(int, int)> &shift);
+hipError_t kv_launch_saa(int nu, int nv, int np, const float *proj, const int32_t *shifts, int nplanes,
+                         const KvSaaPlan &plan, float *out, hipStream_t s);
 hipError_t kv_launch_sum(int64_t n, const float *x, double *partials, int nblocks, hipStream_t s);
 hipError_t kv_launch_loglik(const KvGeom &g, const float *data, const float *ax, double *partials, int nblocks,
                             hipStream_t s);

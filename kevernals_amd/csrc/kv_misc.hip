@@ -2,6 +2,7 @@
 #pragma clang fp contract(off)
 
 #include <algorithm>
+#include <climits>
 #include <functional>
 #include <mutex>
 
@@ -14,81 +15,119 @@ namespace {
 // detector (vtkImageConstantPad), summed in view order in FP64 and stored as
 // FP32.
 //
-// A workgroup owns a strip of SAA_TU detector columns by SAA_RV rows and
-// walks the planes in chunks of kc (<= SAA_KC).  For each chunk it visits the
-// views in order; the rows of view p that the chunk's planes read,
-// [v0 + min_k t, v0 + SAA_RV - 1 + max_k t], are staged once in LDS as their
-// FP64 products x * (1/P) (0 outside the detector), and every (plane, row)
-// of the chunk adds its staged product: each projection row is read from
-// memory once per chunk instead of once per plane, and the product is formed
-// once per staged element.  The sums keep the view order and the
-// per-element arithmetic of the one-lane-per-pixel form, so the result is
-// bit-identical.  The host picks kc so that SAA_RV plus the chunk's largest
-// shift spread fits the SAA_SR staged rows (kc = 1 always fits).
-constexpr int SAA_TU = 64, SAA_RV = 16, SAA_KC = 8, SAA_SR = 64;
+// A workgroup owns SAA_TU detector columns by SAA_RV rows of KC planes
+// (blockIdx.z counts such chunks) and visits the views in order.  The
+// rows of view p that its planes read, [v0 + min_k t, v0 + SAA_RV - 1 + max_k
+// t], are staged in LDS as they are, two views deep: the next view's rows are
+// loaded while this one's are added, one barrier per view.  A thread adds
+// SAA_RPT rows of one column for every plane, forming the FP64 product x * (1/P)
+// as it reads.  The sums keep the view order and the per-element arithmetic of
+// the one-lane-per-pixel form, so the result is bit-identical.  The host picks
+// KC (8, 4, 2 or 1) so that SAA_RV plus the chunk's largest shift spread fits
+// 64 staged rows, or 32 where it can (KC = 1 always fits).
+//
+// Bound by the vector unit's FP64 work (convert, multiply and add per plane
+// and pixel) and the barriers.  Full size (64 planes, 25 views of 2048^2): 2.55
+// ms with the products staged in FP64 (twice the LDS reads), two barriers per
+// view and the loads between them; 1.25 now.  Also measured: two views deep
+// with FP64 products 1.31 ms (LDS-bound); 16 planes a chunk (168 registers, 8
+// wavefronts per CU) 3.07 ms; keeping the rows in registers from plane to
+// plane where the shift allows 1.57-1.98 ms (branches per plane).
+constexpr int SAA_TU = 64, SAA_RV = 16, SAA_KC = 8;
 constexpr int SAA_RPT = SAA_RV / 4;  // output rows per thread (4 wavefronts)
 
+template <int KC, int SR>
 __global__ __launch_bounds__(256) void saa_kernel(int nu, int nv, int np, const float *__restrict__ proj,
-                                                  const int32_t *__restrict__ shifts, int nplanes, int kc,
+                                                  const int32_t *__restrict__ shifts, int stride, int nplanes,
                                                   float *__restrict__ out)
 {
-    __shared__ double st[SAA_SR][SAA_TU];
-    const int lane = threadIdx.x & 63, grp = threadIdx.x >> 6;
+    static_assert(KC <= KV_SAA_PAD, "words read past the shift table");
+    __shared__ float st[2][SR][SAA_TU];
+    const int lane = threadIdx.x & 63, grp = __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
     const int u = blockIdx.x * SAA_TU + lane;
     const int v0 = blockIdx.y * SAA_RV;
+    const int k0 = blockIdx.z * KC, nk = min(KC, nplanes - k0);
     const double wgt = 1.0 / (double)np;
     const size_t plane = (size_t)nu * nv;
-    for (int k0 = 0; k0 < nplanes; k0 += kc) {
-        const int nk = min(kc, nplanes - k0);
-        double acc[SAA_KC][SAA_RPT];
+    double acc[KC][SAA_RPT];
 #pragma unroll
-        for (int j = 0; j < SAA_KC; ++j)
+    for (int j = 0; j < KC; ++j)
+#pragma unroll
+        for (int i = 0; i < SAA_RPT; ++i)
+            acc[j][i] = 0.0;
+    // the chunk's shifts for view p, the smallest of them and the view's rows
+    // (at most SR by the host's choice; the clamps keep every LDS
+    // access inside the array whatever the shifts)
+    auto range = [&](int p, int (&t)[KC], int &tlo, int &nrows) {
+        // one scalar load; the words past the chunk's planes are other
+        // planes' (KV_SAA_PAD words past the table's end may be read)
+        const int32_t *row = shifts + (size_t)p * stride + k0;
+        int lo = row[0], hi = row[0];
+#pragma unroll
+        for (int j = 0; j < KC; ++j)
+            t[j] = row[j];
+#pragma unroll
+        for (int j = 1; j < KC; ++j) {
+            t[j] = j < nk ? t[j] : t[0];
+            lo = min(lo, t[j]);
+            hi = max(hi, t[j]);
+        }
+        tlo = lo;
+        nrows = min(SAA_RV + hi - lo, SR);
+    };
+    // rows grp, grp + 4, ... of the staged rows; 0 outside the detector
+    float f[SR / 4];
+    auto load = [&](int p, int tlo, int nrows) {
+        const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+            (void *)(proj + (size_t)p * plane), (short)0, (int)(unsigned)(plane * 4), 0x00020000);
+#pragma unroll
+        for (int i = 0; i < SR / 4; ++i) {
+            const int r = grp + 4 * i, vv = v0 + tlo + r;
+            const bool ok = r < nrows && vv >= 0 && vv < nv && u < nu;
+            const unsigned off = ok ? ((unsigned)vv * (unsigned)nu + (unsigned)u) * 4u : 0xFFFFFFF0u;
+            f[i] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, (int)off, 0, 0));
+        }
+    };
+    auto store = [&](int buf) {
+#pragma unroll
+        for (int i = 0; i < SR / 4; ++i)
+            st[buf][grp + 4 * i][lane] = f[i];
+    };
+    int t[KC], tlo, nrows;
+    range(0, t, tlo, nrows);
+    load(0, tlo, nrows);
+    store(0);
+    __syncthreads();
+    for (int p = 0; p < np; ++p) {
+        int nt[KC], nlo = 0, nn = 0;
+        const int q = min(p + 1, np - 1);
+        range(q, nt, nlo, nn);
+        load(q, nlo, nn);
+        const float(*s)[SAA_TU] = st[p & 1];
+#pragma unroll
+        for (int j = 0; j < KC; ++j) {
+            // planes past the chunk's last repeat it, unused
+            const int r0 = min(grp * SAA_RPT + t[j] - tlo, SR - SAA_RPT);
 #pragma unroll
             for (int i = 0; i < SAA_RPT; ++i)
-                acc[j][i] = 0.0;
-        for (int p = 0; p < np; ++p) {
-            // the chunk's shifts for view p (wave-uniform)
-            int t[SAA_KC];
-            int tlo = shifts[k0 * np + p], thi = tlo;
-#pragma unroll
-            for (int j = 0; j < SAA_KC; ++j) {
-                t[j] = j < nk ? shifts[(k0 + j) * np + p] : t[0];
-                tlo = min(tlo, t[j]);
-                thi = max(thi, t[j]);
-            }
-            // <= SAA_SR by the host's choice of kc; the clamps below keep
-            // every LDS access inside the array whatever the shifts
-            const int nrows = min(SAA_RV + thi - tlo, SAA_SR);
-            __syncthreads();  // the previous view's readers are done
-            const float *src = proj + (size_t)p * plane;
-            for (int r = grp; r < nrows; r += 4) {
-                const int vv = v0 + tlo + r;
-                double x = 0.0;
-                if (vv >= 0 && vv < nv && u < nu)
-                    x = (double)src[(size_t)vv * nu + u] * wgt;
-                st[r][lane] = x;
-            }
-            __syncthreads();
-#pragma unroll
-            for (int j = 0; j < SAA_KC; ++j) {
-                if (j < nk) {
-                    const int r0 = min(grp * SAA_RPT + t[j] - tlo, SAA_SR - SAA_RPT);
-#pragma unroll
-                    for (int i = 0; i < SAA_RPT; ++i)
-                        acc[j][i] += st[r0 + i][lane];
-                }
-            }
+                acc[j][i] += (double)s[r0 + i][lane] * wgt;
         }
-        if (u < nu) {
+        store((p + 1) & 1);
+        tlo = nlo;
 #pragma unroll
-            for (int j = 0; j < SAA_KC; ++j) {
-                if (j < nk) {
+        for (int j = 0; j < KC; ++j)
+            t[j] = nt[j];
+        __syncthreads();
+    }
+    if (u < nu) {
 #pragma unroll
-                    for (int i = 0; i < SAA_RPT; ++i) {
-                        const int v = v0 + grp * SAA_RPT + i;
-                        if (v < nv)
-                            out[(size_t)(k0 + j) * plane + (size_t)v * nu + u] = (float)acc[j][i];
-                    }
+        for (int j = 0; j < KC; ++j) {
+            if (j < nk) {
+#pragma unroll
+                for (int i = 0; i < SAA_RPT; ++i) {
+                    const int v = v0 + grp * SAA_RPT + i;
+                    if (v < nv)
+                        out[(size_t)(k0 + j) * plane + (size_t)v * nu + u] = (float)acc[j][i];
                 }
             }
         }
@@ -262,7 +301,7 @@ __global__ __launch_bounds__(256) void saa_shift_kernel(int np, int nplanes, flo
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= np * nplanes)
         return;
-    const int k = i / np, p = i - k * np;
+    const int p = i / nplanes, k = i - p * nplanes;
     const float mZ = sid / (sid - plane_z[k]);
     const float coeff = mZ - mF;
     const float world = src_y[p] * coeff;
@@ -276,7 +315,7 @@ __global__ __launch_bounds__(256) void saa_shift_kernel(int np, int nplanes, flo
 // own copy until the process ends).  Host code reaches it only through the
 // per-device address that hipGetSymbolAddress returns.
 static __device__ __align__(256) int32_t scratch[KV_SAA_NOALLOC_MAX_VIEWS + KV_SAA_NOALLOC_MAX_PLANES +
-                                                 KV_SAA_NOALLOC_MAX_SHIFTS];
+                                                 KV_SAA_NOALLOC_MAX_SHIFTS + KV_SAA_PAD];
 
 namespace {
 constexpr int KV_MAX_DEVICES = 64;
@@ -352,10 +391,10 @@ hipError_t kv_launch_sum(int64_t n, const float *x, double *partials, int nblock
     return hipGetLastError();
 }
 
-int kv_saa_chunk(int nplanes, int np, const std::function<int(int, int)> &shift)
+KvSaaPlan kv_saa_plan(int nplanes, int np, const std::function<int(int, int)> &shift)
 {
     for (int kc = SAA_KC; kc > 1; kc /= 2) {
-        int spread = 0;
+        int64_t spread = 0;
         for (int k0 = 0; k0 < nplanes; k0 += kc)
             for (int p = 0; p < np; ++p) {
                 int lo = shift(k0, p), hi = lo;
@@ -364,22 +403,36 @@ int kv_saa_chunk(int nplanes, int np, const std::function<int(int, int)> &shift)
                     lo = std::min(lo, t);
                     hi = std::max(hi, t);
                 }
-                spread = std::max(spread, hi - lo);
+                spread = std::max(spread, (int64_t)hi - lo);
             }
-        if (SAA_RV + spread <= SAA_SR)
-            return kc;
+        if (SAA_RV + spread <= 64)
+            return KvSaaPlan{kc, SAA_RV + spread <= 32 ? 32 : 64};
     }
-    return 1;
+    return KvSaaPlan{1, 32};
 }
 
-hipError_t kv_launch_saa(int nu, int nv, int np, const float *proj, const int32_t *shifts, int nplanes, int kc,
-                         float *out, hipStream_t s)
+hipError_t kv_launch_saa(int nu, int nv, int np, const float *proj, const int32_t *shifts, int nplanes,
+                         const KvSaaPlan &plan, float *out, hipStream_t s)
 {
-    if (kc < 1 || kc > SAA_KC)
-        return hipErrorInvalidValue;
-    const dim3 grid((nu + SAA_TU - 1) / SAA_TU, (nv + SAA_RV - 1) / SAA_RV), block(256);
-    saa_kernel<<<grid, block, 0, s>>>(nu, nv, np, proj, shifts, nplanes, kc, out);
-    return hipGetLastError();
+    const int kc = plan.kc;
+    // (65535 chunks per launch at most)
+    for (int k0 = 0; k0 < nplanes; k0 += 65535 * kc) {
+        const int n = std::min(nplanes - k0, 65535 * kc);
+        const dim3 grid((nu + SAA_TU - 1) / SAA_TU, (nv + SAA_RV - 1) / SAA_RV, (n + kc - 1) / kc);
+        float *o = out + (size_t)k0 * nu * nv;
+        auto launch = [&](auto kernel) { kernel<<<grid, 256, 0, s>>>(nu, nv, np, proj, shifts + k0, nplanes, n, o); };
+        const bool wide = plan.rows > 32;
+        switch (kc) {
+        case 8: wide ? launch(saa_kernel<8, 64>) : launch(saa_kernel<8, 32>); break;
+        case 4: wide ? launch(saa_kernel<4, 64>) : launch(saa_kernel<4, 32>); break;
+        case 2: wide ? launch(saa_kernel<2, 64>) : launch(saa_kernel<2, 32>); break;
+        case 1: launch(saa_kernel<1, 32>); break;
+        default: return hipErrorInvalidValue;
+        }
+        if (const hipError_t e = hipGetLastError())
+            return e;
+    }
+    return hipSuccess;
 }
 
 hipError_t kv_launch_loglik(const KvGeom &g, const float *data, const float *ax, double *partials, int nblocks,
