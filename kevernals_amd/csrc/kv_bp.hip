@@ -386,7 +386,10 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                 mn = fminf(mn, fminf(c * ta, c * tb));
             }
             const float u = clampf((sfx + mn - ofx) * scx - 0.5f, -1e6f, 1e6f);
-            xbase[tid] = (int)floorf(u) - 2;
+            // (no column left of the detector: plane 0's entries would lie
+            // before the table, and a load that starts there returns 0 for
+            // all of its words)
+            xbase[tid] = max((int)floorf(u) - 2, 0);
         }
         __syncthreads();
         // Table bands through a bounds-checked buffer resource over this
