@@ -290,7 +290,7 @@ kv_status ensure_tables(kv_context *ctx, int mode)
 {
     const KvGeom &g = ctx->g;
     const size_t nxe = (size_t)g.np * g.nu * (g.nx + 1), nye = (size_t)g.np * g.nv * (g.ny + 1),
-                 nze = (size_t)g.np * (g.nz + 1), nyz = (size_t)g.np * g.nz * g.ny * KV_YZ;
+                 nze = (size_t)g.np * (g.nz + 1), nyz = ((size_t)g.np * g.nz * g.ny + 1) * KV_YZ;
     if (mode == KV_MODE_R) {
         if (ctx->tab_r_ok)
             return KV_OK;

@@ -189,12 +189,9 @@ __device__ __forceinline__ float clampf(float v, float lo, float hi) { return __
 
 // min/max as signed-integer min/max of the IEEE bit patterns.  They order two
 // floats exactly as fminf/fmaxf when both are >= +0, and put every negative
-// value (including -0) below every non-negative one.  The fast path uses them
-// only in w = min(H, Hy) - max(L, Ly) with L >= +0 (L carries the clip at
-// alpha = 0 as +0): w > 0 needs all of H, Hy and min(H, Hy) positive, where
-// the results are the FP32 ones bit for bit; when any of them is negative both
-// forms give w < 0.  No NaN reaches these operands (entries are finite or
-// +-INF).
+// value (including -0) below every non-negative one, whose own order does not
+// matter to a bound clipped at +0.  On wavefront-uniform operands they are
+// scalar instructions.  No NaN reaches them (entries are finite or +-INF).
 __device__ __forceinline__ float bmin(float a, float b) { return __int_as_float(min(__float_as_int(a), __float_as_int(b))); }
 __device__ __forceinline__ float bmax(float a, float b) { return __int_as_float(max(__float_as_int(a), __float_as_int(b))); }
 
@@ -219,6 +216,16 @@ __device__ __forceinline__ void shadow_affine(float c, float k1a, float k0a, flo
     hi = min((int)floorf(b), n - 1);
 }
 
+// Alpha interval of a detector row's rays inside a voxel row: between its two
+// y-plane crossings and the z interval [lz, uz], lz >= +0, uz <= 1; both ends
+// equal and in [0, 1] where it is empty (crossings may be infinite).  A
+// negative upper end, however ordered, is below lo.
+__device__ __forceinline__ void row_interval(float a, float b, float lz, float uz, float &lo, float &hi)
+{
+    lo = bmin(1.f, bmax(lz, bmin(a, b)));
+    hi = bmax(lo, bmin(uz, bmax(a, b)));
+}
+
 // Per view, y row and z slice: the terms of the backprojector that the
 // voxels of one (y, z) row share (KvTables::yz), with the expressions the
 // backprojector evaluated per row before they were tabulated, so every value
@@ -226,7 +233,8 @@ __device__ __forceinline__ void shadow_affine(float c, float k1a, float k0a, flo
 // slice's planes (shadow_affine on the zs table), in mode R intersected with
 // the +-5 window around the row of the voxel centre's projection and empty
 // when that centre lies off the detector widened by 5 pixels
-// (Projector.cu:473-492, 607-646), and the z-plane alpha interval.
+// (Projector.cu:473-492, 607-646), the z-plane alpha interval and the first
+// rows' alpha intervals.
 template <int MODE>
 __global__ void yz_kernel(KvGeom g, KvTables t)
 {
@@ -266,15 +274,29 @@ __global__ void yz_kernel(KvGeom g, KvTables t)
             }
         }
         const float a1z = t.z[p * nz1 + z], a2z = t.z[p * nz1 + z + 1];
-        float *o = t.yz + i * KV_YZ;
+        const float lz = bmax(0.f, fminf(a1z, a2z)), uz = fminf(1.f, fmaxf(a1z, a2z));
+        float o[KV_YZ];
         o[0] = __int_as_float(f0);
         o[1] = __int_as_float(f1);
         o[2] = __int_as_float(hs ? 1 : 0);
-        o[3] = 0.f;
-        o[4] = fmaxf(0.f, fminf(a1z, a2z));
-        o[5] = fminf(1.f, fmaxf(a1z, a2z));
-        o[6] = bmax(0.f, fminf(a1z, a2z));  // lz with a +0 floor in bit order
-        o[7] = 0.f;
+        o[3] = Z[KV_ZS + 3] + (1.f - 0.02f);
+        o[4] = Z[KV_ZS + 2];
+        o[5] = Z[KV_ZS + 3];
+        o[6] = lz;
+        o[7] = uz;
+        const float *ty0 = t.y + ((size_t)p * (g.ny + 1) + y) * g.nv, *ty1 = ty0 + g.nv;
+#pragma unroll
+        for (int r = 0; r < KV_YZ_ROWS; ++r) {
+            float lo = 0.f, hi = 0.f;
+            if (f0 + r <= f1)
+                row_interval(ty0[f0 + r], ty1[f0 + r], lz, uz, lo, hi);
+            o[8 + 2 * r] = lo;
+            o[9 + 2 * r] = hi;
+        }
+        float4 *d = reinterpret_cast<float4 *>(t.yz + i * KV_YZ);
+#pragma unroll
+        for (int k = 0; k < KV_YZ / 4; ++k)
+            d[k] = make_float4(o[4 * k], o[4 * k + 1], o[4 * k + 2], o[4 * k + 3]);
     }
 }
 
@@ -283,7 +305,7 @@ template <int ZT>
 struct BpShared {
     float xb[(TX + 1) * XBS];
     int xbase[TX + 1];
-    float accs[ZT][2][256];  // (value, weight) per slice of the brick
+    float accs[ZT][2][256];  // (value, weight) per slice of the brick (mode A: value only)
 };
 
 // Read-only device memory seen through the constant address space: loads at
@@ -292,6 +314,9 @@ struct BpShared {
 typedef const __attribute__((address_space(4))) float KvConstF;
 __device__ __forceinline__ KvConstF *kv_const(const float *p) { return (KvConstF *)(size_t)p; }
 
+// An entry of the yz table as one scalar load.
+typedef unsigned KvYz __attribute__((ext_vector_type(KV_YZ)));
+typedef const __attribute__((address_space(4))) KvYz KvYzC;
 
 // IEEE min/max of two floats that are results of arithmetic (never
 // signalling NaNs), without the operand quieting fminf/fmaxf add.
@@ -318,24 +343,49 @@ __device__ __forceinline__ int cvt_flr(float x)
 }
 
 // Backprojection of brick (bxi, byi, bzi) of depth zt <= ZT slices.  Called
-// by all 256 threads of a workgroup (it synchronises).  SR band loads per
-// thread are issued together before their LDS writes.
+// by all 256 threads of a workgroup (it synchronises).
+//
+// The weight of a pixel is the alpha length its ray has inside the voxel,
+// min(Hx, Hy) - max(Lx, Ly) of the x and the (y, z) alpha intervals.  Both
+// are kept non-empty and inside [0, 1] (table bands are clipped when they are
+// staged, row intervals when they are tabulated), so the weight is the row
+// interval's ends clamped to the column's interval and subtracted: where the
+// two overlap the operands are the same FP32 values, elsewhere both ends
+// clamp to one value and the weight is exactly 0.  Two medians and a
+// subtraction replace three minima and maxima, a subtraction and a clamp.
+//
 // FW (mode R): the geometry puts every z plane at alpha >= 1e-6 on every
 // ray (KvGeom::bp_posz), so a positive weight w = H - L has L >= 1e-6 and is
 // at least one FP32 ulp of 1e-6 (~1e-13): w > 1e-24 is then w > 0, and the
-// accumulation takes the clamped weight max(w, +0) with no select (mode A,
-// whose test is w > 0, always does).  The product is a legacy multiply,
-// which gives 0 for a zero weight whatever the pixel value (a skipped
-// pixel's value may be any float, INF and NaN included, as in the
-// reference, which never reads it) and the IEEE product otherwise; adding
-// +0 leaves the sums bit-identical (they are never -0).  The clamp is the
-// subtraction's own [0, 1] output clamp: H <= 1 and L >= +0, so w <= 1 and
-// clamping to [0, 1] is max(w, +0).
-template <int MODE, int EP, int ZT, bool UNIT, int SR, bool FW>
+// accumulation takes the weight with no select (mode A, whose test is w > 0,
+// always does).  The product is a legacy multiply, which gives 0 for a zero
+// weight whatever the pixel value (a skipped pixel's value may be any float,
+// INF and NaN included, as in the reference, which never reads it) and the
+// IEEE product otherwise; adding +0 leaves the sums bit-identical (they are
+// never -0).
+//
+// What bounds it: vector issue for two thirds of the time, and waits for
+// loads.  A wavefront's work per slice is short (2 to 7 detector rows of 2 or
+// 3 columns), so what counts is how many wavefronts a SIMD holds, how many
+// separate loads a slice takes, and what is not done per slice: six
+// workgroups a CU (five: 5.16 ms in mode R where six take 4.51), one scalar
+// load of 16 words per slice, issued a slice ahead, one wide load per
+// detector row, all of the first rows' loads before the first is reduced, and
+// views whose bounds are tested once instead of per slice (`fast` below).
+// Tried and slower or no faster: the next slice's rows loaded a slice ahead
+// (4.40 ms here, but 5 to 15 % more where a workgroup sees fewer rows), the
+// next view's bands touched or loaded early, bricks dealt to the XCDs by
+// neighbourhood.  The MLEM update of 1024x1024x64 voxels from 25 views of
+// 2048x2048 took 5.53 ms (mode R) and 5.45 ms (mode A) with five workgroups,
+// 8-word table entries, per-slice tests and two-sided minima; it takes 4.51
+// and 4.58 ms.  512x512x48 voxels, 21 views of 1024x1024: 0.80 / 0.76 ms
+// before, 0.65 now.
+template <int MODE, int EP, int ZT, bool UNIT, bool FW>
 __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, const float *__restrict__ proj,
                                          float *__restrict__ vol, const float *__restrict__ sens, int bxi, int byi,
                                          int bzi, int zt, BpShared<ZT> &sm)
 {
+    constexpr bool WSUM = MODE == KV_MODE_R || EP == KV_EP_COUNT;
     float *xb = sm.xb;
     int *xbase = sm.xbase;
     auto &accs = sm.accs;
@@ -397,7 +447,9 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
         // detector column lies off the detector are never used (the band
         // slots read below always belong to columns in [0, nu)), so no range
         // test is needed.  A thread stages eight consecutive entries of one
-        // band with two 16-byte loads issued together.
+        // band with two 16-byte loads issued together, clipped to the ray's
+        // alpha range [0, 1] (infinities of mode A's parallel planes with
+        // them), which leaves every positive weight as it is.
         {
             const __amdgpu_buffer_rsrc_t txs =
                 __builtin_amdgcn_make_buffer_rsrc((void *)tx, (short)0, nx1 * g.nu * 4, 0x00020000);
@@ -410,8 +462,8 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                 float *d = xb + i * XBS + j;
 #pragma unroll
                 for (int q = 0; q < 4; ++q) {
-                    d[q] = __uint_as_float(v0[q]);
-                    d[4 + q] = __uint_as_float(v1[q]);
+                    d[q] = clampf(__uint_as_float(v0[q]), 0.f, 1.f);
+                    d[4 + q] = clampf(__uint_as_float(v1[q]), 0.f, 1.f);
                 }
             }
         }
@@ -432,28 +484,140 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
         // (y, z)-row terms: uniform addresses in memory this kernel does not
         // write, read through the constant address space (scalar loads)
         const KvConstF *ty0 = kv_const(ty + (size_t)y * g.nv), *ty1 = kv_const(ty + (size_t)(y + 1) * g.nv);
-        const KvConstF *YZ = kv_const(t.yz + (((size_t)p * g.ny + y) * g.nz + z0) * KV_YZ);
+        KvYzC *YZ = (KvYzC *)(size_t)(t.yz + (((size_t)p * g.ny + y) * g.nz + z0) * KV_YZ);
         // Detector column of the voxel's lateral edges x = cvx and cvx + 1
         // on the plane at the top of slice zi (affine map of the per-view
         // table, bounds only); the bottom plane of slice zi is the top plane
         // of slice zi + 1, so each plane's pair is evaluated once.
         float ua0 = __builtin_fmaf(cvx, Zg[2], Zg[3]), ua1 = __builtin_fmaf(cvx + 1.f, Zg[2], Zg[3]);
+        const unsigned rowbytes = 4u * (unsigned)g.nu;
 
-        for (int zi = 0; zi < nzt; ++zi) {
-            const KvConstF *Z = Zg + zi * KV_ZS;  // plane z0+zi; Z + KV_ZS is the next plane
-            const float ub0 = __builtin_fmaf(cvx, Z[KV_ZS + 2], Z[KV_ZS + 3]);
-            const float ub1 = __builtin_fmaf(cvx + 1.f, Z[KV_ZS + 2], Z[KV_ZS + 3]);
+        // Adds one slice's rows to a voxel's sums: NC columns from lx on, with
+        // their plane crossings A1, A2 (in either order: the medians do not
+        // mind) clipped to [0, 1], equal where a column is not to count.
+        auto reduce = [&](auto nc_tag, const KvYz &E, int lx, const auto &A1, const auto &A2, const auto &L2, float &a,
+                          float &wsm) {
+            constexpr int NC = decltype(nc_tag)::value;
+            auto word = [&](int k) { return __uint_as_float(E[k]); };
+            const int ly = (int)E[0], hyw = (int)E[1];
+            const float lz = word(6), uz = word(7);
+            // Projection values through a bounds-checked buffer resource
+            // over this view's plane: the columns of a row are one 32-bit
+            // offset plus immediate offsets (one wide load) and the row a
+            // scalar offset.  Columns past the row end read the next row
+            // (never used: their weight is not positive), and reads past
+            // the plane return 0 instead of faulting (the check takes the
+            // scalar offset in).
+            constexpr bool LOADS = EP != KV_EP_COUNT && !UNIT;
+            const int off = lx * 4;
+            const unsigned row0 = (unsigned)ly * rowbytes;
+            auto load_row = [&](int r, float (&dst)[NC]) {
+                const int so = (int)(row0 + (unsigned)r * rowbytes);
+                if constexpr (!LOADS) {
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        dst[c] = 0.f;
+                } else if constexpr (NC == 2) {
+                    const auto q = __builtin_amdgcn_raw_buffer_load_b64(prs, off, so, 0);
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        dst[c] = __uint_as_float(q[c]);
+                } else if constexpr (NC == 3) {
+                    const auto q = __builtin_amdgcn_raw_buffer_load_b96(prs, off, so, 0);
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        dst[c] = __uint_as_float(q[c]);
+                } else {
+                    const auto q = __builtin_amdgcn_raw_buffer_load_b128(prs, off, so, 0);
+#pragma unroll
+                    for (int c = 0; c < NC; ++c)
+                        dst[c] = __uint_as_float(q[c]);
+                }
+            };
+            // Row r (detector row ly + r) with its alpha interval
+            // [lo, hi].
+            auto row = [&](int r, const float (&v)[NC], float lo, float hi) {
+                const float lyy = (MODE == KV_MODE_A && UNIT) ? ly2[ly + r] : 0.f;
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    const float w = clampf(hi, A1[c], A2[c]) - clampf(lo, A1[c], A2[c]);
+                    if (EP == KV_EP_COUNT) {
+                        wsm = w > tol ? wsm + 1.f : wsm;
+                    } else if (MODE == KV_MODE_R && FW) {
+                        wsm = wsm + w;
+                        a = a + kv_mul_legacy(w, v[c]);
+                    } else if (MODE == KV_MODE_R) {
+                        const bool ok = w > tol;
+                        wsm = ok ? wsm + w : wsm;
+                        a = ok ? a + w * v[c] : a;
+                    } else if (UNIT) {
+                        const float L = sqrtf((L2[c] + lyy) + lz2);
+                        a = a + w * L;
+                    } else {
+                        // input already multiplied by the ray's length
+                        // factor (kv_launch_scale_a)
+                        a = a + kv_mul_legacy(w, v[c]);
+                    }
+                }
+            };
+            // The first KV_YZ_ROWS rows take their intervals from the
+            // table, and every load is issued before the first row is
+            // reduced; the next ones' loads follow as the registers fall
+            // free, and their y crossings' scalar loads (up to three
+            // entries past the last row: in the table or its padding)
+            // come with the first rows'.
+            constexpr int R = KV_YZ_ROWS;
+            const int n = hyw - ly + 1;
+            float v[R][NC];
+            float y0[R], y1[R];
+            if (n > R) {
+#pragma unroll
+                for (int r = 0; r < R; ++r) {
+                    y0[r] = ty0[ly + R + r];
+                    y1[r] = ty1[ly + R + r];
+                }
+            }
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (r < n)
+                    load_row(r, v[r]);
+#pragma unroll
+            for (int r = 0; r < R; ++r)
+                if (r < n) {
+                    row(r, v[r], word(8 + 2 * r), word(9 + 2 * r));
+                    if (R + r < n)
+                        load_row(R + r, v[r]);
+                }
+            if (n > R) {
+#pragma unroll
+                for (int r = 0; r < R; ++r)
+                    if (R + r < n) {
+                        float lo, hi;
+                        row_interval(y0[r], y1[r], lz, uz, lo, hi);
+                        row(R + r, v[r], lo, hi);
+                    }
+                for (int r = 2 * R; r < n; ++r) {
+                    float lo, hi;
+                    load_row(r, v[0]);
+                    row_interval(ty0[ly + r], ty1[ly + r], lz, uz, lo, hi);
+                    row(r, v[0], lo, hi);
+                }
+            }
+        };
+        auto slice = [&](int zi, const KvYz &E) {
+            auto word = [&](int k) { return __uint_as_float(E[k]); };
+            const float ub0 = __builtin_fmaf(cvx, word(4), word(5));
+            const float ub1 = __builtin_fmaf(cvx + 1.f, word(4), word(5));
             const float mnx = vmin(ua0, ub0), mxx = vmax(ua1, ub1);
             ua0 = ub0;
             ua1 = ub1;
             // the wavefront's detector rows (empty when mode R's voxel
             // centre row lies off the widened detector) and z-plane terms
-            const KvConstF *E = YZ + zi * KV_YZ;
-            const int ly = __float_as_int(E[0]), hyw = __float_as_int(E[1]);
-            const bool has_shadow = __float_as_int(E[2]) != 0;
-            const float lz = E[4], uz = E[5], lzp = E[6];  // one 8-word scalar load with the above
+            const int ly = (int)E[0], hyw = (int)E[1];
+            const bool has_shadow = E[2] != 0;
+            const float lz = word(6), uz = word(7);
             if (ly > hyw)
-                continue;
+                return;
             // Shadow of the voxel box on the detector columns: the columns
             // whose centres lie in [mnx - pad, mxx + pad] (see shadow_affine;
             // floor(a + 1) for ceil(a) only drops a column lying exactly on
@@ -480,9 +644,9 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                 // within the shadow's width (< 5 pixels) of every shadow
                 // column, the window [pc - 5, pc + 5] contains the shadow and
                 // the centre lies on the detector: both tests pass.
-                const float ix = sfx + rdx * Z[1];
+                const float ix = sfx + rdx * Zg[zi * KV_ZS + 1];
                 if (!(ix > ofx - wx && ix < efx + wx))
-                    continue;
+                    return;
                 const float qx = (ix - ofx) * g.sx;
                 // The window is [pc-5, pc+5] with pc = (int)(qx / pu).  When
                 // the shadow fits inside it for every pc within one of an
@@ -505,10 +669,10 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                 }
             }
             if (lx > hxw)
-                continue;
+                return;
             // one running sum per voxel across all views, as the reference
             // accumulates (Projector.cu:727-728)
-            float a = accs[zi][0][tid], wsm = accs[zi][1][tid];
+            float a = accs[zi][0][tid], wsm = WSUM ? accs[zi][1][tid] : 0.f;
             const int ncol = hxw - lx + 1;
             // lx - xb >= 0 and hxw - xb < XBW for both planes' bands, as two
             // unsigned compares (meaningful for the ncol <= 4 it is used with)
@@ -524,124 +688,25 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
             const bool simple = interior && ncol <= 4 && lx + 3 <= g.nu - 1 &&
                                 (unsigned)(lx - xb0) <= (unsigned)(XBW - 4) &&
                                 (unsigned)(lx - xb1) <= (unsigned)(XBW - 4);
-            // x intervals of the (at most NC) columns stay in registers; NC is
-            // the wavefront's widest column range (2, 3 or 4), so narrow
-            // shadows do not pay for four columns per row
+            // crossings of the (at most NC) columns; NC is the wavefront's
+            // widest column range (2, 3 or 4), so narrow shadows do not pay
+            // for four columns per row
             auto rows = [&](auto nc_tag, auto simple_tag) {
                 constexpr int NC = decltype(nc_tag)::value;
                 constexpr bool SIMPLE = decltype(simple_tag)::value;
-                float Lx[NC], Hx[NC], L2[NC];
+                float A1[NC], A2[NC], L2[NC];
 #pragma unroll
                 for (int c = 0; c < NC; ++c) {
-                    Lx[c] = 1.f;
-                    Hx[c] = 0.f;  // empty: any weight <= -1
+                    A1[c] = A2[c] = 0.f;  // empty: any weight is 0
                     L2[c] = 0.f;
                     if (SIMPLE || c < ncol) {
-                        const float a1x = xr0[lx + c - xb0], a2x = xr1[lx + c - xb1];
-                        Lx[c] = bmax(lzp, bmin(a1x, a2x));
-                        Hx[c] = bmin(uz, bmax(a1x, a2x));
+                        A1[c] = xr0[lx + c - xb0];
+                        A2[c] = xr1[lx + c - xb1];
                         if (MODE == KV_MODE_A && UNIT)
                             L2[c] = lx2[lx + c];
                     }
                 }
-                // Projection values through a bounds-checked buffer resource
-                // over this view's plane: the columns of a row are one 32-bit
-                // offset plus immediate offsets (one wide load), columns past
-                // the row end read the next row (never used: their weight is
-                // not positive) and reads past the plane return 0 instead of
-                // faulting.  The next row's values are requested before the
-                // current row is reduced, into two register sets that
-                // alternate between rows (no copies).  (A resource rebuilt
-                // per row on the scalar unit, to save the offset's vector
-                // add, measured 13 % slower: the scalar unit issues at the
-                // vector unit's rate and was the busier of the two.)
-                float va[NC], vb[NC];
-#pragma unroll
-                for (int c = 0; c < NC; ++c)
-                    va[c] = vb[c] = 0.f;
-                constexpr bool LOADS = EP != KV_EP_COUNT && !UNIT;
-                int off = (ly * g.nu + lx) * 4 - 4 * g.nu;
-                auto load_row = [&](int py, float (&dst)[NC]) {
-                    (void)py;
-                    off += 4 * g.nu;
-                    if (LOADS) {
-#pragma unroll
-                        for (int c = 0; c < NC; ++c)
-                            dst[c] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(prs, off + 4 * c, 0, 0));
-                    }
-                };
-                // ly_, hy_: the row's y interval from the wavefront's two
-                // y-plane crossings (uniform: scalar min/max; exact, as the
-                // reference's grouping fmax(fmax(0,mx),fmax(my,mz)) regroups
-                // freely)
-                auto row = [&](int py, const float (&v)[NC], float ly_, float hy_) {
-                    const float lyy = (MODE == KV_MODE_A && UNIT) ? ly2[py] : 0.f;
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) {
-                        const float hmin = bmin(Hx[c], hy_), lmax = bmax(Lx[c], ly_);
-                        if (EP == KV_EP_COUNT) {
-                            const float w = hmin - lmax;
-                            wsm = w > tol ? wsm + 1.f : wsm;
-                        } else if (MODE == KV_MODE_R && FW) {
-                            const float wp = __builtin_amdgcn_fmed3f(hmin - lmax, 0.f, 1.f);
-                            wsm = wsm + wp;
-                            a = a + kv_mul_legacy(wp, v[c]);
-                        } else if (MODE == KV_MODE_R) {
-                            const float w = hmin - lmax;
-                            const bool ok = w > tol;
-                            wsm = ok ? wsm + w : wsm;
-                            a = ok ? a + w * v[c] : a;
-                        } else if (UNIT) {
-                            const float wp = __builtin_amdgcn_fmed3f(hmin - lmax, 0.f, 1.f);
-                            const float L = sqrtf((L2[c] + lyy) + lz2);
-                            a = a + wp * L;
-                        } else {
-                            // input already multiplied by the ray's length
-                            // factor (kv_launch_scale_a)
-                            const float wp = __builtin_amdgcn_fmed3f(hmin - lmax, 0.f, 1.f);
-                            a = a + kv_mul_legacy(wp, v[c]);
-                        }
-                    }
-                };
-                // The y-plane crossings of a row pair are loaded one pair
-                // ahead (row indices clamped to the last row, so every load
-                // stays in the table): the pair's scalar loads complete
-                // while the previous pair is reduced, and the wait that the
-                // first row of a pair needs finds them done.
-                // The y intervals of a row pair come from scalar loads
-                // issued one pair ahead, at the top of the previous pair's
-                // turn, and reduced to (min, max) at its end, so the loads
-                // complete while that pair is reduced (kept in place by
-                // scheduling barriers: the loads of constant memory would
-                // otherwise be re-issued where their values are used).  Rows
-                // up to hyw + 2 <= nv + 1 may be read: they lie in the table,
-                // or in the 16 bytes of padding after it, and are never
-                // used.
-                auto yint = [&](int r, float &lo, float &hi) {
-                    const float a = ty0[r], b = ty1[r];
-                    lo = bmin(a, b);
-                    hi = bmax(a, b);
-                };
-                load_row(ly, va);
-                int py = ly;
-                float lya, hya, lyb, hyb;
-                yint(py, lya, hya);
-                yint(py + 1, lyb, hyb);
-                for (; py < hyw; py += 2) {
-                    const float n0a = ty0[py + 2], n1a = ty1[py + 2], n0b = ty0[py + 3], n1b = ty1[py + 3];
-                    __builtin_amdgcn_sched_barrier(0);
-                    load_row(py + 1, vb);
-                    row(py, va, lya, hya);
-                    load_row(py + 2, va);
-                    row(py + 1, vb, lyb, hyb);
-                    __builtin_amdgcn_sched_barrier(0);
-                    lya = bmin(n0a, n1a);
-                    hya = bmax(n0a, n1a);
-                    lyb = bmin(n0b, n1b);
-                    hyb = bmax(n0b, n1b);
-                }
-                if (py == hyw)
-                    row(py, va, lya, hya);
+                reduce(nc_tag, E, lx, A1, A2, L2, a, wsm);
             };
             auto rows_nc = [&](auto simple_tag) {
                 if (__all(ncol <= 2))
@@ -683,8 +748,84 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                 }
             }
             accs[zi][0][tid] = a;
-            accs[zi][1][tid] = wsm;
+            if (WSUM)
+                accs[zi][1][tid] = wsm;
+        };
+        // The brick's slices of one view, `slice` for each.  Everything a
+        // slice needs from the tables is one 16-word scalar load, issued a
+        // slice ahead (kept there by the empty assembly that takes its
+        // result: a load of constant memory would otherwise be moved to, or
+        // issued again at, its first use and waited for there).
+        auto walk = [&](auto &&one) {
+            KvYz E = *YZ, N;
+            for (int zi = 0; zi < nzt; ++zi) {
+                N = YZ[zi + 1];
+                __builtin_amdgcn_sched_barrier(0);
+                one(zi, E);
+                __builtin_amdgcn_sched_barrier(0);
+                asm volatile("" : "+s"(N));
+                E = N;
+            }
+        };
+
+        // Fast views.  The detector column of a lateral edge is affine in
+        // the planes' scale T, and T (1 / distance from the source) and its
+        // step are monotone over the brick's planes, so the columns of all
+        // its slices lie between those of its first and last plane, and no
+        // slice's shadow is wider than the widest of theirs plus the larger
+        // of the first and last slice's shift.  Where that puts every lane's
+        // shadows, with a pixel to spare, inside the detector and the staged
+        // bands, and at most 2, 3 or 4 columns wide, a slice needs none of
+        // the tests below: it starts at its first column and takes NC of
+        // them (the ones past its shadow have weight 0, as `simple` below).
+        int nc = 0;
+        {
+            const KvConstF *Zb = Zg + nzt * KV_ZS;
+            const KvConstF *Z1 = Zg + KV_ZS, *Zm = Zb - KV_ZS;
+            if (ta > 0.f && tb > 0.f && ta < 1e30f && tb < 1e30f) {
+                const float ua = __builtin_fmaf(cvx, Zg[2], Zg[3]), ub = __builtin_fmaf(cvx, Zb[2], Zb[3]);
+                const float uc = __builtin_fmaf(cvx, Z1[2], Z1[3]), ud = __builtin_fmaf(cvx, Zm[2], Zm[3]);
+                const float lo = fminf(ua, ub), hi = fmaxf(ua, ub);
+                const float width = fmaxf(Zg[2], Zb[2]) + fmaxf(fabsf(uc - ua), fabsf(ub - ud)) + (2.f * pad + 0.01f);
+                const float room = (float)min(xb0, xb1);  // (columns to spare for hi + 1 and NC - 1 more)
+                // (a wider detector's columns would round past the padding)
+                const bool in = nuf < 65536.f && lo >= 1.f && hi <= nuf - 8.f && lo >= (float)max(xb0, xb1) + 1.f &&
+                                hi <= room + (float)(XBW - 7);
+                nc = __all(in && width < 2.f) ? 2 : __all(in && width < 3.f) ? 3 : __all(in && width < 4.f) ? 4 : 0;
+            }
         }
+        auto fast = [&](auto nc_tag) {
+            constexpr int NC = decltype(nc_tag)::value;
+            const float *xl0 = xr0 - xb0, *xl1 = xr1 - xb1;
+            float ua = ua0 + (1.f - pad);
+            walk([&](int zi, const KvYz &E) {
+                const float ub = __builtin_fmaf(cvx, __uint_as_float(E[4]), __uint_as_float(E[3]));
+                const int lx = cvt_flr(vmin(ua, ub));
+                ua = ub;
+                if ((int)E[0] > (int)E[1])
+                    return;
+                float A1[NC], A2[NC], L2[NC];
+#pragma unroll
+                for (int c = 0; c < NC; ++c) {
+                    A1[c] = xl0[lx + c];
+                    A2[c] = xl1[lx + c];
+                    L2[c] = MODE == KV_MODE_A && UNIT ? lx2[lx + c] : 0.f;
+                }
+                float a = accs[zi][0][tid], wsm = WSUM ? accs[zi][1][tid] : 0.f;
+                reduce(nc_tag, E, lx, A1, A2, L2, a, wsm);
+                accs[zi][0][tid] = a;
+                if (WSUM)
+                    accs[zi][1][tid] = wsm;
+            });
+        };
+        if (nc == 2)
+            fast(std::integral_constant<int, 2>{});
+        else if (nc == 3)
+            fast(std::integral_constant<int, 3>{});
+        else if (nc == 4)
+            fast(std::integral_constant<int, 4>{});
+        else
+            walk(slice);
     }
     if (!active)
         return;
@@ -735,21 +876,18 @@ __global__ __launch_bounds__(256) void scale_a_kernel(KvGeom g, KvTables t, cons
 
 // One brick per workgroup.
 template <int MODE, int EP, int ZT, bool UNIT, bool FW>
-__global__ __launch_bounds__(256, 5) void bp_tiled_kernel(KvGeom g, KvTables t, const float *__restrict__ proj,
-                                                       float *__restrict__ vol, const float *__restrict__ sens)
+__global__ __launch_bounds__(256, 6) void bp_tiled_kernel(KvGeom g, KvTables t, const float *__restrict__ proj,
+                                                       float *__restrict__ vol, const float *__restrict__ sens, int zt)
 {
     __shared__ BpShared<ZT> sm;
-    // rounds of 3 loads: mode A measured 3 % faster; mode R's registers would
-    // spill with them
-    bp_brick<MODE, EP, ZT, UNIT, MODE == KV_MODE_A ? 3 : 1, FW>(g, t, proj, vol, sens, blockIdx.x, blockIdx.y,
-                                                               blockIdx.z, ZT, sm);
+    bp_brick<MODE, EP, ZT, UNIT, FW>(g, t, proj, vol, sens, blockIdx.x, blockIdx.y, blockIdx.z, zt, sm);
 }
 
 // Persistent backprojection + MLEM update over a batch of reconstructions:
 // workgroups claim bricks from a global counter until the list is exhausted.
 // Mode A divides by each reconstruction's sensitivity A^T 1.
 template <int MODE>
-__global__ __launch_bounds__(256, 5) void bp_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
+__global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
                                                        long long total, unsigned long long *counter, int iteration)
 {
     __shared__ BpShared<kZT> sm;
@@ -758,7 +896,11 @@ __global__ __launch_bounds__(256, 5) void bp_batch_kernel(const KvProblem *__res
         if (threadIdx.x == 0)
             item_s = (long long)atomicAdd(counter, 1ull);
         __syncthreads();
-        const long long item = item_s;
+        // (uniform: in scalar registers, and with it the descriptor's fields)
+        const long long claimed = item_s;
+        const long long item =
+            (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(claimed >> 32)) << 32) |
+                        (unsigned)__builtin_amdgcn_readfirstlane((int)claimed));
         __syncthreads();
         if (item >= total)
             break;
@@ -773,8 +915,7 @@ __global__ __launch_bounds__(256, 5) void bp_batch_kernel(const KvProblem *__res
         const int bz = (int)(local / per_z);
         const int rem = (int)(local - (long long)bz * per_z);
         const int by = rem / P.bp_bx, bx = rem - by * P.bp_bx;
-        bp_brick<MODE, KV_EP_MLEM, kZT, false, 1, false>(P.g, P.t, P.ratio, P.vol, P.sens, bx, by, bz, P.bp_zt,
-                                                         sm);
+        bp_brick<MODE, KV_EP_MLEM, kZT, false, false>(P.g, P.t, P.ratio, P.vol, P.sens, bx, by, bz, P.bp_zt, sm);
     }
 }
 
@@ -785,15 +926,35 @@ __global__ void zero_u64_kernel(unsigned long long *p, int n)
         p[i] = 0ull;
 }
 
+// Slices per brick.  A workgroup's time is a wait of some 1.7 us per view (the
+// bands, the view's constants and the first detector rows come from memory)
+// and 0.3 to 0.6 us per slice and view, little more with six workgroups on a
+// CU than with one: what counts is to have as many as fit at once, and no
+// second round of a few.  So a volume that fits the chip in one round is cut
+// into as many slabs as keep it there, down to two slices, all of one depth;
+// a larger one into the deepest bricks.  Mode R at 8 slices and as chosen:
+// 128x128x32 voxels, 15 views 60 -> 37 us (2 slices; 1: 53); 256x256x32, 15
+// views 97 -> 85 (6; 5, just past one round: 101); 163x181x54, 13 views 83 ->
+// 69 (5); 561x117x34, 25 views 122 -> 111 (7; 6: 163).
+int brick_depth(const KvGeom &g)
+{
+    constexpr int64_t kSlots = 256 * 6;  // CUs x the launch bounds' workgroups
+    const int64_t tiles = (int64_t)((g.nx + TX - 1) / TX) * ((g.ny + TY - 1) / TY);
+    const int64_t least = (g.nz + kZT - 1) / kZT, most = (g.nz + 1) / 2;
+    const int64_t slabs = std::max(least, std::min(most, kSlots / tiles));
+    return (int)((g.nz + slabs - 1) / slabs);
+}
+
 template <int MODE, int EP, bool UNIT>
 hipError_t launch_tiled(const KvGeom &g, const KvTables &t, const float *proj, float *vol, const float *sens,
                         hipStream_t s)
 {
-    const dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + kZT - 1) / kZT), block(256);
+    const int zt = brick_depth(g);
+    const dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + zt - 1) / zt), block(256);
     if (MODE == KV_MODE_R && (EP == KV_EP_MLEM || EP == KV_EP_SART || EP == KV_EP_PLAIN) && g.bp_posz)
-        bp_tiled_kernel<MODE, EP, kZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens);
+        bp_tiled_kernel<MODE, EP, kZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     else
-        bp_tiled_kernel<MODE, EP, kZT, UNIT, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens);
+        bp_tiled_kernel<MODE, EP, kZT, UNIT, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     return hipGetLastError();
 }
 

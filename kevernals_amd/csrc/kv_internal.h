@@ -146,13 +146,18 @@ struct KvTables {
     // (intersected with the +-5 window around the voxel centre's row in mode
     // R; empty, first > last, when mode R's centre row lies off the widened
     // detector), [2] 1 if the shadow is defined (both planes in front of the
-    // source), as ints; [4] lz = max(0, min z-plane alpha), [5] uz =
-    // min(1, max z-plane alpha), [6] lz with a +0 floor in bit order, as
-    // floats.
+    // source), as ints; [4], [5] = entries 2 and 3 of the zs table's plane
+    // l + 1, [3] = entry 3 plus 1 less the shadow's padding (the floor of
+    // column + 1 - padding is the shadow's first column); [6] lz = max(0, min
+    // z-plane alpha) and [7] uz = min(1, max z-plane alpha); [8 + 2 r], [9 + 2 r]
+    // the alpha interval in which the rays of detector row [0] + r are inside
+    // the voxel row's y and z planes (empty: both ends equal), for the
+    // KV_YZ_ROWS first rows.  One entry more may be read past the end.
     float *yz = nullptr;
 };
 constexpr int KV_ZS = 8;
-constexpr int KV_YZ = 8;
+constexpr int KV_YZ = 16;
+constexpr int KV_YZ_ROWS = 4;
 
 // Epilogues of the projection kernels: plain result, fused MLEM ratio/update,
 // fused SART residual/update, or the count of accepted (ray, voxel) pairs.
