@@ -1,16 +1,13 @@
-// Batched reconstructions: persistent launches over uneven problems,
+// Batched reconstructions: single launches over uneven problems,
 // hipGraph-captured iterations and the tile-shape autotuner.
 //
 // Each reconstruction keeps its own context (geometry, crossing tables,
 // ratio buffer) and volume/data buffers; a device array of KvProblem
-// descriptors tells the persistent kernels where every reconstruction's
+// descriptors tells the kernels where every reconstruction's
 // forward tiles and backprojection bricks sit in the batch-wide work list.
 // One iteration of the whole batch is two launches: the forward pass (ratio
 // epilogue) for every reconstruction, then the backprojection (update
-// epilogue).  Work items are claimed from counters (one per XCD list for the
-// forward pass, one for the backprojection); the counters
-// are cleared by a small kernel (not hipMemsetAsync, which misbehaves inside
-// captured graphs on replay), so the same sequence runs eagerly or replayed.
+// epilogue), a workgroup per item; the same sequence runs eagerly or replayed.
 #include <algorithm>
 #include <cstdio>
 #include <cstring>
@@ -30,10 +27,7 @@ struct kv_batch {
     std::vector<float *> vol, data;
     std::vector<KvProblem> probs;
     KvProblem *d_probs = nullptr;
-    unsigned long long *d_counters = nullptr;
-    int counters_cap = 0;
     long long fp_total = 0, bp_total = 0;
-    int fp_grid = 0, bp_grid = 0;
     // captured iteration sequence
     hipGraphExec_t exec = nullptr;
     int exec_iters = -1;
@@ -71,25 +65,33 @@ void layout_items(kv_batch *b)
     for (auto &P : b->probs) {
         if (P.fp_part == KV_FP_ROWS) {
             P.fp_chunk = KV_ROW_CY;
-            P.fp_tx = kv_row_tiles_x(b->mode == KV_MODE_A ? P.g.nu : P.g.row_cols);
+            P.fp_tx = ((b->mode == KV_MODE_A ? P.g.nu : P.g.row_cols) + 63) / 64 * KV_ROW_CY;
             P.fp_ty = kv_row_tiles_y(P.g.nv);
         } else if (P.fp_part == KV_FP_EDGES) {
             P.fp_chunk = KV_FP_STRIPE / KV_FP_TILE;
-            P.fp_tx = kv_edge_tiles_x(P.g.edge_cols);
+            P.fp_tx = (P.g.edge_cols + KV_FP_TILE - 1) / KV_FP_TILE;
             P.fp_ty = kv_edge_tiles_y(P.g.nv);
         } else {
             const int L = P.fp_layout, wu = 64 / L;
             P.fp_chunk = std::max(1, KV_FP_STRIPE / wu);
-            const int span = KV_XCDS * P.fp_chunk;
-            P.fp_tx = ((P.g.nu + wu - 1) / wu + span - 1) / span * span;
+            P.fp_tx = (P.g.nu + wu - 1) / wu;
             P.fp_ty = (P.g.nv + 4 * L - 1) / (4 * L);
         }
-        P.fp_nch = P.fp_tx / (KV_XCDS * P.fp_chunk);
+        // A view's tiles go round the lists in stripes of fp_chunk, row after
+        // row.  Rows of a round and more are padded to whole rounds, so that a
+        // list keeps its columns; shorter ones follow each other without
+        // padding: an empty tile still costs a workgroup and its descriptor's
+        // loads (the forward pass of six reconstructions of 106x375x69 and
+        // less, detectors of 190 columns and less: 660 us padded, 170 not).
+        const int span = KV_XCDS * P.fp_chunk;
+        if (P.fp_tx >= span)
+            P.fp_tx = (P.fp_tx + span - 1) / span * span;
+        P.fp_nch = (int)(((long long)P.fp_tx * P.fp_ty + span - 1) / span);
         P.fp_dchunk = kv_udiv((unsigned)P.fp_chunk);
         P.fp_dnch = kv_udiv((unsigned)P.fp_nch);
-        P.fp_dty = kv_udiv((unsigned)P.fp_ty);
+        P.fp_dtx = kv_udiv((unsigned)P.fp_tx);
         P.fp_first = fp;
-        fp += (long long)P.g.np * P.fp_ty * (P.fp_tx / KV_XCDS);
+        fp += (long long)P.g.np * P.fp_nch * P.fp_chunk;
         P.bp_bx = (P.g.nx + 63) / 64;
         P.bp_by = (P.g.ny + 3) / 4;
         P.bp_bz = P.fp_part == KV_FP_EDGES ? 0 : (P.g.nz + P.bp_zt - 1) / P.bp_zt;
@@ -109,48 +111,23 @@ kv_status upload_probs(kv_batch *b)
     return e == hipSuccess ? KV_OK : fail_hip(e, "upload of batch descriptors");
 }
 
-// per iteration: KV_XCDS forward-list counters, one backprojection counter
-constexpr int kCountersPerIter = KV_XCDS + 1;
-
-kv_status ensure_counters(kv_batch *b, int iters)
-{
-    const int need = kCountersPerIter * std::max(iters, 1);
-    if (need <= b->counters_cap)
-        return KV_OK;
-    if (b->d_counters)
-        (void)hipFree(b->d_counters);
-    b->d_counters = nullptr;
-    b->counters_cap = 0;
-    const hipError_t e = hipMalloc((void **)&b->d_counters, (size_t)need * sizeof(unsigned long long));
-    if (e != hipSuccess)
-        return e == hipErrorOutOfMemory ? (kv_set_error("out of device memory"), KV_ERR_NOMEM)
-                                        : fail_hip(e, "counter allocation");
-    b->counters_cap = need;
-    // the graph refers to the old counters
-    if (b->exec) {
-        (void)hipGraphExecDestroy(b->exec);
-        b->exec = nullptr;
-    }
-    return KV_OK;
-}
-
 // The iteration sequence on the batch stream (eagerly or under capture).
 hipError_t enqueue_iterations(kv_batch *b, int iters, float relax)
 {
-    hipError_t e = kv_launch_zero_u64(b->d_counters, kCountersPerIter * iters, b->stream);
+    bool posz = true;
+    for (int i = 0; i < b->n; ++i)
+        posz = posz && b->probs[(size_t)i].g.bp_posz;
+    hipError_t e = hipSuccess;
     for (int k = 0; k < iters && e == hipSuccess; ++k) {
-        unsigned long long *c = b->d_counters + (size_t)kCountersPerIter * k;
-        e = kv_launch_fp_batch(b->mode, b->d_probs, (int)b->probs.size(), b->fp_total, c, k, relax, b->fp_grid, b->stream);
+        e = kv_launch_fp_batch(b->mode, b->d_probs, (int)b->probs.size(), b->fp_total, k, relax, b->stream);
         if (e == hipSuccess)
-            e = kv_launch_bp_batch(b->mode, b->d_probs, b->n, b->bp_total, c + KV_XCDS, k, b->bp_grid, b->stream);
+            e = kv_launch_bp_batch(b->mode, b->d_probs, b->n, b->bp_total, k, posz, b->stream);
     }
     return e;
 }
 
 kv_status run(kv_batch *b, int iters, float relax, bool use_graph, float *ms)
 {
-    if (kv_status st = ensure_counters(b, iters))
-        return st;
     if (kv_status st = upload_probs(b))
         return st;
     hipError_t e = hipEventRecord(b->ev0, b->stream);
@@ -242,8 +219,6 @@ void release(kv_batch *b)
             kv_destroy(c);
     if (b->d_probs)
         (void)hipFree(b->d_probs);
-    if (b->d_counters)
-        (void)hipFree(b->d_counters);
     if (b->ev0)
         (void)hipEventDestroy(b->ev0);
     if (b->ev1)
@@ -325,13 +300,6 @@ kv_status kv_batch_create(int device, int n, const kv_geometry *geoms, int mode,
         e = hipMalloc((void **)&b->d_probs, 2 * (size_t)n * sizeof(KvProblem));
         if (e != hipSuccess)
             st = fail_hip(e, "descriptor allocation");
-    }
-    if (st == KV_OK) {
-        int cus = 0;
-        (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device);
-        cus = cus > 0 ? cus : 1;
-        b->fp_grid = cus * kv_fp_batch_blocks_per_cu(mode);
-        b->bp_grid = cus * kv_bp_batch_blocks_per_cu(mode);
     }
     if (st != KV_OK) {
         release(b);

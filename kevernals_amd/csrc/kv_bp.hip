@@ -883,30 +883,23 @@ __global__ __launch_bounds__(256, 6) void bp_tiled_kernel(KvGeom g, KvTables t, 
     bp_brick<MODE, EP, ZT, UNIT, FW>(g, t, proj, vol, sens, blockIdx.x, blockIdx.y, blockIdx.z, zt, sm);
 }
 
-// Persistent backprojection + MLEM update over a batch of reconstructions:
-// workgroups claim bricks from a global counter until the list is exhausted.
-// Mode A divides by each reconstruction's sensitivity A^T 1.
-template <int MODE>
+// Backprojection + MLEM update over a batch of reconstructions, a workgroup
+// per brick (the hardware's dispatch order stands in for a work queue: a
+// queue's claims, atomics on one word of 40 to 70 ns each, took as long as the
+// bricks of small reconstructions).  Mode A divides by each reconstruction's
+// sensitivity A^T 1.  FW: as bp_brick's, for every reconstruction.
+template <int MODE, bool FW>
 __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
-                                                       long long total, unsigned long long *counter, int iteration)
+                                                          long long total, int iteration)
 {
     __shared__ BpShared<kZT> sm;
-    __shared__ long long item_s;
-    for (;;) {
-        if (threadIdx.x == 0)
-            item_s = (long long)atomicAdd(counter, 1ull);
-        __syncthreads();
-        // (uniform: in scalar registers, and with it the descriptor's fields)
-        const long long claimed = item_s;
-        const long long item =
-            (long long)(((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(claimed >> 32)) << 32) |
-                        (unsigned)__builtin_amdgcn_readfirstlane((int)claimed));
-        __syncthreads();
-        if (item >= total)
-            break;
+    for (long long item = blockIdx.x; item < total; item += gridDim.x) {
+        // the last descriptor whose items begin at or before this one (by
+        // halves: each step waits for a load)
         int pi = 0;
-        while (pi + 1 < nprob && probs[pi + 1].bp_first <= item)
-            ++pi;
+        for (int n = nprob; n > 1; n -= n / 2)
+            if (probs[pi + n / 2].bp_first <= item)
+                pi += n / 2;
         const KvProblem &P = probs[pi];
         if (iteration >= P.iters)
             continue;
@@ -915,15 +908,8 @@ __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__res
         const int bz = (int)(local / per_z);
         const int rem = (int)(local - (long long)bz * per_z);
         const int by = rem / P.bp_bx, bx = rem - by * P.bp_bx;
-        bp_brick<MODE, KV_EP_MLEM, kZT, false, false>(P.g, P.t, P.ratio, P.vol, P.sens, bx, by, bz, P.bp_zt, sm);
+        bp_brick<MODE, KV_EP_MLEM, kZT, false, FW>(P.g, P.t, P.ratio, P.vol, P.sens, bx, by, bz, P.bp_zt, sm);
     }
-}
-
-__global__ void zero_u64_kernel(unsigned long long *p, int n)
-{
-    const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n)
-        p[i] = 0ull;
 }
 
 // Slices per brick.  A workgroup's time is a wait of some 1.7 us per view (the
@@ -960,31 +946,17 @@ hipError_t launch_tiled(const KvGeom &g, const KvTables &t, const float *proj, f
 
 }  // namespace
 
-hipError_t kv_launch_bp_batch(int mode, const KvProblem *probs, int nprob, long long total,
-                              unsigned long long *counter, int iteration, int grid, hipStream_t s)
+hipError_t kv_launch_bp_batch(int mode, const KvProblem *probs, int nprob, long long total, int iteration,
+                              bool posz, hipStream_t s)
 {
+    const int grid = (int)std::min<long long>(KV_BATCH_GRID, total);
     if (mode == KV_MODE_A)
-        bp_batch_kernel<KV_MODE_A><<<grid, 256, 0, s>>>(probs, nprob, total, counter, iteration);
+        bp_batch_kernel<KV_MODE_A, false><<<grid, 256, 0, s>>>(probs, nprob, total, iteration);
+    else if (posz)
+        bp_batch_kernel<KV_MODE_R, true><<<grid, 256, 0, s>>>(probs, nprob, total, iteration);
     else
-        bp_batch_kernel<KV_MODE_R><<<grid, 256, 0, s>>>(probs, nprob, total, counter, iteration);
+        bp_batch_kernel<KV_MODE_R, false><<<grid, 256, 0, s>>>(probs, nprob, total, iteration);
     return hipGetLastError();
-}
-
-hipError_t kv_launch_zero_u64(unsigned long long *p, int n, hipStream_t s)
-{
-    zero_u64_kernel<<<(n + 255) / 256, 256, 0, s>>>(p, n);
-    return hipGetLastError();
-}
-
-int kv_bp_batch_blocks_per_cu(int mode)
-{
-    int n = 0;
-    const hipError_t e =
-        mode == KV_MODE_A ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, bp_batch_kernel<KV_MODE_A>, 256, 0)
-                          : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, bp_batch_kernel<KV_MODE_R>, 256, 0);
-    if (e != hipSuccess)
-        return 2;
-    return n > 0 ? n : 1;
 }
 
 hipError_t kv_launch_tables_r(const KvGeom &g, const KvTables &t, hipStream_t s)

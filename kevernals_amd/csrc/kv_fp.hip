@@ -536,71 +536,44 @@ __global__ __launch_bounds__(256) void fp_r_kernel(KvGeom g, const float *__rest
     fp_r_ray<EP>(g, vol, out, data, relax, p, u, v);
 }
 
-// Tiles per claim of the batch kernels, at most.  The claims of a list are
-// atomics on one word, some 70 ns each: a mode-R / mode-A iteration of six
-// reconstructions of 384x320x48 and less (18 000 tiles a list) took 1.67 /
-// 1.65 ms with one tile per claim, 0.96 / 0.90 with four, 0.96 / 0.84 with
-// eight.
-constexpr int KV_FP_CLAIM = 8;
-
-// Persistent forward pass over a batch of reconstructions.  The tiles sit in
-// KV_XCDS lists (KvProblem), list k holding the stripes an XCD-ordered
-// launch gives XCD k (fp_xcd_tile); `total` items per list, one counter per
-// list.  A workgroup claims `per` tiles at a time from the list of the XCD a one-dimensional
-// launch places it on (blockIdx.x % KV_XCDS), then from the other lists in
-// turn, until every list is exhausted: every tile is processed once whatever
-// the placement, which only decides the caches' locality.  Problems whose
-// iteration count is reached skip their tiles; padding columns (u past the
-// detector) are skipped at the bounds test.
+// Forward pass over a batch of reconstructions.  The tiles sit in KV_XCDS
+// lists (KvProblem), list k holding the stripes an XCD-ordered launch gives
+// XCD k (fp_xcd_tile), `total` items per list; the launch deals a workgroup per
+// item round the lists, as a one-dimensional launch deals workgroups round the
+// XCDs (the placement only decides the caches' locality).  Workgroups that
+// stay and claim tiles from a counter per list were slower: claims are atomics
+// on one word, some 70 ns each.  An iteration of six reconstructions of
+// 384x320x48 voxels and less (18 000 tiles a list) took 1.67 / 1.65 ms in mode
+// R / A with one tile per claim, 0.96 / 0.84 with eight; it takes 0.75 / 0.72.
+// Problems whose iteration count is reached skip their tiles; padding columns
+// (u past the detector) are skipped at the bounds test.
 template <typename Tile>
 __device__ __forceinline__ void fp_batch_tiles(const KvProblem *__restrict__ probs, int nprob, long long total,
-                                               unsigned long long *counters, int per, int iteration, Tile &&tile)
+                                               int iteration, Tile &&tile)
 {
-    __shared__ long long item_s;
-    const int own = (int)(blockIdx.x % (unsigned)KV_XCDS);
-    for (int c = 0; c < KV_XCDS; ++c) {
-        const int k = (own + c) % KV_XCDS;
-        // the next claim is in flight while this one's tiles are walked
-        long long claim = 0;
-        if (threadIdx.x == 0)
-            claim = (long long)atomicAdd(counters + k, (unsigned long long)per);
-        for (long long item = 0, end = 0;; ++item) {
-            if (item >= end) {
-                if (threadIdx.x == 0)
-                    item_s = claim;
-                __syncthreads();
-                // the same for the workgroup: in scalar registers, and with
-                // it the descriptor's fields and the tile's row (left to
-                // itself the compiler takes a value read from LDS to differ
-                // between lanes, and reads them by vector loads)
-                const long long claimed = item_s;
-                item = (long long)(
-                    ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(claimed >> 32)) << 32) |
-                    (unsigned)__builtin_amdgcn_readfirstlane((int)claimed));
-                __syncthreads();
-                if (item >= total)
-                    break;
-                end = min(item + per, total);
-                if (threadIdx.x == 0)
-                    claim = (long long)atomicAdd(counters + k, (unsigned long long)per);
-            }
-            int pi = 0;
-            while (pi + 1 < nprob && probs[pi + 1].fp_first <= item)
-                ++pi;
-            const KvProblem &P = probs[pi];
-            if (iteration >= P.iters)
-                continue;
-            // item indices within a reconstruction stay far below 2^31 (it
-            // has fewer than 2^31 rays, 256 per tile): 32-bit divisions by
-            // the precomputed multipliers
-            const unsigned local = (unsigned)(item - P.fp_first);
-            const unsigned ch = (unsigned)P.fp_chunk, nch = (unsigned)P.fp_nch;
-            const unsigned jc = udiv(local, P.fp_dchunk), r = udiv(jc, P.fp_dnch);
-            const int tx = (int)(((jc - r * nch) * KV_XCDS + (unsigned)k) * ch + (local - jc * ch));
-            const unsigned q = udiv(r, P.fp_dty);
-            const int ty = (int)(r - q * (unsigned)P.fp_ty), p = (int)q;
-            tile(P, p, tx, ty);
-        }
+    const int k = (int)(blockIdx.x % (unsigned)KV_XCDS);  // (the grid is a multiple of KV_XCDS)
+    for (long long item = blockIdx.x / (unsigned)KV_XCDS; item < total; item += gridDim.x / (unsigned)KV_XCDS) {
+        // the last descriptor whose items begin at or before this one (by
+        // halves: each step waits for a load)
+        int pi = 0;
+        for (int n = nprob; n > 1; n -= n / 2)
+            if (probs[pi + n / 2].fp_first <= item)
+                pi += n / 2;
+        const KvProblem &P = probs[pi];
+        if (iteration >= P.iters)
+            continue;
+        // item indices within a reconstruction stay far below 2^31 (it
+        // has fewer than 2^31 rays, 256 per tile): 32-bit divisions by
+        // the precomputed multipliers
+        const unsigned local = (unsigned)(item - P.fp_first);
+        const unsigned ch = (unsigned)P.fp_chunk, nch = (unsigned)P.fp_nch;
+        const unsigned jc = udiv(local, P.fp_dchunk), r = udiv(jc, P.fp_dnch);
+        const unsigned lin = ((jc - r * nch) * KV_XCDS + (unsigned)k) * ch + (local - jc * ch);
+        const unsigned q = udiv(lin, P.fp_dtx);
+        const int ty = (int)q, tx = (int)(lin - q * (unsigned)P.fp_tx), p = (int)r;
+        if (ty >= P.fp_ty)
+            continue;  // padding of the view's last stripes
+        tile(P, p, tx, ty);
     }
 }
 
@@ -1821,10 +1794,9 @@ __global__ __launch_bounds__(256) void fp_a_row_multi_kernel(KvGeom g, KvMulti m
 
 template <int EP>
 __global__ __launch_bounds__(256) void fp_r_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
-                                                         long long total, unsigned long long *counters, int per,
-                                                         int iteration, float relax)
+                                                         long long total, int iteration, float relax)
 {
-    fp_batch_tiles(probs, nprob, total, counters, per, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
+    fp_batch_tiles(probs, nprob, total, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
         int u, v;
         if (P.fp_part == KV_FP_ROWS) {
             int first, end;
@@ -1847,10 +1819,9 @@ __global__ __launch_bounds__(256) void fp_r_batch_kernel(const KvProblem *__rest
 // Persistent mode-A forward pass (MLEM ratio) over a batch, as
 // fp_r_batch_kernel; reconstructions with segment lists run row by row.
 __global__ __launch_bounds__(256) void fp_a_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
-                                                         long long total, unsigned long long *counters, int per,
-                                                         int iteration)
+                                                         long long total, int iteration)
 {
-    fp_batch_tiles(probs, nprob, total, counters, per, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
+    fp_batch_tiles(probs, nprob, total, iteration, [&](const KvProblem &P, int p, int tx, int ty) {
         int u, v;
         if (P.fp_part == KV_FP_ROWS) {
             fp_row_pixel(tx, ty, u, v);
@@ -2089,25 +2060,13 @@ hipError_t kv_launch_trace(const KvGeom &g, int mode, int nrays, const int32_t *
     return hipGetLastError();
 }
 
-hipError_t kv_launch_fp_batch(int mode, const KvProblem *probs, int nprob, long long total,
-                              unsigned long long *counters, int iteration, float relax, int grid, hipStream_t s)
+hipError_t kv_launch_fp_batch(int mode, const KvProblem *probs, int nprob, long long total, int iteration, float relax,
+                              hipStream_t s)
 {
-    // as many tiles per claim as leave a workgroup some eight claims
-    const int per = (int)std::max<long long>(1, std::min<long long>(KV_FP_CLAIM, total * KV_XCDS / (8ll * grid)));
+    const int grid = (int)std::min<long long>(KV_BATCH_GRID, total * KV_XCDS);
     if (mode == KV_MODE_A)
-        fp_a_batch_kernel<<<grid, 256, 0, s>>>(probs, nprob, total, counters, per, iteration);
+        fp_a_batch_kernel<<<grid, 256, 0, s>>>(probs, nprob, total, iteration);
     else
-        fp_r_batch_kernel<KV_EP_MLEM><<<grid, 256, 0, s>>>(probs, nprob, total, counters, per, iteration, relax);
+        fp_r_batch_kernel<KV_EP_MLEM><<<grid, 256, 0, s>>>(probs, nprob, total, iteration, relax);
     return hipGetLastError();
-}
-
-int kv_fp_batch_blocks_per_cu(int mode)
-{
-    int n = 0;
-    const hipError_t e = mode == KV_MODE_A
-                             ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fp_a_batch_kernel, 256, 0)
-                             : hipOccupancyMaxActiveBlocksPerMultiprocessor(&n, fp_r_batch_kernel<KV_EP_MLEM>, 256, 0);
-    if (e != hipSuccess)
-        return 4;
-    return n > 0 ? n : 1;
 }

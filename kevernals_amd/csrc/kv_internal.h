@@ -169,12 +169,12 @@ enum KvEpilogue { KV_EP_PLAIN = 0, KV_EP_MLEM = 1, KV_EP_SART = 2, KV_EP_COUNT =
 // two descriptors, the second without bricks.
 enum KvFpPart { KV_FP_WHOLE = 0, KV_FP_ROWS = 1, KV_FP_EDGES = 2 };
 
-// One reconstruction of a batch, as the persistent kernels read it (device
+// One reconstruction of a batch, as the batch kernels read it (device
 // memory, wave-uniform loads).  Work items are numbered consecutively over
 // the batch.  Forward tiles sit in KV_XCDS lists, one per XCD (stripes of
 // fp_chunk tile columns, stripe i in list i % KV_XCDS, as fp_xcd_tile): this
-// reconstruction holds items [fp_first, fp_first + views*fp_ty*fp_tx/KV_XCDS)
-// of every list, fp_tx being padded to whole stripes for all lists.
+// reconstruction holds items [fp_first, fp_first + views*fp_nch*fp_chunk)
+// of every list, each view being padded to whole rounds of stripes.
 // Backprojection bricks: [bp_first, bp_first + bp_bx*bp_by*bp_bz).
 struct KvProblem {
     KvGeom g;
@@ -187,10 +187,10 @@ struct KvProblem {
     int fp_layout;             // forward tile layout: 1, 2, 4 or 8 rows per wavefront
     int fp_part;               // KvFpPart
     int owner;                 // index of the reconstruction (its own, or its first descriptor's)
-    int fp_tx, fp_ty;          // forward tiles per view (fp_tx padded to a multiple of KV_XCDS * fp_chunk)
-    int fp_chunk;              // tile columns per XCD stripe
-    int fp_nch;                // stripes per tile row in one list: fp_tx / (KV_XCDS * fp_chunk)
-    KvUDiv fp_dchunk, fp_dnch, fp_dty;  // divisors fp_chunk, fp_nch, fp_ty
+    int fp_tx, fp_ty;          // forward tiles per view (fp_tx padded to whole rounds of stripes where it has one)
+    int fp_chunk;              // tiles per XCD stripe
+    int fp_nch;                // stripes per view in one list
+    KvUDiv fp_dchunk, fp_dnch, fp_dtx;  // divisors fp_chunk, fp_nch, fp_tx
     long long fp_first;
     int bp_zt;                 // backprojection brick depth: 4 or 8 slices
     int bp_bx, bp_by, bp_bz;   // bricks per axis
@@ -345,17 +345,15 @@ hipError_t kv_launch_bp_a(const KvGeom &g, const KvTables &t, const float *proj,
                           const float *sens, bool unit_input, hipStream_t s);
 // out = proj * length factor of each ray (mode-A tables), np*nv*nu values.
 hipError_t kv_launch_scale_a(const KvGeom &g, const KvTables &t, const float *proj, float *out, hipStream_t s);
-// Batched persistent passes (MLEM epilogues, mode R or A).  `grid` workgroups
-// of 256 threads claim work items: the forward pass from counters[0 ..
-// KV_XCDS-1] (one per XCD list of `total` items), the backprojection from
-// *counter; all zero before the launch.
-hipError_t kv_launch_fp_batch(int mode, const KvProblem *probs, int nprob, long long total,
-                              unsigned long long *counters, int iteration, float relax, int grid, hipStream_t s);
-hipError_t kv_launch_bp_batch(int mode, const KvProblem *probs, int nprob, long long total,
-                              unsigned long long *counter, int iteration, int grid, hipStream_t s);
-hipError_t kv_launch_zero_u64(unsigned long long *p, int n, hipStream_t s);
-int kv_fp_batch_blocks_per_cu(int mode);
-int kv_bp_batch_blocks_per_cu(int mode);
+// Batched passes (MLEM epilogues, mode R or A), a workgroup of 256 threads per
+// work item and no more than KV_BATCH_GRID workgroups, which then take several:
+// the forward pass over KV_XCDS lists of `total` items, the backprojection over
+// one.  posz: every reconstruction has KvGeom::bp_posz.
+constexpr long long KV_BATCH_GRID = 1ll << 22;  // a multiple of KV_XCDS
+hipError_t kv_launch_fp_batch(int mode, const KvProblem *probs, int nprob, long long total, int iteration, float relax,
+                              hipStream_t s);
+hipError_t kv_launch_bp_batch(int mode, const KvProblem *probs, int nprob, long long total, int iteration, bool posz,
+                              hipStream_t s);
 // Per-device address of the no-allocation shift-and-add staging array
 // (kv_misc.hip): _init resolves it once per device, with that device current;
 // kv_internal_scratch returns it (nullptr before _init).  Word layout:
