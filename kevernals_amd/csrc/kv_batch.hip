@@ -65,11 +65,11 @@ void layout_items(kv_batch *b)
     for (auto &P : b->probs) {
         if (P.fp_part == KV_FP_ROWS) {
             P.fp_chunk = KV_ROW_CY;
-            P.fp_tx = ((b->mode == KV_MODE_A ? P.g.nu : P.g.row_cols) + 63) / 64 * KV_ROW_CY;
+            P.fp_tx = kv_row_tiles_x(b->mode == KV_MODE_A ? P.g.nu : P.g.row_cols);
             P.fp_ty = kv_row_tiles_y(P.g.nv);
         } else if (P.fp_part == KV_FP_EDGES) {
             P.fp_chunk = KV_FP_STRIPE / KV_FP_TILE;
-            P.fp_tx = (P.g.edge_cols + KV_FP_TILE - 1) / KV_FP_TILE;
+            P.fp_tx = kv_edge_tiles_x(P.g.edge_cols);
             P.fp_ty = kv_edge_tiles_y(P.g.nv);
         } else {
             const int L = P.fp_layout, wu = 64 / L;

@@ -112,10 +112,11 @@ inline KvUDiv kv_udiv(unsigned d)
 
 // Mapping of a one-dimensional forward launch onto tiles (kv_fp.hip
 // fp_xcd_tile): tile layout, stripe width in tiles, stripes per tile row and
-// tile rows per view with their divisors, first view of the launch.
+// tile rows per view with their divisors, first view of the launch; ntx, if
+// not 0: a view is one row, of the detector's rows of ntx tiles.
 struct KvFpMap {
-    int layout, chunk, nch, gy, p0;
-    KvUDiv dchunk, dnch, dgy;
+    int layout, chunk, nch, gy, p0, ntx;
+    KvUDiv dchunk, dnch, dgy, dntx;
 };
 
 // Per-view plane-crossing tables.  For mode R an entry is the reference's
@@ -299,20 +300,12 @@ constexpr int KV_ROW_CY = 4;
 constexpr int KV_FP_BATCH_LAYOUT_R = 8;
 constexpr int KV_FP_BATCH_LAYOUT_A = 4;
 
-// Tiles of the row-by-row walks along tx (padded to a chunk per XCD) and ty.
-inline int kv_row_tiles_x(int nu)
-{
-    const int w = 64 * KV_XCDS;
-    return (nu + w - 1) / w * KV_XCDS * KV_ROW_CY;
-}
+// Tiles of the row-by-row walks along tx and ty.
+inline int kv_row_tiles_x(int nu) { return (nu + 63) / 64 * KV_ROW_CY; }
 inline int kv_row_tiles_y(int nv) { return (nv + 4 * KV_ROW_CY - 1) / (4 * KV_ROW_CY); }
 // Tiles of 8 columns by 32 rows over mode R's other columns.
 constexpr int KV_FP_TILE = 64 / KV_FP_LAYOUT;
-inline int kv_edge_tiles_x(int cols)
-{
-    const int span = KV_XCDS * (KV_FP_STRIPE / KV_FP_TILE);
-    return ((cols + KV_FP_TILE - 1) / KV_FP_TILE + span - 1) / span * span;
-}
+inline int kv_edge_tiles_x(int cols) { return (cols + KV_FP_TILE - 1) / KV_FP_TILE; }
 inline int kv_edge_tiles_y(int nv) { return (nv + 4 * KV_FP_LAYOUT - 1) / (4 * KV_FP_LAYOUT); }
 
 hipError_t kv_launch_fp_r(const KvGeom &g, const float *vol, float *out, int epilogue, const float *data,
