@@ -26,7 +26,7 @@ sys.path.insert(0, ROOT)
 
 HBM_PEAK_GBS = 8000.0
 # rocprofv3 (demangled) names of the two fused MLEM kernels
-FP_KERNEL = "fp_r_kernel<1>"
+FP_KERNEL = "fp_r_row_kernel<1>"
 BP_KERNEL = "bp_tiled_kernel<0, 1, 8, false, true>"
 METRIC = "time to RMSE≤1% vs converged MLEM, learned vs plain; GRays/s fwd+back"
 
@@ -168,7 +168,7 @@ def traffic_from_profiles(kernel):
 
 def bench_batched(args, torch, K, G):
     """32 uneven plain-MLEM reconstructions (seed 3; phantoms 3000+i), 15
-    iterations each per step, in the persistent batched launches replayed
+    iterations each per step, in batched launches replayed
     from one captured hipGraph; tiles chosen by the autotuner."""
     from kevernals_amd.phantom import phantom
 
@@ -218,7 +218,7 @@ def bench_batched(args, torch, K, G):
         "data": "synthetic (seeded ellipsoid phantoms, noise-free reference-discretisation projections)",
         "config": {
             "workload": "batched plain MLEM: 32 uneven reconstructions x 15 iterations per step, "
-                        "persistent launches replayed from a hipGraph",
+                        "shared launches replayed from a hipGraph",
             "reconstructions": len(gs),
             "iterations": iters,
             "total_voxels": vox,
@@ -446,7 +446,7 @@ def _learned_schedule(name):
 def learned_batched_runs(torch, K, G, n, weights=LEARNED_WEIGHTS):
     """Learned plus batched at full size: n reconstructions of
     1024x1024x64 / 25 views (phantom seeds 5000+i with 200
-    microcalcifications, I0 = 5e3) in one mode-A batch (persistent launches,
+    microcalcifications, I0 = 5e3) in one mode-A batch (shared launches,
     hipGraph replay).  Plain batched MLEM-A against the accelerated batched
     reconstruction: the two-stretch trajectory-jump schedule (18 batched
     MLEM iterations; each reconstruction's jumps gated on its Poisson
@@ -679,10 +679,10 @@ def bench_sart_saa(K, ctx, g, data, torch, saa_reps=5):
                  "wall_ms_per_iteration": round(sart_wall, 4),
                  "grays_per_s": round(g.nrays / (sart_ms * 1e-3) / 1e9, 4)},
         "shift_and_add": {"planes": len(planes), "ms": round(saa_ms, 4),
-                          "roofline": {"bound": "hbm", "kernel": "saa_kernel",
+                          "roofline": {"bound": "hbm", "kernel": "saa_kernel<8, 32>",
                                        "achieved": round(saa_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                        "frac": round(saa_gbs / HBM_PEAK_GBS, 4),
-                                       "traffic": traffic_from_profiles("saa_kernel"),
+                                       "traffic": traffic_from_profiles("saa_kernel<8, 32>"),
                                        "algorithmic_bytes": saa_bytes}},
     }
 

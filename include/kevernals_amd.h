@@ -168,9 +168,11 @@ kv_status kv_log_likelihood(kv_context *ctx, const float *d_data, const float *d
 /* kv_log_likelihood of n <= KV_LL_MAX volumes (out[i] for d_vols[i], each
  * bit-identical to a kv_log_likelihood call) with one ray walk for all of
  * them: the likelihood gates compare up to three candidates.  Uses two more
- * projection-sized buffers of the context and, for n >= 2, a buffer of 16
- * bytes per voxel into which the volumes are interleaved (all allocated on
- * first use and kept with the context).  Synchronous. */
+ * projection-sized buffers of the context and, for n >= 2 on a geometry
+ * without segment lists (which are made unless they would take over 1 GiB or
+ * memory is short), a buffer of 16 bytes per voxel into which the volumes are
+ * interleaved (all allocated on first use and kept with the context).
+ * Synchronous. */
 #define KV_LL_MAX 3
 kv_status kv_log_likelihoods(kv_context *ctx, const float *d_data, const float *const *d_vols, int n, double *out);
 
@@ -194,7 +196,7 @@ kv_status kv_count_pairs(kv_context *ctx, int mode, int64_t *fp_pairs, int64_t *
 
 /* ---- batched reconstructions (no reference counterpart) ------------------
  * Many reconstructions of uneven volume and projection-count sizes share one
- * persistent forward launch and one persistent backprojection launch per
+ * forward launch and one backprojection launch per
  * iteration (fused MLEM in mode R -- the reference's recons::MLEM -- or mode A,
  * x <- x/s * A^T(data/Ax); the per-reconstruction result is bit-identical to
  * kv_mlem_iteration on its own); the iterations can be captured once into a
@@ -355,7 +357,7 @@ typedef struct kv_accel_schedule {
 kv_status kv_mlem_accelerated(kv_context *ctx, float *d_vol, const float *d_data, const kv_accel_schedule *schedule,
                               const float *d_params, float scale, int *kept);
 /* The same schedule on every reconstruction of a mode-A batch: the MLEM
- * iterations of all reconstructions run as the batch's persistent launches;
+ * iterations of all reconstructions run as the batch's shared launches;
  * each reconstruction's jumps and gates run through its batch context.
  * Volumes start from the batch's current contents; kept[i] (optional) per
  * reconstruction.  Each result is bit-identical to kv_mlem_accelerated on

@@ -467,7 +467,7 @@ def _geometry_struct(g: Geometry, keep: list) -> _KvGeometry:
 
 class Batch:
     """A kv_batch: many mode-R MLEM reconstructions of uneven sizes advanced
-    together by persistent forward/backprojection launches, optionally
+    together by shared forward/backprojection launches, optionally
     replayed from a captured hipGraph.  Host arrays in and out; every call is
     synchronous."""
 

@@ -1201,8 +1201,8 @@ __global__ __launch_bounds__(64) void seg_a_kernel(KvGeom g, KvSeg *__restrict__
 // A step of walk_r takes 32.5 vector instructions; a segment, 1.25 steps on
 // average, takes 18 here and one row load instead of gathers.  Forward pass of
 // 1024x1024x64 / 25 views of 2048^2 6.45 -> 4.43 ms, 512x512x48 / 21 views of
-// 1024^2 0.79 -> 0.55, 256x256x32 / 15 views of 512^2 0.087 -> 0.073, 128x128x32
-// / 15 views of 256^2 0.026 -> 0.025 (bound by the latency of a wavefront).
+// 1024^2 0.79 -> 0.55, 256x256x32 / 15 views of 512^2 0.087 -> 0.071, 128x128x32
+// / 15 views of 256^2 0.026 -> 0.022 (bound by the latency of a wavefront).
 
 typedef const __attribute__((address_space(4))) KvSegHeadR KvSegHeadRC;
 typedef const __attribute__((address_space(4))) KvSegR KvSegRC;

@@ -205,7 +205,7 @@ class BatchedRun:
 def batched_gated_mlem(batch, iters: int, params: Optional[np.ndarray] = None, scale: float = DEFAULT_SCALE,
                        every: int = 2, first: int = 5, patience: Optional[int] = 2, references=None) -> BatchedRun:
     """MLEM-A on every reconstruction of a mode-A batch (kv_batch: one
-    persistent forward and one persistent backprojection launch per
+    forward and one backprojection launch per
     iteration, replayed from a captured hipGraph), with a CNN candidate per
     reconstruction after iteration `first` and every `every` iterations after
     it, kept only if that reconstruction's Poisson log-likelihood does not
@@ -382,7 +382,7 @@ def batched_accelerated_mlem(batch, schedule=None, params: Optional[np.ndarray] 
     """The two-stretch jump schedule on every reconstruction of a mode-A batch
     (as accelerated_mlem, reconstruction by reconstruction): the MLEM
     iterations of all reconstructions (estimates and probes alike) run as
-    one persistent forward and one persistent backprojection launch per
+    one forward and one backprojection launch per
     iteration (captured hipGraph); each reconstruction records its own
     stretches straight from the batch's volume buffers and makes its own
     jumps and gated final steps through its batch context.  Volumes start
