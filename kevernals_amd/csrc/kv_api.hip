@@ -126,6 +126,27 @@ bool bp_posz_ok(const kv_geometry &q)
     return true;
 }
 
+// Largest distance, in detector columns, between the shadows of a voxel's x
+// edge on neighbouring z planes (the scale T = (det - src) / (plane - src) is
+// steepest at an outer slice, the shadows farthest apart at an outer x
+// plane); 0 where some plane is not in front of the source.
+float bp_shift(const kv_geometry &q)
+{
+    double most = 1e-6;
+    for (int p = 0; p < q.np; ++p) {
+        const double sx = q.src[3 * p] / (double)q.sx, sz = q.src[3 * p + 2] / (double)q.sz,
+                     dz = q.det[3 * p + 2] / (double)q.sz - sz, hx = q.nx / 2.0, hz = q.nz / 2.0;
+        auto scale = [&](double k) { return dz / ((k - hz) - sz); };
+        for (int k = 0; k < q.nz; k += std::max(1, q.nz - 1)) {
+            const double t0 = scale(k), t1 = scale(k + 1);
+            if (!(t0 > 0.0 && t1 > 0.0 && t0 < 1e6 && t1 < 1e6))
+                return 0.f;
+            most = std::max(most, (hx + std::fabs(sx)) * std::fabs(t1 - t0) * (q.sx / (double)q.pu));
+        }
+    }
+    return most < 1e6 ? (float)most : 0.f;
+}
+
 // Rounding, in voxels, of an x plane's position relative to the source s in
 // the mode-R walk against exact arithmetic: the run's (-h - s) + k, and h + s
 // of the midpoint (evaluated here, plus half an ulp where the sum with k need
@@ -515,6 +536,7 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     g.rc = ctx->d_rc;
     g.walk_fast = walk_fast_ok(q) ? 1 : 0;
     g.bp_posz = bp_posz_ok(q) ? 1 : 0;
+    g.bp_shift = bp_shift(q);
     // Segment lists of the detector rows.  They are an option: without them
     // (too large, or no memory left) the rays are walked voxel by voxel.
     g.seg_a = nullptr;

@@ -301,11 +301,17 @@ __global__ void yz_kernel(KvGeom g, KvTables t)
 }
 
 // LDS of one brick: the x-table bands and the per-voxel running sums.
-template <int ZT>
+// Running sums per voxel: (value, weight), mode A's without the weight.
+template <int MODE, int EP>
+constexpr int bp_sums()
+{
+    return MODE == KV_MODE_R || EP == KV_EP_COUNT ? 2 : 1;
+}
+template <int ZT, int NS>
 struct BpShared {
     float xb[(TX + 1) * XBS];
     int xbase[TX + 1];
-    float accs[ZT][2][256];  // (value, weight) per slice of the brick (mode A: value only)
+    float accs[ZT][NS][256];  // (value, weight) per slice of the brick (mode A: value only)
 };
 
 // Read-only device memory seen through the constant address space: loads at
@@ -383,9 +389,9 @@ __device__ __forceinline__ int cvt_flr(float x)
 template <int MODE, int EP, int ZT, bool UNIT, bool FW>
 __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, const float *__restrict__ proj,
                                          float *__restrict__ vol, const float *__restrict__ sens, int bxi, int byi,
-                                         int bzi, int zt, BpShared<ZT> &sm)
+                                         int bzi, int zt, BpShared<ZT, bp_sums<MODE, EP>()> &sm)
 {
-    constexpr bool WSUM = MODE == KV_MODE_R || EP == KV_EP_COUNT;
+    constexpr bool WSUM = bp_sums<MODE, EP>() == 2;
     float *xb = sm.xb;
     int *xbase = sm.xbase;
     auto &accs = sm.accs;
@@ -411,7 +417,8 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
     const float nuf = (float)g.nu;
 
     for (int i = 0; i < ZT; ++i)
-        accs[i][0][tid] = accs[i][1][tid] = 0.f;
+        for (int k = 0; k < bp_sums<MODE, EP>(); ++k)
+            accs[i][k][tid] = 0.f;
 
     for (int p = 0; p < g.np; ++p) {
         // Per-view terms, uniform over the workgroup and evaluated once per
@@ -672,7 +679,7 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                 return;
             // one running sum per voxel across all views, as the reference
             // accumulates (Projector.cu:727-728)
-            float a = accs[zi][0][tid], wsm = WSUM ? accs[zi][1][tid] : 0.f;
+            float a = accs[zi][0][tid], wsm = WSUM ? accs[zi][WSUM ? 1 : 0][tid] : 0.f;
             const int ncol = hxw - lx + 1;
             // lx - xb >= 0 and hxw - xb < XBW for both planes' bands, as two
             // unsigned compares (meaningful for the ncol <= 4 it is used with)
@@ -749,7 +756,7 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
             }
             accs[zi][0][tid] = a;
             if (WSUM)
-                accs[zi][1][tid] = wsm;
+                accs[zi][WSUM ? 1 : 0][tid] = wsm;
         };
         // The brick's slices of one view, `slice` for each.  Everything a
         // slice needs from the tables is one 16-word scalar load, issued a
@@ -811,11 +818,11 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
                     A2[c] = xl1[lx + c];
                     L2[c] = MODE == KV_MODE_A && UNIT ? lx2[lx + c] : 0.f;
                 }
-                float a = accs[zi][0][tid], wsm = WSUM ? accs[zi][1][tid] : 0.f;
+                float a = accs[zi][0][tid], wsm = WSUM ? accs[zi][WSUM ? 1 : 0][tid] : 0.f;
                 reduce(nc_tag, E, lx, A1, A2, L2, a, wsm);
                 accs[zi][0][tid] = a;
                 if (WSUM)
-                    accs[zi][1][tid] = wsm;
+                    accs[zi][WSUM ? 1 : 0][tid] = wsm;
             });
         };
         if (nc == 2)
@@ -831,7 +838,7 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
         return;
     for (int zi = 0; zi < nzt; ++zi) {
         const size_t o = ((size_t)(z0 + zi) * g.ny + y) * g.nx + x;
-        const float a = accs[zi][0][tid], wsm = accs[zi][1][tid];
+        const float a = accs[zi][0][tid], wsm = accs[zi][WSUM ? 1 : 0][tid];
         if (EP == KV_EP_COUNT) {
             vol[o] = wsm;
         } else if (MODE == KV_MODE_R) {
@@ -854,6 +861,7 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
 }
 
 constexpr int kZT = 8;
+constexpr int kDeepZT = 16;  // mode A, one sum per voxel: the same LDS
 
 // out[p][v][u] = proj[p][v][u] * sqrt((lx2[p][u] + ly2[p][v]) + lz2[p]): each
 // ray's length factor, applied once per pixel.  The mode-A backprojector's
@@ -879,7 +887,7 @@ template <int MODE, int EP, int ZT, bool UNIT, bool FW>
 __global__ __launch_bounds__(256, 6) void bp_tiled_kernel(KvGeom g, KvTables t, const float *__restrict__ proj,
                                                        float *__restrict__ vol, const float *__restrict__ sens, int zt)
 {
-    __shared__ BpShared<ZT> sm;
+    __shared__ BpShared<ZT, bp_sums<MODE, EP>()> sm;
     bp_brick<MODE, EP, ZT, UNIT, FW>(g, t, proj, vol, sens, blockIdx.x, blockIdx.y, blockIdx.z, zt, sm);
 }
 
@@ -892,7 +900,7 @@ template <int MODE, bool FW>
 __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
                                                           long long total, int iteration)
 {
-    __shared__ BpShared<kZT> sm;
+    __shared__ BpShared<kZT, bp_sums<MODE, KV_EP_MLEM>()> sm;
     for (long long item = blockIdx.x; item < total; item += gridDim.x) {
         // the last descriptor whose items begin at or before this one (by
         // halves: each step waits for a load)
@@ -922,11 +930,21 @@ __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__res
 // 128x128x32 voxels, 15 views 60 -> 37 us (2 slices; 1: 53); 256x256x32, 15
 // views 97 -> 85 (6; 5, just past one round: 101); 163x181x54, 13 views 83 ->
 // 69 (5); 561x117x34, 25 views 122 -> 111 (7; 6: 163).
-int brick_depth(const KvGeom &g)
+// Mode A's larger volumes take up to 16 slices where the bands hold their
+// shadows (KvGeom::bp_shift, 13 columns over a brick), which halves the waits:
+// 512x512x48, 21 views 0.65 -> 0.57 ms; 333x287x45, 13 views 172 -> 154 us (one
+// round instead of 1.7); with wider shifts the outer bricks read the global
+// table (1024x1024x64, 25 views: 4.60 ms at 8 slices, 4.90 at 12, 7.03 at 16).
+int brick_depth(const KvGeom &g, int deepest)
 {
     constexpr int64_t kSlots = 256 * 6;  // CUs x the launch bounds' workgroups
     const int64_t tiles = (int64_t)((g.nx + TX - 1) / TX) * ((g.ny + TY - 1) / TY);
-    const int64_t least = (g.nz + kZT - 1) / kZT, most = (g.nz + 1) / 2;
+    int64_t least = (g.nz + kZT - 1) / kZT;
+    const int64_t most = (g.nz + 1) / 2;
+    if (tiles * least > kSlots && g.bp_shift > 0.f) {
+        const int depth = (int)std::min<float>((float)deepest, std::max((float)kZT, 13.25f / g.bp_shift));
+        least = (g.nz + depth - 1) / depth;
+    }
     const int64_t slabs = std::max(least, std::min(most, kSlots / tiles));
     return (int)((g.nz + slabs - 1) / slabs);
 }
@@ -935,12 +953,13 @@ template <int MODE, int EP, bool UNIT>
 hipError_t launch_tiled(const KvGeom &g, const KvTables &t, const float *proj, float *vol, const float *sens,
                         hipStream_t s)
 {
-    const int zt = brick_depth(g);
+    constexpr int ZT = MODE == KV_MODE_A && EP != KV_EP_COUNT && !UNIT ? kDeepZT : kZT;
+    const int zt = brick_depth(g, ZT);
     const dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + zt - 1) / zt), block(256);
     if (MODE == KV_MODE_R && (EP == KV_EP_MLEM || EP == KV_EP_SART || EP == KV_EP_PLAIN) && g.bp_posz)
-        bp_tiled_kernel<MODE, EP, kZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
+        bp_tiled_kernel<MODE, EP, ZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     else
-        bp_tiled_kernel<MODE, EP, kZT, UNIT, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
+        bp_tiled_kernel<MODE, EP, ZT, UNIT, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     return hipGetLastError();
 }
 

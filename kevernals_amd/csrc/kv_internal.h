@@ -54,6 +54,7 @@ struct KvGeom {
     // (rc[KV_RC*p + 11, 12]), and the other columns together
     int row_cols, edge_cols;
     int walk_fast;  // forward walk may use end thresholds and 24-bit indices (see kv_fp.hip)
+    float bp_shift; // largest shift of a voxel edge's shadow over one slice, in detector columns (0: unbounded)
     int bp_posz;    // every view's z planes at alpha >= 1e-6: clamped backprojection weights (see kv_bp.hip)
 };
 

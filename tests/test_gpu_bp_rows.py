@@ -35,6 +35,9 @@ CASES = {
     # the first voxel's shadow begins left of the detector
     "left": ((40, 10, 3), (0.4, 1.5, 1.0), (60, 120), (0.4, 0.24), 3, 1.0),
     "left_far": ((40, 10, 9), (0.4, 1.5, 1.0), (57, 120), (0.4, 0.24), 3, 1.0),
+    # mode A's deep bricks: a tall and a wide brick grid of more than one round
+    "deep": ((333, 287, 33), (0.25, 0.25, 0.6), (400, 380), (0.35, 0.35), 2, 1.0),
+    "deep_wide": ((450, 230, 37), (0.25, 0.25, 1.2), (500, 300), (0.4, 0.4), 2, 1.0),
     # detector smaller than the volume's shadow, and off to one side
     "cut": ((96, 64, 9), (0.5, 0.5, 1.0), (61, 37), (0.4, 0.4), 3, 1.5),
     "side": ((96, 64, 9), (0.5, 0.5, 1.0), (61, 37), (0.4, 0.4), 3, 1.5),
