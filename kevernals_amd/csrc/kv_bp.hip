@@ -920,33 +920,47 @@ __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__res
     }
 }
 
-// Slices per brick.  A workgroup's time is a wait of some 1.7 us per view (the
-// bands, the view's constants and the first detector rows come from memory)
-// and 0.3 to 0.6 us per slice and view, little more with six workgroups on a
-// CU than with one: what counts is to have as many as fit at once, and no
-// second round of a few.  So a volume that fits the chip in one round is cut
-// into as many slabs as keep it there, down to two slices, all of one depth;
-// a larger one into the deepest bricks.  Mode R at 8 slices and as chosen:
-// 128x128x32 voxels, 15 views 60 -> 37 us (2 slices; 1: 53); 256x256x32, 15
-// views 97 -> 85 (6; 5, just past one round: 101); 163x181x54, 13 views 83 ->
-// 69 (5); 561x117x34, 25 views 122 -> 111 (7; 6: 163).
-// Mode A's larger volumes take up to 16 slices where the bands hold their
-// shadows (KvGeom::bp_shift, 13 columns over a brick), which halves the waits:
-// 512x512x48, 21 views 0.65 -> 0.57 ms; 333x287x45, 13 views 172 -> 154 us (one
-// round instead of 1.7); with wider shifts the outer bricks read the global
-// table (1024x1024x64, 25 views: 4.60 ms at 8 slices, 4.90 at 12, 7.03 at 16).
+// Slices per brick, the depth of least time by what was measured: per view a
+// workgroup waits some 1.7 us (the bands, the view's constants and the first
+// detector rows come from memory) and takes 0.22 us + 0.075 us per workgroup
+// of its CU for each slice; bricks start in rounds of all that fit the chip,
+// dispatched to the emptiest CU first, and the last round is as long as its
+// own occupancy makes it.  So a round of a few workgroups costs nearly a whole
+// one, and a volume that fits in one round is best cut into as many slabs as
+// keep it there.  Measured (8 slices and as chosen): 128x128x32 voxels, 15
+// views 60 -> 37 us (2 slices); 256x256x32, 15 views 97 -> 85 (6; 5, just past
+// one round: 101); 163x181x54, 13 views 83 -> 69 (5); 561x117x34, 25 views
+// 122 -> 111 (7; 6: 163).  Mode A, one sum per voxel, has the LDS for 16
+// slices, used as far as the bands hold their shadows (KvGeom::bp_shift, 13
+// columns over a brick): 512x512x48, 21 views 0.65 -> 0.57 ms (16);
+// 333x287x45, 13 views 172 -> 154 us (15, one round; 12: 195); with wider
+// shifts the outer bricks read the global table (1024x1024x64, 25 views: 4.60
+// ms at 8 slices, 4.90 at 12, 7.03 at 16).
 int brick_depth(const KvGeom &g, int deepest)
 {
     constexpr int64_t kSlots = 256 * 6;  // CUs x the launch bounds' workgroups
     const int64_t tiles = (int64_t)((g.nx + TX - 1) / TX) * ((g.ny + TY - 1) / TY);
-    int64_t least = (g.nz + kZT - 1) / kZT;
-    const int64_t most = (g.nz + 1) / 2;
-    if (tiles * least > kSlots && g.bp_shift > 0.f) {
-        const int depth = (int)std::min<float>((float)deepest, std::max((float)kZT, 13.25f / g.bp_shift));
-        least = (g.nz + depth - 1) / depth;
+    if (deepest > kZT)
+        deepest = g.bp_shift > 0.f
+                      ? (int)std::min<float>((float)deepest, std::max((float)kZT, 13.25f / g.bp_shift))
+                      : kZT;
+    int best = 1;
+    float least = kInf;
+    for (int zt = std::min(deepest, g.nz); zt >= std::min(2, g.nz); --zt) {
+        const int slabs = (g.nz + zt - 1) / zt;
+        if (zt > (g.nz + slabs - 1) / slabs)
+            continue;  // the same number of slabs, unevenly
+        auto round_time = [&](int64_t n) {
+            return n ? 1.7f + (float)zt * (0.22f + 0.075f * (float)((n + 255) / 256)) : 0.f;
+        };
+        const int64_t n = tiles * slabs;
+        const float time = (float)(n / kSlots) * round_time(kSlots) + round_time(n % kSlots);
+        if (time < least) {
+            least = time;
+            best = zt;
+        }
     }
-    const int64_t slabs = std::max(least, std::min(most, kSlots / tiles));
-    return (int)((g.nz + slabs - 1) / slabs);
+    return best;
 }
 
 template <int MODE, int EP, bool UNIT>
