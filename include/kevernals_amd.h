@@ -78,7 +78,8 @@ const char *kv_last_error(void);
 const char *kv_version(void);
 
 /* Geometry -> kernel arguments (Projector.cu:876-940).  Copies the per-view
- * arrays to the device and builds the per-view crossing tables. */
+ * arrays to the device.  The crossing tables and the forward passes' segment
+ * lists of a mode are built by the first calls that need them. */
 kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom);
 
 /* ---- device memory helpers (for hosts without their own allocator) ----- */
@@ -169,8 +170,8 @@ kv_status kv_log_likelihood(kv_context *ctx, const float *d_data, const float *d
  * bit-identical to a kv_log_likelihood call) with one ray walk for all of
  * them: the likelihood gates compare up to three candidates.  Uses two more
  * projection-sized buffers of the context and, for n >= 2 on a geometry
- * without segment lists (which are made unless they would take over 1 GiB or
- * memory is short), a buffer of 16 bytes per voxel into which the volumes are
+ * without segment lists (which the first forward pass of the mode makes unless
+ * they would take over 1 GiB or memory is short), a buffer of 16 bytes per voxel into which the volumes are
  * interleaved (all allocated on first use and kept with the context).
  * Synchronous. */
 #define KV_LL_MAX 3

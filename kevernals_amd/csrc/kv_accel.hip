@@ -269,15 +269,15 @@ kv_status accel_alloc(kv_context *ctx, const kv_accel_schedule *s, bool cnn, Acc
     st.na = s->first - s->start + 1;
     st.nslots = st.na + s->second + 1;
     st.vox_bytes = (size_t)kv_nvox(g) * 4;
-    if (hipMalloc(&st.slots.p, st.vox_bytes * st.nslots) != hipSuccess ||
-        hipMalloc(&st.cands.p, st.vox_bytes * 2) != hipSuccess) {
+    if (kv_internal_alloc(ctx, &st.slots.p, st.vox_bytes * st.nslots) ||
+        kv_internal_alloc(ctx, &st.cands.p, st.vox_bytes * 2)) {
         kv_set_error("accelerated MLEM: cannot allocate %d volumes", st.nslots + 2);
         return KV_ERR_NOMEM;
     }
     if (cnn) {
         if (kv_status e = kv_cnn_workspace_size(g.nx, g.ny, g.nz, 0, &st.work_bytes))
             return e;
-        if (hipMalloc(&st.work.p, st.work_bytes) != hipSuccess) {
+        if (kv_internal_alloc(ctx, &st.work.p, st.work_bytes)) {
             kv_set_error("accelerated MLEM: cannot allocate the CNN workspace");
             return KV_ERR_NOMEM;
         }

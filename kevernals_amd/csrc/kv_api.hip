@@ -46,10 +46,22 @@ kv_status dev_alloc(void **p, size_t bytes)
     const hipError_t e = hipMalloc(p, bytes);
     if (e != hipSuccess) {
         *p = nullptr;
+        (void)hipGetLastError();  // not the next launch's
         kv_set_error("hipMalloc(%zu bytes) failed: %s", bytes, hipGetErrorString(e));
         return e == hipErrorOutOfMemory ? KV_ERR_NOMEM : KV_ERR_DEVICE;
     }
     return KV_OK;
+}
+
+// Memory that a call cannot do without: the context's segment lists, which
+// are an option, make room for it.
+kv_status ctx_alloc(kv_context *ctx, void **p, size_t bytes)
+{
+    kv_status st = dev_alloc(p, bytes);
+    if (st == KV_ERR_NOMEM && !ctx->lists_held && (ctx->d_seg_a || ctx->d_seg_r) &&
+        (st = kv_internal_drop_lists(ctx)) == KV_OK)
+        st = dev_alloc(p, bytes);
+    return st;
 }
 
 // Grows the context's reduction buffer to at least n doubles.  The capacity
@@ -62,7 +74,7 @@ kv_status ensure_red(kv_context *ctx, size_t n)
         return KV_OK;
     free_dev(ctx->d_red);
     ctx->red_cap = 0;
-    if (kv_status st = dev_alloc((void **)&ctx->d_red, n * sizeof(double)))
+    if (kv_status st = ctx_alloc(ctx, (void **)&ctx->d_red, n * sizeof(double)))
         return st;
     ctx->red_cap = n;
     return KV_OK;
@@ -237,11 +249,13 @@ bool row_r_ok(const kv_geometry &q, float &delta)
     return true;
 }
 
-// Entries per list of KvGeom::seg_a, or 0 if the lists would take more than
-// KV_SEG_MAX_BYTES.  A ray crosses at most nz + 1 z planes and the y planes
-// between its entry into the volume and its exit, which lie within the z
-// faces' crossings; the margins cover FP32 rounding in the list's builder.
-int seg_stride(const kv_geometry &q)
+// Entries per list of KvGeom::seg_a and seg_r.  A ray crosses at most nz + 1 z
+// planes and the y planes between its entry into the volume and its exit,
+// which lie within the z faces' crossings.  The lists' builders evaluate the
+// crossings in FP32, each within 4 ulps, and count values that differ: at
+// most 8 more than in exact arithmetic, besides the first and last partial
+// segment, for which the margins leave 17.
+int64_t seg_stride(const kv_geometry &q)
 {
     int most = 0;
     for (int p = 0; p < q.np; ++p) {
@@ -259,9 +273,7 @@ int seg_stride(const kv_geometry &q)
             most = std::max(most, y < q.ny ? (int)y : q.ny);
         }
     }
-    const int64_t n = (int64_t)std::min(most + 8, q.ny + 2) + q.nz + 8 + KV_SEG_PAD;
-    const double bytes = (double)n * q.np * q.nv * sizeof(KvSegR);
-    return bytes <= (double)KV_SEG_MAX_BYTES ? (int)n : 0;
+    return (int64_t)std::min(most + 8, q.ny + 2) + q.nz + 8 + KV_SEG_PAD;
 }
 
 // KvGeom's rc[KV_RC*p + 11, 12], row_cols and edge_cols: per view the first
@@ -310,6 +322,7 @@ kv_status check_mode(int mode)
 kv_status ensure_tables(kv_context *ctx, int mode)
 {
     const KvGeom &g = ctx->g;
+    auto alloc = [&](float **p, size_t bytes) { return ctx_alloc(ctx, (void **)p, bytes); };
     const size_t nxe = (size_t)g.np * g.nu * (g.nx + 1), nye = (size_t)g.np * g.nv * (g.ny + 1),
                  nze = (size_t)g.np * (g.nz + 1), nyz = ((size_t)g.np * g.nz * g.ny + 1) * KV_YZ;
     if (mode == KV_MODE_R) {
@@ -317,9 +330,8 @@ kv_status ensure_tables(kv_context *ctx, int mode)
             return KV_OK;
         KvTables &t = ctx->tab_r;
         kv_status st;
-        if ((st = dev_alloc((void **)&t.x, nxe * 4)) || (st = dev_alloc((void **)&t.y, nye * 4 + 16)) ||
-            (st = dev_alloc((void **)&t.z, nze * 4)) || (st = dev_alloc((void **)&t.zs, nze * KV_ZS * 4)) ||
-            (st = dev_alloc((void **)&t.yz, nyz * 4))) {
+        if ((st = alloc(&t.x, nxe * 4)) || (st = alloc(&t.y, nye * 4 + 16)) || (st = alloc(&t.z, nze * 4)) ||
+            (st = alloc(&t.zs, nze * KV_ZS * 4)) || (st = alloc(&t.yz, nyz * 4))) {
             free_tables(t);
             return st;
         }
@@ -331,11 +343,10 @@ kv_status ensure_tables(kv_context *ctx, int mode)
         return KV_OK;
     KvTables &t = ctx->tab_a;
     kv_status st;
-    if ((st = dev_alloc((void **)&t.x, nxe * 4)) || (st = dev_alloc((void **)&t.y, nye * 4 + 16)) ||
-        (st = dev_alloc((void **)&t.z, nze * 4)) || (st = dev_alloc((void **)&t.lx2, (size_t)g.np * g.nu * 4)) ||
-        (st = dev_alloc((void **)&t.ly2, (size_t)g.np * g.nv * 4)) ||
-        (st = dev_alloc((void **)&t.lz2, (size_t)g.np * 4)) || (st = dev_alloc((void **)&t.zs, nze * KV_ZS * 4)) ||
-        (st = dev_alloc((void **)&t.yz, nyz * 4))) {
+    if ((st = alloc(&t.x, nxe * 4)) || (st = alloc(&t.y, nye * 4 + 16)) || (st = alloc(&t.z, nze * 4)) ||
+        (st = alloc(&t.lx2, (size_t)g.np * g.nu * 4)) || (st = alloc(&t.ly2, (size_t)g.np * g.nv * 4)) ||
+        (st = alloc(&t.lz2, (size_t)g.np * 4)) || (st = alloc(&t.zs, nze * KV_ZS * 4)) ||
+        (st = alloc(&t.yz, nyz * 4))) {
         free_tables(t);
         return st;
     }
@@ -351,18 +362,25 @@ kv_status ensure_sens(kv_context *ctx)
     kv_status st = ensure_tables(ctx, KV_MODE_A);
     if (st)
         return st;
-    if (!ctx->d_sens && (st = dev_alloc((void **)&ctx->d_sens, (size_t)kv_nvox(ctx->g) * 4)))
+    if (!ctx->d_sens && (st = ctx_alloc(ctx, (void **)&ctx->d_sens, (size_t)kv_nvox(ctx->g) * 4)))
         return st;
     KV_TRY_HIP(kv_launch_bp_a(ctx->g, ctx->tab_a, nullptr, ctx->d_sens, KV_EP_PLAIN, nullptr, true, ctx->stream));
     ctx->sens_ok = true;
     return KV_OK;
 }
 
-void release_geometry(kv_context *ctx)
+// Whether work enqueued on s goes into a graph that is being captured (which
+// the null stream's cannot).
+bool capturing(hipStream_t s)
 {
-    free_dev(ctx->d_det);
-    free_dev(ctx->d_src);
-    free_dev(ctx->d_rc);
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &c) != hipSuccess)
+        (void)hipGetLastError();
+    return c != hipStreamCaptureStatusNone;
+}
+
+void free_lists(kv_context *ctx)
+{
     free_dev(ctx->d_seg_a);
     free_dev(ctx->d_seg_a_head);
     free_dev(ctx->d_seg_r);
@@ -371,6 +389,61 @@ void release_geometry(kv_context *ctx)
     ctx->g.seg_a_head = nullptr;
     ctx->g.seg_r = nullptr;
     ctx->g.seg_r_head = nullptr;
+}
+
+// Builds the segment lists of a mode on its first forward pass.  They are an
+// option: without them (none for this geometry, or no memory to spare) the
+// rays are walked voxel by voxel, with the same result.  The call waits for
+// the lists, so that they are complete whatever stream reads them later.  A
+// first pass under graph capture goes without, and leaves them to a later
+// call: the graph would hold the building.
+kv_status ensure_lists(kv_context *ctx, int mode)
+{
+    KvGeom &g = ctx->g;
+    const bool a = mode == KV_MODE_A, graph = capturing(ctx->stream);
+    if (ctx->lists_ok[mode] && !graph) {
+        ctx->lists_ok[mode] = false;
+        const size_t rows = (size_t)g.np * g.nv, n = rows * (size_t)g.seg_stride;
+        const size_t bytes = a ? n * sizeof(KvSeg) + rows * sizeof(KvSegHead)
+                               : n * sizeof(KvSegR) + rows * sizeof(KvSegHeadR);
+        size_t avail = 0, total = 0;
+        auto alloc = [](auto *&p, size_t k) { return hipMalloc((void **)&p, k * sizeof(*p)) == hipSuccess; };
+        if (hipMemGetInfo(&avail, &total) != hipSuccess || avail < bytes + KV_SEG_SPARE_BYTES ||
+            !(a ? alloc(ctx->d_seg_a, n) && alloc(ctx->d_seg_a_head, rows)
+                : alloc(ctx->d_seg_r, n) && alloc(ctx->d_seg_r_head, rows))) {
+            (void)hipGetLastError();  // the failed call's
+            if (a) {
+                free_dev(ctx->d_seg_a);
+                free_dev(ctx->d_seg_a_head);
+            } else {
+                free_dev(ctx->d_seg_r);
+                free_dev(ctx->d_seg_r_head);
+            }
+            return KV_OK;
+        }
+        KV_TRY_HIP(a ? kv_launch_seg_a(g, ctx->d_seg_a, ctx->d_seg_a_head, ctx->stream)
+                     : kv_launch_seg_r(g, ctx->d_seg_r, ctx->d_seg_r_head, ctx->stream));
+        KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
+        if (a) {
+            g.seg_a = ctx->d_seg_a;
+            g.seg_a_head = ctx->d_seg_a_head;
+        } else {
+            g.seg_r = ctx->d_seg_r;
+            g.seg_r_head = ctx->d_seg_r_head;
+        }
+    }
+    if (graph && (a ? g.seg_a != nullptr : g.seg_r != nullptr))
+        ctx->lists_held = true;  // the graph keeps their addresses
+    return KV_OK;
+}
+
+void release_geometry(kv_context *ctx)
+{
+    free_dev(ctx->d_det);
+    free_dev(ctx->d_src);
+    free_dev(ctx->d_rc);
+    free_lists(ctx);
+    ctx->lists_ok[0] = ctx->lists_ok[1] = ctx->lists_held = false;
     free_tables(ctx->tab_r);
     free_tables(ctx->tab_a);
     free_dev(ctx->d_ratio);
@@ -396,6 +469,23 @@ bool almost_equal_relative(float a, float b)
 
 kv_status kv_internal_ensure_tables(kv_context *ctx, int mode) { return ensure_tables(ctx, mode); }
 kv_status kv_internal_ensure_sens(kv_context *ctx) { return ensure_sens(ctx); }
+
+kv_status kv_internal_alloc(kv_context *ctx, void **p, size_t bytes) { return ctx_alloc(ctx, p, bytes); }
+
+kv_status kv_internal_hold_lists(kv_context *ctx, int mode)
+{
+    const kv_status st = ensure_lists(ctx, mode);
+    ctx->lists_held = true;
+    return st;
+}
+
+kv_status kv_internal_drop_lists(kv_context *ctx)
+{
+    KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
+    free_lists(ctx);
+    ctx->lists_ok[0] = ctx->lists_ok[1] = false;
+    return KV_OK;
+}
 
 void kv_set_error(const char *fmt, ...)
 {
@@ -511,10 +601,10 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
     release_geometry(ctx);
     kv_status st;
-    if ((st = dev_alloc((void **)&ctx->d_det, (size_t)q.np * 12)) ||
-        (st = dev_alloc((void **)&ctx->d_src, (size_t)q.np * 12)) ||
-        (st = dev_alloc((void **)&ctx->d_rc, (size_t)q.np * (KV_RC + 4 * q.nu + 4 * q.nv) * 4)) ||
-        (st = dev_alloc((void **)&ctx->d_ratio, (size_t)nray * 4))) {
+    if ((st = ctx_alloc(ctx, (void **)&ctx->d_det, (size_t)q.np * 12)) ||
+        (st = ctx_alloc(ctx, (void **)&ctx->d_src, (size_t)q.np * 12)) ||
+        (st = ctx_alloc(ctx, (void **)&ctx->d_rc, (size_t)q.np * (KV_RC + 4 * q.nu + 4 * q.nv) * 4)) ||
+        (st = ctx_alloc(ctx, (void **)&ctx->d_ratio, (size_t)nray * 4))) {
         release_geometry(ctx);
         return st;
     }
@@ -537,40 +627,14 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     g.walk_fast = walk_fast_ok(q) ? 1 : 0;
     g.bp_posz = bp_posz_ok(q) ? 1 : 0;
     g.bp_shift = bp_shift(q);
-    // Segment lists of the detector rows.  They are an option: without them
-    // (too large, or no memory left) the rays are walked voxel by voxel.
-    g.seg_a = nullptr;
-    g.seg_a_head = nullptr;
-    g.seg_stride = seg_stride(q);
-    g.seg_r = nullptr;
-    g.seg_r_head = nullptr;
     g.row_cols = row_cols;
     g.edge_cols = edge_cols;
-    const size_t rows = (size_t)q.np * q.nv;
-    auto alloc = [](auto *&p, size_t n) { return hipMalloc((void **)&p, n * sizeof(*p)) == hipSuccess; };
-    if (g.seg_stride > 0) {
-        if (alloc(ctx->d_seg_a, rows * g.seg_stride) && alloc(ctx->d_seg_a_head, rows)) {
-            KV_TRY_HIP(kv_launch_seg_a(g, ctx->d_seg_a, ctx->d_seg_a_head, ctx->stream));
-            g.seg_a = ctx->d_seg_a;
-            g.seg_a_head = ctx->d_seg_a_head;
-        } else {
-            (void)hipGetLastError();  // the failed allocation's
-            free_dev(ctx->d_seg_a);
-            free_dev(ctx->d_seg_a_head);
-        }
-    }
-    if (g.seg_stride > 0 && g.walk_fast && row_cols > 0 && row_r_ok(q, g.seg_delta)) {
-        if (alloc(ctx->d_seg_r, rows * g.seg_stride) && alloc(ctx->d_seg_r_head, rows)) {
-            KV_TRY_HIP(kv_launch_seg_r(g, ctx->d_seg_r, ctx->d_seg_r_head, ctx->stream));
-            g.seg_r = ctx->d_seg_r;
-            g.seg_r_head = ctx->d_seg_r_head;
-        } else {
-            (void)hipGetLastError();
-            free_dev(ctx->d_seg_r);
-            free_dev(ctx->d_seg_r_head);
-        }
-    }
-    KV_TRY_HIP(hipStreamSynchronize(ctx->stream));
+    const int64_t stride = seg_stride(q);
+    const double entries = (double)stride * q.np * q.nv;
+    g.seg_stride = (int)stride;
+    ctx->lists_ok[KV_MODE_A] = entries * sizeof(KvSeg) <= (double)KV_SEG_MAX_BYTES;
+    ctx->lists_ok[KV_MODE_R] = entries * sizeof(KvSegR) <= (double)KV_SEG_MAX_BYTES && g.walk_fast && row_cols > 0 &&
+                               row_r_ok(q, g.seg_delta);
     ctx->has_geom = true;
     return KV_OK;
 }
@@ -583,7 +647,7 @@ kv_status kv_malloc(kv_context *ctx, size_t bytes, void **d_ptr)
         kv_set_error("null output pointer");
         return KV_ERR_INVALID;
     }
-    return dev_alloc(d_ptr, bytes ? bytes : 1);
+    return ctx_alloc(ctx, d_ptr, bytes ? bytes : 1);
 }
 
 kv_status kv_free(kv_context *ctx, void *d_ptr)
@@ -643,6 +707,8 @@ kv_status kv_forward_project(kv_context *ctx, const float *d_vol, float *d_proj,
         kv_set_error("null buffer");
         return KV_ERR_INVALID;
     }
+    if (kv_status st = ensure_lists(ctx, mode))
+        return st;
     if (mode == KV_MODE_R)
         KV_TRY_HIP(kv_launch_fp_r(ctx->g, d_vol, d_proj, KV_EP_PLAIN, nullptr, 0.f, ctx->stream));
     else
@@ -686,6 +752,8 @@ kv_status kv_mlem_forward(kv_context *ctx, const float *d_vol, const float *d_da
     // tables (and the mode-A sensitivity) are built here so that the
     // backward half enqueues a single kernel
     if (kv_status st = (mode == KV_MODE_R) ? ensure_tables(ctx, KV_MODE_R) : ensure_sens(ctx))
+        return st;
+    if (kv_status st = ensure_lists(ctx, mode))
         return st;
     if (mode == KV_MODE_R)
         KV_TRY_HIP(kv_launch_fp_r(ctx->g, d_vol, ctx->d_ratio, KV_EP_MLEM, d_data, relax, ctx->stream));
@@ -737,7 +805,7 @@ kv_status kv_count_pairs(kv_context *ctx, int mode, int64_t *fp_pairs, int64_t *
     if (kv_status st = ensure_red(ctx, (size_t)nb))
         return st;
     float *d_cnt = nullptr;
-    if (kv_status st = dev_alloc((void **)&d_cnt, (size_t)kv_nvox(ctx->g) * 4))
+    if (kv_status st = ctx_alloc(ctx, (void **)&d_cnt, (size_t)kv_nvox(ctx->g) * 4))
         return st;
     std::vector<double> part(nb);
     double sums[2] = {0.0, 0.0};
@@ -780,6 +848,8 @@ kv_status kv_sart_iteration(kv_context *ctx, float *d_vol, const float *d_data, 
         return KV_ERR_INVALID;
     }
     if (kv_status st = ensure_tables(ctx, KV_MODE_R))
+        return st;
+    if (kv_status st = ensure_lists(ctx, KV_MODE_R))
         return st;
     KV_TRY_HIP(kv_launch_fp_r(ctx->g, d_vol, ctx->d_ratio, KV_EP_SART, d_data, relax, ctx->stream));
     KV_TRY_HIP(kv_launch_bp_r(ctx->g, ctx->tab_r, ctx->d_ratio, d_vol, KV_EP_SART, ctx->stream));
@@ -891,7 +961,7 @@ kv_status kv_shift_and_add(kv_context *ctx, const float *d_proj, const float *sr
         return st;
     const KvSaaPlan plan = kv_saa_plan(nplanes, g.np, [&](int k, int p) { return shifts[(size_t)p * nplanes + k]; });
     int32_t *d_shifts = nullptr;
-    if (kv_status st = dev_alloc((void **)&d_shifts, shifts.size() * 4))
+    if (kv_status st = ctx_alloc(ctx, (void **)&d_shifts, shifts.size() * 4))
         return st;
     hipError_t e = hipMemcpyAsync(d_shifts, shifts.data(), shifts.size() * 4, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess)
@@ -964,6 +1034,8 @@ kv_status kv_log_likelihood(kv_context *ctx, const float *d_data, const float *d
     const int nb = 1024;
     if (kv_status st = ensure_red(ctx, (size_t)nb))
         return st;
+    if (kv_status st = ensure_lists(ctx, KV_MODE_A))
+        return st;
     KV_TRY_HIP(kv_launch_fp_a(ctx->g, ctx->tab_a, d_vol, ctx->d_ratio, KV_EP_PLAIN, nullptr, ctx->stream));
     KV_TRY_HIP(kv_launch_loglik(ctx->g, d_data, ctx->d_ratio, ctx->d_red, nb, ctx->stream));
     std::vector<double> part(nb);
@@ -993,13 +1065,15 @@ kv_status kv_log_likelihoods(kv_context *ctx, const float *d_data, const float *
     const int nb = 1024;
     if (kv_status st = ensure_red(ctx, (size_t)nb))
         return st;
+    if (kv_status st = ensure_lists(ctx, KV_MODE_A))
+        return st;
     const size_t nray = (size_t)kv_nray(ctx->g);
     if (n > 1 && !ctx->d_ll) {
-        if (kv_status st = dev_alloc((void **)&ctx->d_ll, (KV_LL_MAX - 1) * nray * sizeof(float)))
+        if (kv_status st = ctx_alloc(ctx, (void **)&ctx->d_ll, (KV_LL_MAX - 1) * nray * sizeof(float)))
             return st;
     }
     if (n > 1 && !ctx->g.seg_a && !ctx->d_pack) {
-        if (kv_status st = dev_alloc((void **)&ctx->d_pack, 4 * (size_t)kv_nvox(ctx->g) * sizeof(float)))
+        if (kv_status st = ctx_alloc(ctx, (void **)&ctx->d_pack, 4 * (size_t)kv_nvox(ctx->g) * sizeof(float)))
             return st;
     }
     float *outs[KV_LL_MAX] = {ctx->d_ratio, ctx->d_ll, ctx->d_ll ? ctx->d_ll + nray : nullptr};
@@ -1045,7 +1119,7 @@ kv_status kv_phantom(kv_context *ctx, float background, const kv_pave *paves, in
                  bsph = (size_t)nspheres * sizeof(kv_sphere);
     const size_t opav = (bpos + 255) & ~(size_t)255, osph = (opav + bpav + 255) & ~(size_t)255;
     char *d_buf = nullptr;
-    if (kv_status st = dev_alloc((void **)&d_buf, osph + bsph + 4))
+    if (kv_status st = ctx_alloc(ctx, (void **)&d_buf, osph + bsph + 4))
         return st;
     hipError_t e = hipMemcpyAsync(d_buf, pos.data(), bpos, hipMemcpyHostToDevice, ctx->stream);
     if (e == hipSuccess && bpav)
@@ -1189,8 +1263,9 @@ kv_status kv_trace_rays(kv_context *ctx, int mode, int nrays, const int32_t *ray
     float *d_w = nullptr;
     kv_status st = KV_OK;
     const size_t slots = (size_t)nrays * cap;
-    if ((st = dev_alloc((void **)&d_rays, (size_t)nrays * 4)) || (st = dev_alloc((void **)&d_counts, (size_t)nrays * 4)) ||
-        (st = dev_alloc((void **)&d_idx, slots * 8)) || (st = dev_alloc((void **)&d_w, slots * 4))) {
+    if ((st = ctx_alloc(ctx, (void **)&d_rays, (size_t)nrays * 4)) ||
+        (st = ctx_alloc(ctx, (void **)&d_counts, (size_t)nrays * 4)) ||
+        (st = ctx_alloc(ctx, (void **)&d_idx, slots * 8)) || (st = ctx_alloc(ctx, (void **)&d_w, slots * 4))) {
         free_dev(d_rays);
         free_dev(d_counts);
         free_dev(d_idx);
@@ -1224,7 +1299,7 @@ static kv_status host_roundtrip(kv_context *ctx, const float *h_in, size_t in_n,
 {
     float *d_in = nullptr, *d_out = nullptr;
     kv_status st;
-    if ((st = dev_alloc((void **)&d_in, in_n * 4)) || (st = dev_alloc((void **)&d_out, out_n * 4))) {
+    if ((st = ctx_alloc(ctx, (void **)&d_in, in_n * 4)) || (st = ctx_alloc(ctx, (void **)&d_out, out_n * 4))) {
         free_dev(d_in);
         free_dev(d_out);
         return st;

@@ -232,6 +232,21 @@ void release(kv_batch *b)
 int kv_internal_batch_size(const kv_batch *b) { return b ? b->n : 0; }
 int kv_internal_batch_mode(const kv_batch *b) { return b ? b->mode : -1; }
 
+kv_status kv_internal_batch_drop_lists(kv_batch *b)
+{
+    KV_TRY_HIP(hipStreamSynchronize(b->stream));
+    for (int i = 0; i < b->n; ++i) {
+        if (kv_status st = kv_internal_drop_lists(b->ctx[(size_t)i]))
+            return st;
+        b->probs[(size_t)i].g = b->ctx[(size_t)i]->g;
+    }
+    layout_items(b);
+    if (b->exec)
+        (void)hipGraphExecDestroy(b->exec);  // captured for other work lists
+    b->exec = nullptr;
+    return KV_OK;
+}
+
 extern "C" {
 
 kv_status kv_batch_create(int device, int n, const kv_geometry *geoms, int mode, kv_batch **out)
@@ -285,7 +300,6 @@ kv_status kv_batch_create(int device, int n, const kv_geometry *geoms, int mode,
             break;
         }
         KvProblem &P = b->probs[(size_t)i];
-        P.g = c->g;
         P.t = mode == KV_MODE_A ? c->tab_a : c->tab_r;
         P.vol = b->vol[(size_t)i];
         P.data = b->data[(size_t)i];
@@ -296,11 +310,17 @@ kv_status kv_batch_create(int device, int n, const kv_geometry *geoms, int mode,
         P.bp_zt = 8;
     }
     if (st == KV_OK) {
-        layout_items(b);
         e = hipMalloc((void **)&b->d_probs, 2 * (size_t)n * sizeof(KvProblem));
         if (e != hipSuccess)
             st = fail_hip(e, "descriptor allocation");
     }
+    // the segment lists, an option, once every reconstruction has what it needs
+    for (int i = 0; i < n && st == KV_OK; ++i) {
+        st = kv_internal_hold_lists(b->ctx[(size_t)i], mode);
+        b->probs[(size_t)i].g = b->ctx[(size_t)i]->g;
+    }
+    if (st == KV_OK)
+        layout_items(b);
     if (st != KV_OK) {
         release(b);
         delete b;

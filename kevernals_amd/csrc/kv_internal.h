@@ -37,9 +37,10 @@ struct KvGeom {
     // and detector row for y.
     const float *rc;
     // Mode-A forward walk of a detector row: the (y, z) segments its rays
-    // share (KvSeg lists of seg_stride entries per view and row, built by
-    // kv_set_geometry), and per list its alpha range and count.  Null when the lists would exceed
-    // KV_SEG_MAX_BYTES: the rays are then walked voxel by voxel.
+    // share (KvSeg lists of seg_stride entries per view and row, built on the
+    // first forward pass), and per list its alpha range and count.  Null before
+    // that, when the lists would exceed KV_SEG_MAX_BYTES, and when memory is
+    // short: the rays are then walked voxel by voxel.
     const struct KvSeg *seg_a;
     const struct KvSegHead *seg_a_head;
     int seg_stride;
@@ -90,7 +91,10 @@ struct KvSegHeadR {
     int empty;         // no ray of the row meets the volume
 };
 constexpr int KV_SEG_PAD = 16;
+// The lists of one mode take at most KV_SEG_MAX_BYTES, and only where they
+// leave KV_SEG_SPARE_BYTES free.
 constexpr size_t KV_SEG_MAX_BYTES = size_t(1) << 30;
+constexpr size_t KV_SEG_SPARE_BYTES = size_t(1) << 30;
 
 // Unsigned division by a divisor fixed for a launch: n / d =
 // (umulhi(n, m) + n) >> l for every n < 2^31, with l = ceil(log2 d) and
@@ -212,6 +216,8 @@ struct kv_context {
     KvSegHead *d_seg_a_head = nullptr;
     KvSegR *d_seg_r = nullptr;  // KvGeom::seg_r
     KvSegHeadR *d_seg_r_head = nullptr;
+    bool lists_ok[2] = {false, false};  // mode's lists not built yet, and worth it for the geometry
+    bool lists_held = false;            // their addresses are kept elsewhere (a batch, a captured graph)
     KvTables tab_r{};
     bool tab_r_ok = false;
     KvTables tab_a{};
@@ -236,6 +242,17 @@ void kv_set_error(const char *fmt, ...);
 kv_status kv_internal_ensure_tables(kv_context *ctx, int mode);
 // Computes the mode-A sensitivity A^T 1 (once).
 kv_status kv_internal_ensure_sens(kv_context *ctx);
+// Device memory that a call cannot do without (hipMalloc): the context's
+// segment lists make room for it, unless they are held.
+kv_status kv_internal_alloc(kv_context *ctx, void **p, size_t bytes);
+// Builds a mode's segment lists where the geometry has them, for a caller
+// that copies KvGeom: the context keeps them as long as its geometry.
+kv_status kv_internal_hold_lists(kv_context *ctx, int mode);
+// Frees the segment lists; the geometry's later passes go without.  Not for
+// a context whose lists are held.
+kv_status kv_internal_drop_lists(kv_context *ctx);
+// The same for every reconstruction of a batch.
+kv_status kv_internal_batch_drop_lists(kv_batch *b);
 
 #define KV_TRY_HIP(expr)                                                                        \
     do {                                                                                        \
