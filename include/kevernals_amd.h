@@ -171,9 +171,9 @@ kv_status kv_log_likelihood(kv_context *ctx, const float *d_data, const float *d
  * them: the likelihood gates compare up to three candidates.  Uses two more
  * projection-sized buffers of the context and, for n >= 2 on a geometry
  * without segment lists (which the first forward pass of the mode makes unless
- * they would take over 1 GiB or memory is short), a buffer of 16 bytes per voxel into which the volumes are
- * interleaved (all allocated on first use and kept with the context).
- * Synchronous. */
+ * they would take over 1 GiB or memory is short), a buffer of 16 bytes per voxel
+ * into which the volumes are interleaved (all allocated on first use and kept
+ * with the context).  Synchronous. */
 #define KV_LL_MAX 3
 kv_status kv_log_likelihoods(kv_context *ctx, const float *d_data, const float *const *d_vols, int n, double *out);
 
@@ -217,8 +217,8 @@ kv_status kv_batch_get_volume(kv_batch *b, int i, float *h_vol);
  * Synchronous. */
 kv_status kv_batch_mlem(kv_batch *b, const int32_t *iters, float relax, int use_graph, float *ms);
 /* Tile shapes of reconstruction i: forward layout 1, 2, 4 or 8 (detector
- * rows per wavefront), backprojection brick depth 4 or 8 slices.  Results do
- * not depend on them. */
+ * rows per wavefront; of effect only on a geometry without segment lists),
+ * backprojection brick depth 4 or 8 slices.  Results do not depend on them. */
 kv_status kv_batch_set_tiles(kv_batch *b, int i, int fp_layout, int bp_slices);
 /* Reconstruction i's context (owned by the batch: do not destroy it; its
  * geometry and tables are those of the batch) and device buffers, for
@@ -229,9 +229,11 @@ kv_status kv_batch_context(kv_batch *b, int i, kv_context **ctx);
 kv_status kv_batch_buffers(kv_batch *b, int i, float **d_vol, float **d_data);
 kv_status kv_batch_get_tiles(kv_batch *b, int i, int *fp_layout, int *bp_slices);
 /* Times the tile shapes per size class (volume voxel count < 16 Mi, < 40 Mi,
- * larger) on this batch and applies the fastest; with a cache file, classes
- * already tuned on this device are read from it instead and new results are
- * written back.  Volumes are restored afterwards. */
+ * larger) on this batch and applies the fastest: brick depths, and forward
+ * layouts where a class has reconstructions without segment lists.  With a
+ * cache file, what is already tuned on this device is read from it instead
+ * and new results are written back (layout 0: none timed).  Volumes are
+ * restored afterwards. */
 kv_status kv_batch_autotune(kv_batch *b, const char *cache_path);
 
 /* ---- learned step: 3D residual CNN (no reference counterpart) ------------

@@ -457,7 +457,8 @@ kv_status kv_batch_autotune(kv_batch *b, const char *cache_path)
     (void)hipGetDeviceProperties(&prop, b->device);
     const std::string dev = prop.gcnArchName[0] ? prop.gcnArchName : "gpu";
     const std::string devkey = dev.substr(0, dev.find(':'));
-    // cached choices: "<device> <class> <layout> <slices> <ms>" per line
+    // cached choices: "<device> <class> <layout> <slices> <ms>" per line, layout
+    // 0 where no reconstruction of the class was walked in tiles of a layout
     int best_l[3] = {0, 0, 0}, best_z[3] = {0, 0, 0};
     float best_ms[3] = {0.f, 0.f, 0.f};
     std::vector<std::string> kept;
@@ -471,7 +472,8 @@ kv_status kv_batch_autotune(kv_batch *b, const char *cache_path)
             float t;
             if (!(ls >> d >> c >> l >> z >> t))
                 continue;
-            if (d == devkey && c >= 0 && c < 3 && (l == 1 || l == 2 || l == 4 || l == 8) && (z == 4 || z == 8)) {
+            if (d == devkey && c >= 0 && c < 3 && (l == 0 || l == 1 || l == 2 || l == 4 || l == 8) &&
+                (z == 4 || z == 8)) {
                 best_l[c] = l;
                 best_z[c] = z;
                 best_ms[c] = t;
@@ -480,12 +482,23 @@ kv_status kv_batch_autotune(kv_batch *b, const char *cache_path)
             }
         }
     }
-    bool present[3] = {false, false, false};
-    for (const auto &P : b->probs)
+    // Row-by-row forward passes have no layout to choose: one that is timed for
+    // them is picked by chance, and others would read it from the file.
+    bool present[3] = {false, false, false}, tiled[3] = {false, false, false};
+    for (const auto &P : b->probs) {
         present[size_class(P)] = true;
-    bool need = false;
-    for (int c = 0; c < 3; ++c)
-        need = need || (present[c] && best_l[c] == 0);
+        tiled[size_class(P)] = tiled[size_class(P)] || P.fp_part == KV_FP_WHOLE;
+    }
+    auto open = [&](int c) { return present[c] && (best_z[c] == 0 || (tiled[c] && best_l[c] == 0)); };
+    auto apply = [&](int c, int l, int z) {
+        for (auto &P : b->probs)
+            if (size_class(P) == c) {
+                if (l && P.fp_part == KV_FP_WHOLE)
+                    P.fp_layout = l;
+                P.bp_zt = z;
+            }
+    };
+    const bool need = open(0) || open(1) || open(2);
     hipError_t e = hipSuccess;
     std::vector<float *> backup((size_t)b->n, nullptr);
     kv_status st = KV_OK;
@@ -497,21 +510,18 @@ kv_status kv_batch_autotune(kv_batch *b, const char *cache_path)
             if (e == hipSuccess)
                 e = hipMemcpyAsync(backup[(size_t)i], b->vol[(size_t)i], bytes, hipMemcpyDeviceToDevice, b->stream);
         }
-        const int layouts[4] = {1, 2, 4, 8}, slices[2] = {4, 8};
+        const std::vector<int> layouts[2] = {{0}, {1, 2, 4, 8}};
+        const int slices[2] = {4, 8};
         std::vector<int32_t> it((size_t)b->n);
         for (int c = 0; c < 3 && e == hipSuccess && st == KV_OK; ++c) {
-            if (!present[c] || best_l[c] != 0)
+            if (!open(c))
                 continue;
             for (int i = 0; i < b->n; ++i)
                 it[(size_t)i] = size_class(b->probs[(size_t)i]) == c ? 1 : 0;
             float best = 1e30f;
-            for (int l : layouts)
+            for (int l : layouts[tiled[c]])
                 for (int z : slices) {
-                    for (auto &P : b->probs)
-                        if (size_class(P) == c) {
-                            P.fp_layout = l;
-                            P.bp_zt = z;
-                        }
+                    apply(c, l, z);
                     layout_items(b);
                     float t = 1e30f;
                     for (int rep = 0; rep < 2 && st == KV_OK; ++rep) {
@@ -541,20 +551,16 @@ kv_status kv_batch_autotune(kv_batch *b, const char *cache_path)
         return st;
     if (e != hipSuccess)
         return fail_hip(e, "autotune");
-    for (auto &P : b->probs) {
-        const int c = size_class(P);
-        if (best_l[c]) {
-            P.fp_layout = best_l[c];
-            P.bp_zt = best_z[c];
-        }
-    }
+    for (int c = 0; c < 3; ++c)
+        if (present[c])
+            apply(c, best_l[c], best_z[c]);
     layout_items(b);
     if (need && cache_path && *cache_path) {
         std::ofstream outf(cache_path);
         for (const auto &l : kept)
             outf << l << "\n";
         for (int c = 0; c < 3; ++c)
-            if (best_l[c])
+            if (best_z[c])
                 outf << devkey << " " << c << " " << best_l[c] << " " << best_z[c] << " " << best_ms[c] << "\n";
     }
     return KV_OK;

@@ -173,3 +173,32 @@ H.fake_budget(have + 1000)
 assert L.kv_back_project(c.handle, buf, buf, A) == 3  # no memory
 assert H.fake_used() == have and ran(forward(c, A), "fp_a_row_kernel")
 """)
+
+
+def test_tuner_leaves_forward_layouts_of_row_by_row_passes(run, tmp_path):
+    """Without a layout to choose none is timed, applied or written down; a
+    batch that needs one times it, whatever the file says of brick depths."""
+    run("""
+path = %r
+gs = [arc(16), arc(20, 100)]
+
+def tuned(b, cache):
+    n = sum("fp_a_batch_kernel" in k for k in launches(L.kv_batch_autotune, b.handle, cache))
+    return n, [b.get_tiles(i) for i in range(len(gs))]
+
+b = K.Batch(gs, mode=A)
+before = [l for l, _ in (b.get_tiles(i) for i in range(len(gs)))]
+n, tiles = tuned(b, path)
+assert n == 2 * 2 and [l for l, _ in tiles] == before, (n, tiles)
+assert [ln.split()[2] for ln in open(path)] == ["0"]
+assert tuned(b, path) == (0, tiles)
+assert batch_drop(b.handle) == 0
+n, tiles = tuned(b, path)
+assert n == 2 * 4 * 2
+(line,) = open(path).readlines()
+assert all((str(l), str(z)) == tuple(line.split()[2:4]) for l, z in tiles) and tiles[0][0] in (1, 2, 4, 8)
+assert tuned(b, path) == (0, tiles)
+b = K.Batch(gs, mode=A)  # with lists: the file's depth, its own layout
+n, again = tuned(b, path)
+assert n == 0 and [l for l, _ in again] == before and [z for _, z in again] == [z for _, z in tiles]
+""" % str(tmp_path / "tiles").encode())
