@@ -970,9 +970,13 @@ hipError_t launch_tiled(const KvGeom &g, const KvTables &t, const float *proj, f
     constexpr int ZT = MODE == KV_MODE_A && EP != KV_EP_COUNT && !UNIT ? kDeepZT : kZT;
     const int zt = brick_depth(g, ZT);
     const dim3 grid((g.nx + TX - 1) / TX, (g.ny + TY - 1) / TY, (g.nz + zt - 1) / zt), block(256);
-    if (MODE == KV_MODE_R && (EP == KV_EP_MLEM || EP == KV_EP_SART || EP == KV_EP_PLAIN) && g.bp_posz)
-        bp_tiled_kernel<MODE, EP, ZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
-    else
+    bool fw = false;
+    if constexpr (MODE == KV_MODE_R && EP != KV_EP_COUNT) {
+        fw = g.bp_posz != 0;
+        if (fw)
+            bp_tiled_kernel<MODE, EP, ZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
+    }
+    if (!fw)
         bp_tiled_kernel<MODE, EP, ZT, UNIT, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     return hipGetLastError();
 }

@@ -33,6 +33,8 @@ size_t fake_used(void) { return used; }
 void fake_capture(int on) { capture = on; }
 const char *fake_log(void) { return log_text; }
 void fake_log_clear(void) { log_text[0] = 0; }
+int fake_kernels(void) { return nfn; }
+const char *fake_kernel(int i) { return fn[i].name; }
 
 /* ---- memory ---- */
 int hipMalloc(void **p, size_t n)

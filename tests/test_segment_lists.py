@@ -202,3 +202,14 @@ b = K.Batch(gs, mode=A)  # with lists: the file's depth, its own layout
 n, again = tuned(b, path)
 assert n == 0 and [l for l, _ in again] == before and [z for _, z in again] == [z for _, z in tiles]
 """ % str(tmp_path / "tiles").encode())
+
+
+def test_backprojectors_without_a_caller_are_not_built(run):
+    """Weights without their test (FW, the last parameter) are mode R's, and
+    not of the pair count, which needs the test."""
+    run("""
+H.fake_kernel.restype = ctypes.c_char_p
+names = [H.fake_kernel(i).decode() for i in range(H.fake_kernels())]
+fw = [n for n in names if "bp_tiled_kernel" in n and "Lb1EEEv" in n]
+assert len(fw) == 3 and all("ILi0ELi%dE" % ep in n for ep, n in enumerate(sorted(fw))), fw
+""")
