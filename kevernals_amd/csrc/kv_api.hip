@@ -159,6 +159,33 @@ float bp_shift(const kv_geometry &q)
     return most < 1e6 ? (float)most : 0.f;
 }
 
+// Whether enough backprojection bricks lie beside the detector rows of views
+// (kv_bp.hip) for looking for them to pay: 12 % of the (view, brick) pairs, as
+// the kernel which looks is up to 4 % slower and the bricks' time goes by the
+// last ones to end.  Of 63 sizes measured those with 5 to 12 % became 3 %
+// slower to 4 % faster, those with more 2 % slower to 4.9 times as fast.
+// Bricks of KV_BP_TY voxel rows and 8 slices: on a plane of scale t, row edge
+// c reaches the detector's lower edge oy at c = sy + (oy - sy) / t.
+bool bp_beside(const kv_geometry &q)
+{
+    double rows = 0.0, all = 0.0;
+    for (int p = 0; p < q.np; ++p) {
+        const double sy = q.src[3 * p + 1] / (double)q.sy, sz = q.src[3 * p + 2] / (double)q.sz,
+                     dz = q.det[3 * p + 2] / (double)q.sz - sz, oy = q.det[3 * p + 1] / (double)q.sy,
+                     ey = oy + q.nv * (double)q.pv / q.sy, hy = q.ny / 2.0;
+        for (int k = 0; k < q.nz; k += 8) {
+            const double t0 = dz / ((k - q.nz / 2.0) - sz), t1 = dz / ((std::min(k + 8, q.nz) - q.nz / 2.0) - sz);
+            all += q.ny;
+            if (!(t0 > 0.0 && t1 > 0.0))
+                continue;
+            const double below = std::min(sy + (oy - sy) / t0, sy + (oy - sy) / t1) + hy - KV_BP_TY,
+                         above = hy - std::max(sy + (ey - sy) / t0, sy + (ey - sy) / t1) - KV_BP_TY;
+            rows += std::min(std::max(below, 0.0) + std::max(above, 0.0), (double)q.ny);
+        }
+    }
+    return rows >= 0.12 * all;
+}
+
 // Rounding, in voxels, of an x plane's position relative to the source s in
 // the mode-R walk against exact arithmetic: the run's (-h - s) + k, and h + s
 // of the midpoint (evaluated here, plus half an ulp where the sum with k need
@@ -627,6 +654,7 @@ kv_status kv_set_geometry(kv_context *ctx, const kv_geometry *geom)
     g.walk_fast = walk_fast_ok(q) ? 1 : 0;
     g.bp_posz = bp_posz_ok(q) ? 1 : 0;
     g.bp_shift = bp_shift(q);
+    g.bp_beside = bp_beside(q) ? 1 : 0;
     g.row_cols = row_cols;
     g.edge_cols = edge_cols;
     const int64_t stride = seg_stride(q);

@@ -176,7 +176,7 @@ __global__ void zs_kernel(KvGeom g, float *__restrict__ zs)
 
 // ------------------------------------------------------ tiled kernel -----
 constexpr int TX = 64;           // voxels along x per workgroup (one per lane)
-constexpr int TY = 4;            // y rows per workgroup (one per wavefront)
+constexpr int TY = KV_BP_TY;     // y rows per workgroup (one per wavefront)
 // x band width (detector columns per plane): it must hold the shadows of a
 // plane's voxels over the brick's slices (beyond it, table reads go to
 // global memory); 24 measured 2 % faster than 32 at full size, 16 26 %
@@ -383,10 +383,11 @@ __device__ __forceinline__ int cvt_flr(float x)
 // next view's bands touched or loaded early, bricks dealt to the XCDs by
 // neighbourhood.  The MLEM update of 1024x1024x64 voxels from 25 views of
 // 2048x2048 took 5.53 ms (mode R) and 5.45 ms (mode A) with five workgroups,
-// 8-word table entries, per-slice tests and two-sided minima; it takes 4.51
-// and 4.58 ms.  512x512x48 voxels, 21 views of 1024x1024: 0.80 / 0.76 ms
-// before, 0.65 now.
-template <int MODE, int EP, int ZT, bool UNIT, bool FW>
+// 8-word table entries, per-slice tests and two-sided minima, then 4.39 and
+// 4.59 ms, and takes 4.11 and 4.29 ms without the views beside a brick (below).
+// 512x512x48 voxels, 21 views of 1024x1024: 0.79 / 0.79 ms, then 0.64 / 0.60,
+// now 0.61 / 0.59.
+template <int MODE, int EP, int ZT, bool UNIT, bool FW, bool BESIDE>
 __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, const float *__restrict__ proj,
                                          float *__restrict__ vol, const float *__restrict__ sens, int bxi, int byi,
                                          int bzi, int zt, BpShared<ZT, bp_sums<MODE, EP>()> &sm)
@@ -420,7 +421,42 @@ __device__ __forceinline__ void bp_brick(const KvGeom &g, const KvTables &t, con
         for (int k = 0; k < bp_sums<MODE, EP>(); ++k)
             accs[i][k][tid] = 0.f;
 
-    for (int p = 0; p < g.np; ++p) {
+    // Views whose rays all pass beside the brick in y give no slice a detector
+    // row (shadow_affine); those at either end of the scan are left out, with
+    // their bands, barriers and slices.  A row's position is affine in y and
+    // in the planes' scale T, which is monotone over the brick's planes, so
+    // its extremes lie at the brick's corners; positions up to 65536 rows are
+    // good to a hundredth of the 0.05 allowed for.  Each lane tests a view,
+    // the same in every wavefront.
+    // A slice without rows still costs its table entry, and of a wide volume
+    // of few rows most views pass beside most bricks, where six workgroups of
+    // such slices were slower than the five of before (671x103x40 voxels, 15
+    // views: 61 us with five, 76 with six, 17 without these views; 1024x1024x64
+    // voxels, 25 views 4.39 -> 4.11 ms).  Where few bricks are beside a view
+    // (KvGeom::bp_beside) the kernel with the test is 2 to 4 % slower, in mode
+    // R by its register allocation (mode A: under 1 %, one kernel).
+    int first = 0, end = g.np;
+    if (BESIDE && g.bp_beside) {
+        first = g.np;
+        end = 0;
+        for (int p = 0; p < g.np; p += 64) {
+            const int q = min(p + lane, g.np - 1);
+            const float *Za = t.zs + ((size_t)q * nz1 + z0) * KV_ZS, *Zb = Za + nzt * KV_ZS;
+            const float c0 = (float)y0 - 0.5f * (float)g.ny, c1 = c0 + (float)TY, room = pad + 0.05f;
+            const float lo = fminf(__builtin_fmaf(c0, Za[4], Za[5]), __builtin_fmaf(c0, Zb[4], Zb[5]));
+            const float hi = fmaxf(__builtin_fmaf(c1, Za[4], Za[5]), __builtin_fmaf(c1, Zb[4], Zb[5]));
+            const bool front = Za[0] > 0.f && Zb[0] > 0.f && Za[0] < 1e30f && Zb[0] < 1e30f;
+            const bool fine = g.nv < 65536 && fabsf(Za[5]) < 65536.f && fabsf(Zb[5]) < 65536.f;
+            const unsigned long long views = __builtin_amdgcn_ballot_w64(
+                !front || !fine || (hi >= -room && lo <= (float)(g.nv - 1) + room));
+            if (views) {
+                first = min(first, p + __builtin_ctzll(views));
+                end = min(p + 64 - __builtin_clzll(views), g.np);
+            }
+        }
+    }
+
+    for (int p = first; p < end; ++p) {
         // Per-view terms, uniform over the workgroup and evaluated once per
         // geometry with the same FP32 operations (scalar loads): source x
         // over sx, detector corner and far edge x over sx, and the lateral
@@ -883,12 +919,12 @@ __global__ __launch_bounds__(256) void scale_a_kernel(KvGeom g, KvTables t, cons
 }
 
 // One brick per workgroup.
-template <int MODE, int EP, int ZT, bool UNIT, bool FW>
+template <int MODE, int EP, int ZT, bool UNIT, bool FW, bool BESIDE>
 __global__ __launch_bounds__(256, 6) void bp_tiled_kernel(KvGeom g, KvTables t, const float *__restrict__ proj,
                                                        float *__restrict__ vol, const float *__restrict__ sens, int zt)
 {
     __shared__ BpShared<ZT, bp_sums<MODE, EP>()> sm;
-    bp_brick<MODE, EP, ZT, UNIT, FW>(g, t, proj, vol, sens, blockIdx.x, blockIdx.y, blockIdx.z, zt, sm);
+    bp_brick<MODE, EP, ZT, UNIT, FW, BESIDE>(g, t, proj, vol, sens, blockIdx.x, blockIdx.y, blockIdx.z, zt, sm);
 }
 
 // Backprojection + MLEM update over a batch of reconstructions, a workgroup
@@ -916,7 +952,7 @@ __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__res
         const int bz = (int)(local / per_z);
         const int rem = (int)(local - (long long)bz * per_z);
         const int by = rem / P.bp_bx, bx = rem - by * P.bp_bx;
-        bp_brick<MODE, KV_EP_MLEM, kZT, false, FW>(P.g, P.t, P.ratio, P.vol, P.sens, bx, by, bz, P.bp_zt, sm);
+        bp_brick<MODE, KV_EP_MLEM, kZT, false, FW, true>(P.g, P.t, P.ratio, P.vol, P.sens, bx, by, bz, P.bp_zt, sm);
     }
 }
 
@@ -930,7 +966,8 @@ __global__ __launch_bounds__(256, 6) void bp_batch_kernel(const KvProblem *__res
 // keep it there.  Measured (8 slices and as chosen): 128x128x32 voxels, 15
 // views 60 -> 37 us (2 slices); 256x256x32, 15 views 97 -> 85 (6; 5, just past
 // one round: 101); 163x181x54, 13 views 83 -> 69 (5); 561x117x34, 25 views
-// 122 -> 111 (7; 6: 163).  Mode A, one sum per voxel, has the LDS for 16
+// 122 -> 111 (7; 6: 163); all with every view's bands staged, which
+// KvGeom::bp_beside may leave out.  Mode A, one sum per voxel, has the LDS for 16
 // slices, used as far as the bands hold their shadows (KvGeom::bp_shift, 13
 // columns over a brick): 512x512x48, 21 views 0.65 -> 0.57 ms (16);
 // 333x287x45, 13 views 172 -> 154 us (15, one round; 12: 195); with wider
@@ -973,11 +1010,13 @@ hipError_t launch_tiled(const KvGeom &g, const KvTables &t, const float *proj, f
     bool fw = false;
     if constexpr (MODE == KV_MODE_R && EP != KV_EP_COUNT) {
         fw = g.bp_posz != 0;
-        if (fw)
-            bp_tiled_kernel<MODE, EP, ZT, UNIT, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
+        if (fw && g.bp_beside)
+            bp_tiled_kernel<MODE, EP, ZT, UNIT, true, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
+        else if (fw)
+            bp_tiled_kernel<MODE, EP, ZT, UNIT, true, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     }
     if (!fw)
-        bp_tiled_kernel<MODE, EP, ZT, UNIT, false><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
+        bp_tiled_kernel<MODE, EP, ZT, UNIT, false, true><<<grid, block, 0, s>>>(g, t, proj, vol, sens, zt);
     return hipGetLastError();
 }
 

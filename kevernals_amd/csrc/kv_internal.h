@@ -56,6 +56,7 @@ struct KvGeom {
     int row_cols, edge_cols;
     int walk_fast;  // forward walk may use end thresholds and 24-bit indices (see kv_fp.hip)
     float bp_shift; // largest shift of a voxel edge's shadow over one slice, in detector columns (0: unbounded)
+    int bp_beside;  // many backprojection bricks lie beside views' detector rows (see kv_bp.hip)
     int bp_posz;    // every view's z planes at alpha >= 1e-6: clamped backprojection weights (see kv_bp.hip)
 };
 
@@ -161,6 +162,7 @@ struct KvTables {
     // KV_YZ_ROWS first rows.  One entry more may be read past the end.
     float *yz = nullptr;
 };
+constexpr int KV_BP_TY = 4;  // voxel rows of a backprojection brick
 constexpr int KV_ZS = 8;
 constexpr int KV_YZ = 16;
 constexpr int KV_YZ_ROWS = 4;

@@ -205,11 +205,11 @@ assert n == 0 and [l for l, _ in again] == before and [z for _, z in again] == [
 
 
 def test_backprojectors_without_a_caller_are_not_built(run):
-    """Weights without their test (FW, the last parameter) are mode R's, and
-    not of the pair count, which needs the test."""
+    """Weights without their test (FW, the last parameter but one) are mode R's,
+    and not of the pair count, which needs the test."""
     run("""
 H.fake_kernel.restype = ctypes.c_char_p
 names = [H.fake_kernel(i).decode() for i in range(H.fake_kernels())]
-fw = [n for n in names if "bp_tiled_kernel" in n and "Lb1EEEv" in n]
-assert len(fw) == 3 and all("ILi0ELi%dE" % ep in n for ep, n in enumerate(sorted(fw))), fw
+fw = [n for n in names if "bp_tiled_kernel" in n and ("Lb1ELb0EEEv" in n or "Lb1ELb1EEEv" in n)]
+assert len(fw) == 6 and all("ILi0ELi%dE" % (i // 2) in n for i, n in enumerate(sorted(fw))), fw
 """)
