@@ -8,13 +8,15 @@ import ctypes
 import numpy as np
 import pytest
 
-from test_gpu_rows import CASES, CASES_R
+from test_gpu_rows import CASES, CASES_R, arc
 
 pytestmark = pytest.mark.gpu
 
 torch = pytest.importorskip("torch")
 
-NAMES = sorted(CASES) + ["wide", "offset", "slices1"]
+NAMES = sorted(CASES) + ["wide", "offset", "slices1", "coarse_hit"]
+# pixels of several voxels, in views that all meet the volume
+COARSE = ((150, 60, 12), (0.2, 0.4, 2.0), (130, 50), (0.9, 0.7), 4, 3.0)
 
 
 @pytest.fixture(scope="module")
@@ -34,6 +36,8 @@ def drop_lists(obj):
 
 
 def geometry(name):
+    if name == "coarse_hit":
+        return arc(*COARSE)
     return (CASES.get(name) or CASES_R[name])()
 
 
@@ -70,12 +74,34 @@ def test_passes_without_lists(K, name):
     assert ll_plain == ll
 
 
+@pytest.mark.parametrize("name", ["faces", "wide", "offset", "coarse_hit"])
+def test_mode_r_infinities_and_nan_reach_the_oracles_rays(K, name):
+    """A ray's value is INF or NaN where the reference's is, and all others
+    keep their bits: voxels taken with weight zero, or read and rejected, leave
+    the sums alone.  Row by row and without lists."""
+    from oracle.oracle import Oracle
+
+    g = geometry(name)
+    vol = random(g.vol_shape, 6)
+    rng = np.random.Generator(np.random.PCG64(7))
+    for value in (np.inf, -np.inf, np.nan):
+        vol.ravel()[rng.integers(0, vol.size, 30)] = value
+    ref = Oracle(g).fp_r(vol)
+    assert 0 < np.count_nonzero(~np.isfinite(ref)) < ref.size // 2
+    ctx = K.Context(0, g)
+    for _ in range(2):
+        out = torch.empty(g.proj_shape, device="cuda")
+        ctx.forward_project(torch.from_numpy(vol).cuda(), out, K.MODE_R)
+        np.testing.assert_array_equal(out.cpu().numpy(), ref)
+        drop_lists(ctx)
+
+
 @pytest.mark.parametrize("layout", [1, 2, 4, 8])
 @pytest.mark.parametrize("mode", ["R", "A"])
 def test_batches_without_lists(K, mode, layout):
     """One detector column, less and more than a tile, wide cones."""
     mode = {"R": K.MODE_R, "A": K.MODE_A}[mode]
-    gs = [geometry(n) for n in ("nu65", "faces", "nu1", "coarse", "cone")]
+    gs = [geometry(n) for n in ("nu65", "faces", "nu1", "coarse_hit", "cone")]
     iters = [2, 1, 2, 1, 2]
     data = [random(g.proj_shape, 20 + i, 0.2) for i, g in enumerate(gs)]
     b = K.Batch(gs, mode=mode)
