@@ -13,6 +13,7 @@ typedef struct { uint32_t x, y, z; } dim3_t;
 
 static size_t budget = (size_t)1 << 40, used;
 static int capture, last_error;
+static dim3_t last_grid;
 static char log_text[1 << 20];
 static struct { const void *host; char name[512]; } fn[512];
 static int nfn;
@@ -33,6 +34,7 @@ size_t fake_used(void) { return used; }
 void fake_capture(int on) { capture = on; }
 const char *fake_log(void) { return log_text; }
 void fake_log_clear(void) { log_text[0] = 0; }
+unsigned fake_grid_z(void) { return last_grid.z; } /* of the last launch */
 int fake_kernels(void) { return nfn; }
 const char *fake_kernel(int i) { return fn[i].name; }
 
@@ -108,6 +110,7 @@ int hipLaunchKernel(const void *f, dim3_t g, dim3_t b, void **args, size_t m, vo
     (void)b, (void)args, (void)m, (void)s;
     if (!g.x || !g.y || !g.z)
         return fail(9); /* an empty grid */
+    last_grid = g;
     for (int i = 0; i < nfn; ++i)
         if (fn[i].host == f)
             note(fn[i].name);
