@@ -211,13 +211,17 @@ std::vector<float> ray_constants(const kv_geometry &q)
     // per detector column (row): centre coordinate, the reference's face
     // alphas of the axis (Projector.cu:54-61, 0 unless |d| > 1e-6) and 1/d
     // (0 when d = 0; the mode-R walk uses it only when |d| > 1e-6)
-    auto axis = [](float *o, float q, float s, float h) {
-        const float d = q - s;
-        const bool ok = std::fabs(d) > 1e-6f;
-        o[0] = q;
-        o[1] = ok ? (-h - s) / d : 0.f;
-        o[2] = ok ? (h - s) / d : 0.f;
-        o[3] = d != 0.f ? 1.f / d : 0.f;
+    // (scalars by value: read through q or rc, which the stores may change for
+    // all the compiler knows, the loop is not vectorised and 8 times as long)
+    auto axis = [](float *o, int n, float corner, float pitch, float spacing, float s, float h) {
+        for (int i = 0; i < n; ++i, o += 4) {
+            const float q = (corner + ((float)i + 0.5f) * pitch) / spacing, d = q - s;
+            const bool ok = std::fabs(d) > 1e-6f;
+            o[0] = q;
+            o[1] = ok ? (-h - s) / d : 0.f;
+            o[2] = ok ? (h - s) / d : 0.f;
+            o[3] = d != 0.f ? 1.f / d : 0.f;
+        }
     };
     for (int p = 0; p < q.np; ++p) {
         const float *S = q.src + 3 * p, *D = q.det + 3 * p;
@@ -234,10 +238,8 @@ std::vector<float> ray_constants(const kv_geometry &q)
         c[8] = D[0] / q.sx;
         c[9] = (D[0] + (float)q.nu * q.pu) / q.sx;
         c[10] = x_rounding(hx, c[0], q.nx);
-        for (int u = 0; u < q.nu; ++u)
-            axis(qx + ((size_t)p * q.nu + u) * 4, (D[0] + ((float)u + 0.5f) * q.pu) / q.sx, c[0], hx);
-        for (int v = 0; v < q.nv; ++v)
-            axis(qy + ((size_t)p * q.nv + v) * 4, (D[1] + ((float)v + 0.5f) * q.pv) / q.sy, c[1], hy);
+        axis(qx + (size_t)p * q.nu * 4, q.nu, D[0], q.pu, q.sx, c[0], hx);
+        axis(qy + (size_t)p * q.nv * 4, q.nv, D[1], q.pv, q.sy, c[1], hy);
     }
     return rc;
 }
@@ -294,7 +296,7 @@ int64_t seg_stride(const kv_geometry &q)
             lo = std::max(lo, std::min(a, b));
             hi = std::min(hi, std::max(a, b));
         }
-        for (int v = 0; v < q.nv; ++v) {
+        for (int v : {0, q.nv - 1}) {  // the steepest rows
             const double dy = ((double)q.det[3 * p + 1] + (v + 0.5) * q.pv) / q.sy - sy;
             const double y = std::max(0.0, hi - lo) * std::fabs(dy);
             most = std::max(most, y < q.ny ? (int)y : q.ny);
