@@ -9,7 +9,9 @@ backprojection + update).  Inputs are resident in HBM before timing starts.
 Output: one JSON line.  value = GRays/s forward+back = views*nu*nv / t(step).
 roofline: the dominant kernel's algorithmic bytes per launch (accepted
 (ray, voxel) pairs * 4 B + its streamed arrays) over its average duration,
-measured with HIP events on the stream the kernels run on.  cpu_baseline: the
+measured with HIP events on the stream the kernels run on; caches serve most of
+them, and traffic_frac is the share of the HBM peak by the profiled physical
+bytes.  cpu_baseline: the
 CPU oracle (a port of the reference arithmetic, OpenMP) timed on a bounded
 sample of the same workload on this host, extrapolated to one full step.
 """
@@ -27,7 +29,7 @@ sys.path.insert(0, ROOT)
 HBM_PEAK_GBS = 8000.0
 # rocprofv3 (demangled) names of the two fused MLEM kernels
 FP_KERNEL = "fp_r_row_kernel<1>"
-BP_KERNEL = "bp_tiled_kernel<0, 1, 8, false, true>"
+BP_KERNEL = "bp_tiled_kernel<0, 1, 8, false, true, true>"
 METRIC = "time to RMSE≤1% vs converged MLEM, learned vs plain; GRays/s fwd+back"
 
 
@@ -154,6 +156,13 @@ def cpu_baseline(g, mu_h, data_h, seconds):
                      "seconds_per_step_extrapolated": one_s},
         "small_workload_full": small,
     }
+
+
+def hbm_frac(kernel, ms):
+    """Share of the HBM peak that the profiled physical traffic of a launch
+    makes over its measured time."""
+    traffic = traffic_from_profiles(kernel)
+    return traffic and round(traffic / (ms * 1e-3) / 1e9 / HBM_PEAK_GBS, 4)
 
 
 def traffic_from_profiles(kernel):
@@ -670,8 +679,7 @@ def bench_sart_saa(K, ctx, g, data, torch, saa_reps=5):
     saa_ms = _event_ms(torch, lambda: ctx.shift_and_add(data, out, g.src[:, 1], planes, sid, 0.0, g.sy),
                        saa_reps)
     del out
-    plane_px = g.nu * g.nv * len(planes)
-    saa_bytes = 4 * g.nviews * plane_px + 4 * plane_px  # every view read per output pixel + the write
+    saa_bytes = 4 * g.nu * g.nv * (g.nviews + len(planes))  # every projection read once, every plane written
     saa_gbs = saa_bytes / (saa_ms * 1e-3) / 1e9
     log(f"[bench] SART {sart_ms:.3f} ms per iteration; shift-and-add ({len(planes)} planes) {saa_ms:.3f} ms")
     return {
@@ -683,6 +691,7 @@ def bench_sart_saa(K, ctx, g, data, torch, saa_reps=5):
                                        "achieved": round(saa_gbs, 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                                        "frac": round(saa_gbs / HBM_PEAK_GBS, 4),
                                        "traffic": traffic_from_profiles("saa_kernel<8, 32>"),
+                                       "traffic_frac": hbm_frac("saa_kernel<8, 32>", saa_ms),
                                        "algorithmic_bytes": saa_bytes}},
     }
 
@@ -844,6 +853,7 @@ def main():
             "unit": "GB/s",
             "frac": round(achieved / HBM_PEAK_GBS, 4),
             "traffic": traffic_from_profiles(kname),
+            "traffic_frac": hbm_frac(kname, kms),
             "algorithmic_bytes": kbytes,
         },
         "cpu_baseline": cpu,
