@@ -924,8 +924,8 @@ __device__ __forceinline__ void seg_sums(const KvRsrc (&rs)[NV], int nx, KvSegC 
 // lane takes its two voxels by a lane permute (which selects by index modulo
 // 64 itself).  The gathers were bound by the L1 (10 cycles per load and CU:
 // 4.0 ms at the size above, 8.0 / 11.9 ms for two / three volumes); this form
-// takes 3.0 ms, bound by instruction issue, and 5.9 / 8.6 ms, bound by the
-// L1's row loads.
+// takes 3.0 ms, bound by instruction issue, and 6.3 / 9.2 ms, bound by the
+// L1's row loads (texture addressers 83 % busy).
 //
 // Rows are loaded one block ahead.  A window placed when block n starts holds
 // every voxel of blocks n and n + 1: the lanes' range now, plus `below` /
@@ -1823,7 +1823,7 @@ __global__ __launch_bounds__(256) void fp_r_batch_kernel(const KvProblem *__rest
     });
 }
 
-// Persistent mode-A forward pass (MLEM ratio) over a batch, as
+// Mode-A forward pass (MLEM ratio) over a batch, as
 // fp_r_batch_kernel; reconstructions with segment lists run row by row.
 __global__ __launch_bounds__(256) void fp_a_batch_kernel(const KvProblem *__restrict__ probs, int nprob,
                                                          long long total, int iteration)
