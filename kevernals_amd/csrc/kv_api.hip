@@ -53,15 +53,39 @@ kv_status dev_alloc(void **p, size_t bytes)
     return KV_OK;
 }
 
+// Whether work enqueued on s goes into a graph that is being captured (which
+// the null stream's cannot).
+bool capturing(hipStream_t s)
+{
+    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
+    if (s && hipStreamIsCapturing(s, &c) != hipSuccess)
+        (void)hipGetLastError();
+    return c != hipStreamCaptureStatusNone;
+}
+
+// Bytes of a mode's segment lists.
+size_t list_bytes(const KvGeom &g, int mode)
+{
+    const size_t rows = (size_t)g.np * g.nv, n = rows * (size_t)g.seg_stride;
+    return mode == KV_MODE_A ? n * sizeof(KvSeg) + rows * sizeof(KvSegHead)
+                             : n * sizeof(KvSegR) + rows * sizeof(KvSegHeadR);
+}
+
 // Memory that a call cannot do without: the context's segment lists, which
-// are an option, make room for it.
+// are an option, make room for it if they can (not under capture, which a
+// wait would end).
 kv_status ctx_alloc(kv_context *ctx, void **p, size_t bytes)
 {
     kv_status st = dev_alloc(p, bytes);
-    if (st == KV_ERR_NOMEM && !ctx->lists_held && (ctx->d_seg_a || ctx->d_seg_r) &&
-        (st = kv_internal_drop_lists(ctx)) == KV_OK)
-        st = dev_alloc(p, bytes);
-    return st;
+    if (st != KV_ERR_NOMEM || ctx->lists_held || capturing(ctx->stream))
+        return st;
+    const size_t lists = (ctx->d_seg_a ? list_bytes(ctx->g, KV_MODE_A) : 0) +
+                         (ctx->d_seg_r ? list_bytes(ctx->g, KV_MODE_R) : 0);
+    size_t avail = 0, total = 0;
+    if (lists == 0 || hipMemGetInfo(&avail, &total) != hipSuccess || avail + lists < bytes)
+        return st;
+    st = kv_internal_drop_lists(ctx);
+    return st == KV_OK ? dev_alloc(p, bytes) : st;
 }
 
 // Grows the context's reduction buffer to at least n doubles.  The capacity
@@ -398,16 +422,6 @@ kv_status ensure_sens(kv_context *ctx)
     return KV_OK;
 }
 
-// Whether work enqueued on s goes into a graph that is being captured (which
-// the null stream's cannot).
-bool capturing(hipStream_t s)
-{
-    hipStreamCaptureStatus c = hipStreamCaptureStatusNone;
-    if (s && hipStreamIsCapturing(s, &c) != hipSuccess)
-        (void)hipGetLastError();
-    return c != hipStreamCaptureStatusNone;
-}
-
 void free_lists(kv_context *ctx)
 {
     free_dev(ctx->d_seg_a);
@@ -433,11 +447,9 @@ kv_status ensure_lists(kv_context *ctx, int mode)
     if (ctx->lists_ok[mode] && !graph) {
         ctx->lists_ok[mode] = false;
         const size_t rows = (size_t)g.np * g.nv, n = rows * (size_t)g.seg_stride;
-        const size_t bytes = a ? n * sizeof(KvSeg) + rows * sizeof(KvSegHead)
-                               : n * sizeof(KvSegR) + rows * sizeof(KvSegHeadR);
         size_t avail = 0, total = 0;
         auto alloc = [](auto *&p, size_t k) { return hipMalloc((void **)&p, k * sizeof(*p)) == hipSuccess; };
-        if (hipMemGetInfo(&avail, &total) != hipSuccess || avail < bytes + KV_SEG_SPARE_BYTES ||
+        if (hipMemGetInfo(&avail, &total) != hipSuccess || avail < list_bytes(g, mode) + KV_SEG_SPARE_BYTES ||
             !(a ? alloc(ctx->d_seg_a, n) && alloc(ctx->d_seg_a_head, rows)
                 : alloc(ctx->d_seg_r, n) && alloc(ctx->d_seg_r_head, rows))) {
             (void)hipGetLastError();  // the failed call's

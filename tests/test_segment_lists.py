@@ -111,11 +111,13 @@ tables = H.fake_used() - none
 c.set_geometry(arc())
 forward(c, A)
 have = H.fake_used()
+p = ctypes.c_void_p()
+assert L.kv_malloc(c.handle, 1 << 40, ctypes.byref(p)) == 3 and not p.value  # of no use here
+assert H.fake_used() == have
 H.fake_budget(have + tables - (have - none) // 2)  # enough without the lists
 names = launches(L.kv_back_project, c.handle, buf, buf, A)
 assert ran(names, "tables_a_kernel")
 assert ran(forward(c, A), "fp_a_kernel")
-p = ctypes.c_void_p()
 assert L.kv_malloc(c.handle, 1 << 40, ctypes.byref(p)) == 3 and not p.value
 assert launches(L.kv_memset, c.handle, buf, 0, 16) == []  # no error left behind
 assert ran(forward(c, A), "fp_a_kernel")
@@ -172,6 +174,15 @@ have = H.fake_used()
 H.fake_budget(have + 1000)
 assert L.kv_back_project(c.handle, buf, buf, A) == 3  # no memory
 assert H.fake_used() == have and ran(forward(c, A), "fp_a_row_kernel")
+H.fake_budget(1 << 40)
+c = context(arc())  # lists that no graph holds: kept too, since freeing them waits
+forward(c, A)
+have = H.fake_used()
+H.fake_budget(have + 1000)
+H.fake_capture(1)
+assert L.kv_back_project(c.handle, buf, buf, A) == 3 and H.fake_used() == have
+H.fake_capture(0)
+assert ran(forward(c, A), "fp_a_row_kernel")
 """)
 
 
